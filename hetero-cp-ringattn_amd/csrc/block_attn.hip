@@ -36,6 +36,8 @@
 // General path (any other shape, head_dim <= 256): one thread per (query row, head),
 // K/V tiles staged in LDS as fp32.
 #include <algorithm>
+#include <atomic>
+#include <cmath>
 #include <cstdlib>
 #include <vector>
 
@@ -344,6 +346,11 @@ __device__ __forceinline__ void write_final_row(void* out, int dtype, int64_t of
 // three (160 KiB of LDS, all of it; V's third buffer gives its loads a super-step more
 // slack).  The kernel also compiles for 64-key tiles with rings of three; 128 keys
 // halve the per-tile barriers, DMA issue and softmax bookkeeping and measured 5% faster.
+// Short launches run a split form (KW = 2 or 4): the workgroup has 256 / KW rows and KW
+// waves share a 32-row block, each folding its part of every tile's keys with its own
+// (m, l, O); the parts are merged in LDS before the rows are written.  A block of 512
+// queries against 8192 keys has only 64 workgroups of 256 rows: 166 us for it and its
+// diagonal, 94 us with KW = 4; KW and the reason for the line: key_parts.
 // The half-width instantiation (head dims up to 64) keeps 64 dims per LDS row: 8 rows
 // per DMA instruction, swizzles K (r >> 1) & 7 and V 4 ((r >> 1) & 1), 16 KiB tiles
 // (80 KiB of LDS; against 128-dim rows with a zero half, +2.6% on a 32k Qwen2-0.5B
@@ -427,7 +434,7 @@ static_assert(sizeof(RingPlan) <= 4096, "kernel arguments are limited to 4 KiB")
 // the workgroup moved past that source, two words each (0: never visited).
 constexpr int kTraceHeaderWords = 16;
 
-template <int DT, int G, bool POS, int BK, bool RING, class P, bool TRACE = false, int DWN = kD3>
+template <int DT, int G, bool POS, int BK, bool RING, class P, bool TRACE = false, int DWN = kD3, int KW = 1>
 __device__ __forceinline__ void pingpong_body(const P& plan) {
   using Ops = MfmaOps<DT>;
   using frag = typename Ops::frag;
@@ -436,8 +443,10 @@ __device__ __forceinline__ void pingpong_body(const P& plan) {
   // on 128-byte LDS rows: half the LDS, half the DMA instructions, its own swizzles.
   static_assert(DWN == kD3 || DWN == kD3 / 2, "dims folded: 128 or 64");
   constexpr int DW = DWN;
-  static_assert(kWaves % G == 0, "heads per group must divide the waves");
-  constexpr int TB = kWaves / G;
+  // KW waves split the keys of every tile of one (head, 32-row block) between them.
+  static_assert(kWaves % (G * KW) == 0, "heads per group times key parts must divide the waves");
+  constexpr int TB = kWaves / (G * KW);
+  constexpr int BKW = BK / KW;                   // keys of a tile that one wave folds
   constexpr int TQ = 32 * TB;
   constexpr int KS = DW / 16;
   constexpr int DB = DW / 32;
@@ -448,8 +457,8 @@ __device__ __forceinline__ void pingpong_body(const P& plan) {
   constexpr int RPI = 1024 / PW;
   constexpr int kDmaPerWave = BK / RPI / kWaves;  // 1 KiB DMA instructions per wave per tile (K or V)
   constexpr int kTile = BK * PW;                 // bytes of one K or V tile
-  constexpr int NKB = BK / 32;                   // 32-key blocks of S^T per tile
-  constexpr int NPS = BK / 16;                   // 16-key steps of the PV product per tile
+  constexpr int NKB = BKW / 32;                  // 32-key blocks of S^T per tile and wave
+  constexpr int NPS = BKW / 16;                  // 16-key steps of the PV product per tile and wave
   // LDS buffers per ring: 3 + 3 tiles of 64 keys (96 KiB); 2 K + 3 V tiles of 128 keys
   // (160 KiB at 128 dims, 80 KiB at 64; two V buffers measured 0.4% slower).
   constexpr int NBK = BK == 64 ? 3 : 2;
@@ -524,7 +533,8 @@ __device__ __forceinline__ void pingpong_body(const P& plan) {
   const int head = hg * G + (wave % G);  // this wave's query head
   const int kvh = (hg * G) / rep;          // the KV head whose rows the tiles hold
   const int tq0 = qt * TQ;
-  const int wq0 = tq0 + (wave / G) * 32;
+  const int wq0 = tq0 + (KW == 1 ? wave / G : wave / G % TB) * 32;
+  const int kw0 = KW == 1 ? 0 : wave / (G * TB) * BKW;  // first key of a tile that this wave folds
   const int my_q = wq0 + lcol;
   const int q_end = min(lq, tq0 + TQ);
 
@@ -667,7 +677,7 @@ __device__ __forceinline__ void pingpong_body(const P& plan) {
   // K fragment s of a lane sits at k_rd0 ^ (s << 5) in a tile: (lhalf + 2s) ^ (krow & 15)
   // changes only bits 1-3 of the 16-byte column index with s, and tile bases are
   // 1 KiB-aligned, so the XOR commutes with adding the base.
-  const uint32_t k_rd0 = krow * PW + ((lhalf ^ swz_k(krow)) << 4);
+  const uint32_t k_rd0 = (kw0 + krow) * PW + ((lhalf ^ swz_k(krow)) << 4);
   const int g16 = lane >> 4, sl = lane & 15;
   uint32_t v_rd[DB];
 #pragma unroll
@@ -675,7 +685,7 @@ __device__ __forceinline__ void pingpong_body(const P& plan) {
     // row 8 (g16 >> 1) + (sl >> 2) of a 16-key step (and 4 rows on), so swz_v of that
     // row is 4 (sl >> 2) for 256-byte rows and 4 ((sl >> 3) & 1) for 128-byte ones
     const int vs = PW == 256 ? (sl >> 2) : ((sl >> 3) & 1);
-    v_rd[b] = (8 * (g16 >> 1) + (sl >> 2)) * PW + ((4 * (b ^ vs) + 2 * (g16 & 1) + ((sl & 3) >> 1)) << 4) + 8 * (sl & 1);
+    v_rd[b] = (kw0 + 8 * (g16 >> 1) + (sl >> 2)) * PW + ((4 * (b ^ vs) + 2 * (g16 & 1) + ((sl & 3) >> 1)) << 4) + 8 * (sl & 1);
   }
   const uint32_t k_lds_off = lds_offset(k_lds);
   const char* v_lds_c = reinterpret_cast<const char*>(v_lds);
@@ -785,15 +795,16 @@ __device__ __forceinline__ void pingpong_body(const P& plan) {
   auto xphase = [&](int t) __attribute__((always_inline)) {
     int kv0, ke;
     tile_rows(t, kv0, ke);
-    const int rows_left = ke - kv0;                     // visible rows from the tile's first key on
+    kv0 += kw0;                                         // this wave's keys of the tile: [kv0, kv0 + BKW)
+    const int rows_left = ke - kv0;                     // visible rows from the first of them on
     const int64_t krel = kv0 + kdelta;                  // position of that key relative to query row 0
-    bool need_mask = rows_left < BK;
-    if (causal) need_mask = need_mask || (POS ? kv0 + BK - 1 > wave_lim_first : krel + BK - 1 > wq0);
+    bool need_mask = rows_left < BKW;
+    if (causal) need_mask = need_mask || (POS ? kv0 + BKW - 1 > wave_lim_first : krel + BKW - 1 > wq0);
     if (need_mask) {
       // key kv0 + j of the segment is visible to this lane iff j <= lim
       int64_t lim64 = rows_left - 1;
       if (causal) lim64 = min(lim64, POS ? qlim64 - kv0 : static_cast<int64_t>(my_q) - krel);
-      const int lim = static_cast<int>(max(min(lim64, static_cast<int64_t>(BK)), static_cast<int64_t>(-1))) - 8 * lhalf;
+      const int lim = static_cast<int>(max(min(lim64, static_cast<int64_t>(BKW)), static_cast<int64_t>(-1))) - 8 * lhalf;
 #pragma unroll
       for (int b = 0; b < NKB; ++b)
 #pragma unroll
@@ -946,6 +957,45 @@ __device__ __forceinline__ void pingpong_body(const P& plan) {
     if (!lead) issue(u + 1);
   }
 
+  if constexpr (KW > 1) {
+    // The key parts of a row block meet in LDS: parts 1 .. KW - 1 leave (O, m, l) over the
+    // K / V tiles, part 0 folds them in and writes the rows.
+    constexpr int kPer = G * TB;             // waves of one key part
+    static_assert((kWaves - kPer) * DB * 4096 <= NBV * kTile, "parts of O fit the V buffers");
+    float* const ml = reinterpret_cast<float*>(k_lds);
+    f32x4* const os = reinterpret_cast<f32x4*>(v_lds);
+    __syncthreads();                         // every wave is past its last read of the tiles
+    const int part = wave - kPer;
+    if (part >= 0) {
+      ml[2 * part * 64 + lane] = m_run;
+      ml[(2 * part + 1) * 64 + lane] = l_run;
+#pragma unroll
+      for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          os[((part * DB + b) * 4 + j) * 64 + lane] =
+              f32x4{oacc[b][4 * j], oacc[b][4 * j + 1], oacc[b][4 * j + 2], oacc[b][4 * j + 3]};
+    }
+    __syncthreads();
+    if (part >= 0) return;
+#pragma unroll 1
+    for (int i = wave; i < kWaves - kPer; i += kPer) {
+      const float m2 = ml[2 * i * 64 + lane], l2 = ml[(2 * i + 1) * 64 + lane];
+      const float m_new = fmaxf(m_run, m2);
+      const float a1 = exp2f(m_run - m_new), a2 = exp2f(m2 - m_new);
+      l_run = l_run * a1 + l2 * a2;
+      m_run = m_new;
+#pragma unroll
+      for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const f32x4 o2 = os[((i * DB + b) * 4 + j) * 64 + lane];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) oacc[b][4 * j + e] = oacc[b][4 * j + e] * a1 + o2[e] * a2;
+        }
+    }
+  }
+
   if (my_q >= lq) return;
   if constexpr (RING) {
     const int64_t row = static_cast<int64_t>(plan.off[t_dom]) + my_q;
@@ -977,14 +1027,14 @@ __device__ __forceinline__ void pingpong_body(const P& plan) {
   }
 }
 
-template <int DT, int G, bool POS, int BK, int DWN>
+template <int DT, int G, bool POS, int BK, int DWN, int KW = 1>
 __global__ __launch_bounds__(kThreads, 1) void flash_block_pingpong_kernel(BlockGroup grp) {
-  pingpong_body<DT, G, POS, BK, false, BlockGroup, false, DWN>(grp);
+  pingpong_body<DT, G, POS, BK, false, BlockGroup, false, DWN, KW>(grp);
 }
 
-template <int DT, int G, int BK, bool TRACE, int DWN>
+template <int DT, int G, int BK, bool TRACE, int DWN, int KW = 1>
 __global__ __launch_bounds__(kThreads, 1) void flash_ring_kernel(RingPlan plan) {
-  pingpong_body<DT, G, false, BK, true, RingPlan, TRACE, DWN>(plan);
+  pingpong_body<DT, G, false, BK, true, RingPlan, TRACE, DWN, KW>(plan);
 }
 
 // ----------------------------------------------------------------------------------
@@ -1391,14 +1441,74 @@ static int heads_per_group(int rep) {
 // Work decomposition of the matrix-core kernels: query heads per group (sharing a K/V
 // tile), query rows per workgroup and head groups per query tile.
 struct Geometry {
-  int g, tq, n_groups;
+  int g, kw, tq, n_groups;
 };
-static Geometry geometry(int hq, int hkv) {
+static Geometry geometry(int hq, int hkv, int kw = 1) {
   Geometry r;
-  r.g = heads_per_group(hq / hkv);
-  r.tq = 32 * (kWaves / r.g);
+  r.g = std::min(heads_per_group(hq / hkv), kWaves / kw);
+  r.kw = kw;
+  r.tq = 32 * (kWaves / (r.g * kw));
   r.n_groups = hq / r.g;
   return r;
+}
+
+// Compute units of the current device (256 when none can be queried).
+static int device_cus() {
+  static std::atomic<int> known[64];
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return 256;
+  }
+  if (dev < 0 || dev >= 64) return 256;
+  cus = known[dev].load(std::memory_order_relaxed);
+  if (cus > 0) return cus;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
+    (void)hipGetLastError();
+    return 256;
+  }
+  known[dev].store(cus, std::memory_order_relaxed);
+  return cus;
+}
+
+static bool half_width_d(int d);
+
+// Key parts (KW) of a launch.  A workgroup of 256 / KW rows splits every tile's keys over
+// KW waves: KW times the workgroups, each with a shorter chain of tiles, for launches that
+// leave CUs idle; but every workgroup still brings whole K / V tiles to LDS, so on a full
+// chip it costs more.  Modelled time: the longest workgroup (its tiles alone on a CU) and
+// the whole work over the CUs (tiles with every CU busy: lower clock, shared L2), joined as
+// a 4-norm since the workgroups of a causal launch neither all run at once nor queue
+// evenly; a split form has to be 6% ahead.  Per KW = 1, 2, 4, in us: `own` per workgroup
+// (first loads, rows written), `alone` and `full` per 128-key tile, fitted on MI355X to 74
+// launches: blocks of 16-4096 queries against 256-16384 keys, causal rings of 512-8192
+// tokens and ZigZag ones, with 32/8, 16/2, 16/16 heads of 128 and 14/2 of 64 dims.  There
+// it costs at most 3% against KW = 1 and saves up to 59% (512 x 16384, 32/8 heads: 271 us
+// with KW = 1, 165 with 2, 143 with 4; a 900-token ring 24.6, 19.0, 24.7; 3000 tokens 76,
+// 86, 117).
+//   pairs, rows, n_max: visible (query, key) pairs of one query head, query rows (of
+//   `blocks` chunks), and the most 128-key tiles that one row folds
+static int key_parts(double pairs, double rows, int blocks, double n_max, int hq, int hkv, int d) {
+  static const double own[3] = {4.0, 3.0, 3.0};
+  static const double alone[2][3] = {{2.03, 1.20, 0.81}, {1.83, 1.04, 0.67}};
+  static const double full[2][3] = {{3.26, 1.77, 1.07}, {2.22, 1.20, 0.55}};
+  const int w = half_width_d(d) ? 1 : 0;
+  const double cus = device_cus();
+  int best = 1;
+  double best_t = 0.0;
+  for (int i = 0; i < 3; ++i) {
+    const Geometry geo = geometry(hq, hkv, 1 << i);
+    const double items = geo.n_groups * (rows / geo.tq + 0.5 * blocks);
+    const double tiles = geo.n_groups * (pairs / kBK3 + 0.5 * rows) / geo.tq;
+    const double chain = own[i] + n_max * alone[w][i];
+    const double spread = (items * own[i] + tiles * full[w][i]) / cus;
+    const double t = (i == 0 ? 1.0 : 1.06) * std::pow(std::pow(chain, 4) + std::pow(spread, 4), 0.25);
+    if (i == 0 || t < best_t) {
+      best = 1 << i;
+      best_t = t;
+    }
+  }
+  return best;
 }
 
 // The head-dim-128 kernels form buffer descriptors with 32-bit row arithmetic: a tile of
@@ -1408,7 +1518,7 @@ static void check_tile_bytes(int64_t k_ss, int64_t v_ss) {
           "k/v sequence strides too large for the matrix-core kernel");
 }
 
-static BlockArgs make_args(const BlockLaunch& L) {
+static BlockArgs make_args(const BlockLaunch& L, const Geometry& geo) {
   BlockArgs a;
   a.q = static_cast<const uint16_t*>(L.q);
   a.k = static_cast<const uint16_t*>(L.k);
@@ -1435,7 +1545,6 @@ static BlockArgs make_args(const BlockLaunch& L) {
   a.alt_hs = L.alt_hs;
   a.alt_ss = L.alt_ss;
   a.d = static_cast<int32_t>(L.d);
-  const Geometry geo = geometry(L.hq, L.hkv);
   a.n_qtiles = static_cast<int32_t>(ceil_div(L.lq, geo.tq));
   a.n_groups = geo.n_groups;
   return a;
@@ -1447,24 +1556,29 @@ static bool half_width_d(int d) { return d <= kD3 / 2; }
 
 // One launch of the head-dim-128 kernel over grp.a[0 .. grp.n) (same dtype, heads, and
 // positions mode; every pair has at least one query tile).
-template <int DT, int G, int DWN>
+template <int DT, int G, int KW, int DWN>
 static void launch_pingpong_g(const BlockGroup& grp, bool pos, dim3 grid, hipStream_t stream) {
-  if (pos) flash_block_pingpong_kernel<DT, G, true, kBK3, DWN><<<grid, kThreads, 0, stream>>>(grp);
-  else flash_block_pingpong_kernel<DT, G, false, kBK3, DWN><<<grid, kThreads, 0, stream>>>(grp);
+  if (pos) flash_block_pingpong_kernel<DT, G, true, kBK3, DWN, KW><<<grid, kThreads, 0, stream>>>(grp);
+  else flash_block_pingpong_kernel<DT, G, false, kBK3, DWN, KW><<<grid, kThreads, 0, stream>>>(grp);
 }
 
 template <int DT, int DWN>
-static void launch_pingpong_w(const BlockGroup& grp, int g, bool pos, dim3 grid, hipStream_t stream) {
-  switch (g) {
-    case 8: launch_pingpong_g<DT, 8, DWN>(grp, pos, grid, stream); break;
-    case 4: launch_pingpong_g<DT, 4, DWN>(grp, pos, grid, stream); break;
-    case 2: launch_pingpong_g<DT, 2, DWN>(grp, pos, grid, stream); break;
-    default: launch_pingpong_g<DT, 1, DWN>(grp, pos, grid, stream); break;
+static void launch_pingpong_w(const BlockGroup& grp, const Geometry& geo, bool pos, dim3 grid, hipStream_t stream) {
+  switch (16 * geo.kw + geo.g) {
+    case 16 + 8: launch_pingpong_g<DT, 8, 1, DWN>(grp, pos, grid, stream); break;
+    case 16 + 4: launch_pingpong_g<DT, 4, 1, DWN>(grp, pos, grid, stream); break;
+    case 16 + 2: launch_pingpong_g<DT, 2, 1, DWN>(grp, pos, grid, stream); break;
+    case 16 + 1: launch_pingpong_g<DT, 1, 1, DWN>(grp, pos, grid, stream); break;
+    case 32 + 4: launch_pingpong_g<DT, 4, 2, DWN>(grp, pos, grid, stream); break;
+    case 32 + 2: launch_pingpong_g<DT, 2, 2, DWN>(grp, pos, grid, stream); break;
+    case 32 + 1: launch_pingpong_g<DT, 1, 2, DWN>(grp, pos, grid, stream); break;
+    case 64 + 2: launch_pingpong_g<DT, 2, 4, DWN>(grp, pos, grid, stream); break;
+    default: launch_pingpong_g<DT, 1, 4, DWN>(grp, pos, grid, stream); break;
   }
 }
 
 template <int DT>
-static void launch_pingpong(BlockGroup& grp, hipStream_t stream) {
+static void launch_pingpong(BlockGroup& grp, const Geometry& geo, hipStream_t stream) {
   const BlockArgs& a0 = grp.a[0];
   for (int i = 0; i < grp.n; ++i) {
     check_tile_bytes(grp.a[i].k_ss, grp.a[i].v_ss);
@@ -1474,17 +1588,49 @@ static void launch_pingpong(BlockGroup& grp, hipStream_t stream) {
   for (int i = 0; i < grp.n; ++i) grp.qt_begin[i + 1] = grp.qt_begin[i] + grp.a[i].n_qtiles;
   const dim3 grid(static_cast<unsigned>(grp.qt_begin[grp.n] * a0.n_groups));
   const bool pos = a0.q_lim != nullptr;
-  const int g = geometry(a0.hq, a0.hkv).g;
-  if (half_width_d(a0.d)) launch_pingpong_w<DT, kD3 / 2>(grp, g, pos, grid, stream);
-  else launch_pingpong_w<DT, kD3>(grp, g, pos, grid, stream);
+  if (half_width_d(a0.d)) launch_pingpong_w<DT, kD3 / 2>(grp, geo, pos, grid, stream);
+  else launch_pingpong_w<DT, kD3>(grp, geo, pos, grid, stream);
+}
+
+// Visible (query, key) pairs of one block and head: exact for
+// contiguous positions, lq * lk / 2 for explicit ones.
+static double block_work(const BlockLaunch& L) {
+  const double lq = static_cast<double>(L.lq), lk = static_cast<double>(L.lk);
+  if (!L.causal) return lq * lk;
+  if (L.q_lim != nullptr) return lq * lk / 2;
+  // row i sees min(max(c + i, 0), lk) keys, c = q_off - k_off + 1
+  const int64_t c = L.q_off - L.k_off + 1;
+  const int64_t i0 = std::min<int64_t>(std::max<int64_t>(0, 1 - c), L.lq);
+  const int64_t i1 = std::min<int64_t>(std::max<int64_t>(0, L.lk - c), L.lq);
+  double w = static_cast<double>(L.lq - std::max(i0, i1)) * lk;
+  if (i1 > i0) w += static_cast<double>(i1 - i0) * static_cast<double>(c) + 0.5 * static_cast<double>(i0 + i1 - 1) * static_cast<double>(i1 - i0);
+  return w;
+}
+
+// Decomposition of a launch over the blocks Ls[0 .. n) (same heads and head dim).
+static Geometry block_geometry(const BlockLaunch* const* Ls, int n) {
+  double pairs = 0.0, rows = 0.0, n_max = 0.0;
+  for (int i = 0; i < n; ++i) {
+    const BlockLaunch& L = *Ls[i];
+    pairs += block_work(L);
+    rows += static_cast<double>(L.lq);
+    // keys that the last row sees (explicit positions: some row may see all of them)
+    int64_t keys = L.lk;
+    if (L.causal && L.q_lim == nullptr)
+      keys = std::max<int64_t>(0, std::min(L.lk, L.q_off + L.lq - L.k_off));
+    n_max = std::max(n_max, static_cast<double>(ceil_div(keys, kBK3)));
+  }
+  return geometry(Ls[0]->hq, Ls[0]->hkv, key_parts(pairs, rows, n, n_max, Ls[0]->hq, Ls[0]->hkv, Ls[0]->d));
 }
 
 template <int DT>
 static void launch_mfma(const BlockLaunch& L, hipStream_t stream) {
   BlockGroup grp;
   grp.n = 1;
-  grp.a[0] = make_args(L);
-  launch_pingpong<DT>(grp, stream);
+  const BlockLaunch* const one = &L;
+  const Geometry geo = block_geometry(&one, 1);
+  grp.a[0] = make_args(L, geo);
+  launch_pingpong<DT>(grp, geo, stream);
 }
 
 static GenArgs make_gen_args(const BlockLaunch& L) {
@@ -1571,21 +1717,6 @@ void launch_block_partial(const BlockLaunch& L, hipStream_t stream) {
   HCP_HIP(hipGetLastError());
 }
 
-// Visible (query, key) pairs of one block, for ordering the pairs of a group: exact for
-// contiguous positions, lq * lk / 2 for explicit ones.
-static double block_work(const BlockLaunch& L) {
-  const double lq = static_cast<double>(L.lq), lk = static_cast<double>(L.lk);
-  if (!L.causal) return lq * lk;
-  if (L.q_lim != nullptr) return lq * lk / 2;
-  // row i sees min(max(c + i, 0), lk) keys, c = q_off - k_off + 1
-  const int64_t c = L.q_off - L.k_off + 1;
-  const int64_t i0 = std::min<int64_t>(std::max<int64_t>(0, 1 - c), L.lq);
-  const int64_t i1 = std::min<int64_t>(std::max<int64_t>(0, L.lk - c), L.lq);
-  double w = static_cast<double>(L.lq - std::max(i0, i1)) * lk;
-  if (i1 > i0) w += static_cast<double>(i1 - i0) * static_cast<double>(c) + 0.5 * static_cast<double>(i0 + i1 - 1) * static_cast<double>(i1 - i0);
-  return w;
-}
-
 void launch_block_group(const BlockLaunch* Ls, int n, hipStream_t stream) {
   std::vector<const BlockLaunch*> live;
   for (int i = 0; i < n; ++i)
@@ -1606,30 +1737,51 @@ void launch_block_group(const BlockLaunch* Ls, int n, hipStream_t stream) {
   for (size_t base = 0; base < live.size(); base += kMaxGroup) {
     BlockGroup grp;
     grp.n = static_cast<int32_t>(std::min<size_t>(kMaxGroup, live.size() - base));
-    for (int i = 0; i < grp.n; ++i) grp.a[i] = make_args(*live[base + i]);
-    if (f.dtype == kBF16) launch_pingpong<kBF16>(grp, stream);
-    else launch_pingpong<kF16>(grp, stream);
+    const Geometry geo = block_geometry(&live[base], grp.n);
+    for (int i = 0; i < grp.n; ++i) grp.a[i] = make_args(*live[base + i], geo);
+    if (f.dtype == kBF16) launch_pingpong<kBF16>(grp, geo, stream);
+    else launch_pingpong<kF16>(grp, geo, stream);
   }
   HCP_HIP(hipGetLastError());
 }
 
 template <int DT, bool TRACE, int DWN>
-static void launch_ring_kernel_w(int g, dim3 grid, const RingPlan& p, hipStream_t stream) {
-  switch (g) {
-    case 8: flash_ring_kernel<DT, 8, kBK3, TRACE, DWN><<<grid, kThreads, 0, stream>>>(p); break;
-    case 4: flash_ring_kernel<DT, 4, kBK3, TRACE, DWN><<<grid, kThreads, 0, stream>>>(p); break;
-    case 2: flash_ring_kernel<DT, 2, kBK3, TRACE, DWN><<<grid, kThreads, 0, stream>>>(p); break;
-    default: flash_ring_kernel<DT, 1, kBK3, TRACE, DWN><<<grid, kThreads, 0, stream>>>(p); break;
+static void launch_ring_kernel_w(const Geometry& geo, dim3 grid, const RingPlan& p, hipStream_t stream) {
+  auto go = [&](auto g, auto kw) {
+    flash_ring_kernel<DT, decltype(g)::value, kBK3, TRACE, DWN, decltype(kw)::value><<<grid, kThreads, 0, stream>>>(p);
+  };
+  switch (16 * geo.kw + geo.g) {
+    case 16 + 8: go(IntC<8>{}, IntC<1>{}); break;
+    case 16 + 4: go(IntC<4>{}, IntC<1>{}); break;
+    case 16 + 2: go(IntC<2>{}, IntC<1>{}); break;
+    case 16 + 1: go(IntC<1>{}, IntC<1>{}); break;
+    case 32 + 4: go(IntC<4>{}, IntC<2>{}); break;
+    case 32 + 2: go(IntC<2>{}, IntC<2>{}); break;
+    case 32 + 1: go(IntC<1>{}, IntC<2>{}); break;
+    case 64 + 2: go(IntC<2>{}, IntC<4>{}); break;
+    default: go(IntC<1>{}, IntC<4>{}); break;
   }
 }
 
 template <int DT, bool TRACE>
-static void launch_ring_kernel(int g, dim3 grid, const RingPlan& p, hipStream_t stream) {
-  if (half_width_d(p.d)) launch_ring_kernel_w<DT, TRACE, kD3 / 2>(g, grid, p, stream);
-  else launch_ring_kernel_w<DT, TRACE, kD3>(g, grid, p, stream);
+static void launch_ring_kernel(const Geometry& geo, dim3 grid, const RingPlan& p, hipStream_t stream) {
+  if (half_width_d(p.d)) launch_ring_kernel_w<DT, TRACE, kD3 / 2>(geo, grid, p, stream);
+  else launch_ring_kernel_w<DT, TRACE, kD3>(geo, grid, p, stream);
 }
 
 bool ring_fused_applies(int dtype, int d) { return (dtype == kBF16 || dtype == kF16) && padded_d_ok(d); }
+
+// Decomposition of a fused ring: its sources and rows as one launch (see key_parts).
+static Geometry ring_geometry(int d, int hq, int hkv, int n, const int64_t* len, int causal) {
+  double rows = 0.0, n_max = 0.0;
+  for (int i = 0; i < n; ++i) {
+    const double own = static_cast<double>(ceil_div(len[i], kBK3)), below = static_cast<double>(ceil_div(static_cast<int64_t>(rows), kBK3));
+    n_max = std::max(n_max, own + below);  // without a causal mask: the last domain's, within a tile of every domain's
+    rows += static_cast<double>(len[i]);
+  }
+  const double pairs = causal ? 0.5 * rows * (rows + 1.0) : rows * rows;
+  return geometry(hq, hkv, key_parts(pairs, rows, n, n_max, hq, hkv, d));
+}
 
 void launch_ring_fused(const RingLaunch& L, hipStream_t stream) {
   require(ring_fused_applies(L.dtype, L.d),
@@ -1646,8 +1798,8 @@ void launch_ring_fused(const RingLaunch& L, hipStream_t stream) {
   p.dtype = L.dtype;
   p.d = L.d;
   p.hq = L.hq; p.hkv = L.hkv; p.rep = L.hq / L.hkv;
-  const Geometry geo = geometry(L.hq, L.hkv);
-  const int g = geo.g, tq = geo.tq;
+  const Geometry geo = ring_geometry(L.d, L.hq, L.hkv, L.n, L.len, L.causal);
+  const int tq = geo.tq;
   p.n_groups = geo.n_groups;
   p.n = L.n;
   p.causal = L.causal;
@@ -1665,26 +1817,26 @@ void launch_ring_fused(const RingLaunch& L, hipStream_t stream) {
   for (int s = 0; s < L.n; ++s) p.qt_begin[s + 1] = p.qt_begin[s] + static_cast<int32_t>(ceil_div(p.len[L.n - 1 - s], tq));
   const int64_t blocks = static_cast<int64_t>(p.qt_begin[L.n]) * p.n_groups;
   require(blocks <= INT32_MAX, "fused ring: too many workgroups");
-  require(blocks == ring_fused_workgroups(L.hq, L.hkv, L.n, L.len), "fused ring: workgroup count");
+  require(blocks == ring_fused_shape(L.d, L.hq, L.hkv, L.n, L.len, L.causal).workgroups, "fused ring: workgroup count");
   p.trace = L.trace;
   p.trace_stride = L.trace_stride;
   if (L.trace != nullptr) require(L.trace_stride >= kTraceHeaderWords + 2 * L.n, "fused ring: trace stride");
   const dim3 grid(static_cast<unsigned>(blocks));
   if (L.dtype == kBF16) {
-    if (L.trace != nullptr) launch_ring_kernel<kBF16, true>(g, grid, p, stream);
-    else launch_ring_kernel<kBF16, false>(g, grid, p, stream);
+    if (L.trace != nullptr) launch_ring_kernel<kBF16, true>(geo, grid, p, stream);
+    else launch_ring_kernel<kBF16, false>(geo, grid, p, stream);
   } else {
-    if (L.trace != nullptr) launch_ring_kernel<kF16, true>(g, grid, p, stream);
-    else launch_ring_kernel<kF16, false>(g, grid, p, stream);
+    if (L.trace != nullptr) launch_ring_kernel<kF16, true>(geo, grid, p, stream);
+    else launch_ring_kernel<kF16, false>(geo, grid, p, stream);
   }
   HCP_HIP(hipGetLastError());
 }
 
-int64_t ring_fused_workgroups(int hq, int hkv, int n, const int64_t* len) {
-  const Geometry geo = geometry(hq, hkv);
+RingShape ring_fused_shape(int d, int hq, int hkv, int n, const int64_t* len, int causal) {
+  const Geometry geo = ring_geometry(d, hq, hkv, n, len, causal), whole = geometry(hq, hkv);
   int64_t tiles = 0;
   for (int i = 0; i < n; ++i) tiles += ceil_div(len[i], geo.tq);
-  return tiles * geo.n_groups;
+  return {tiles * geo.n_groups, whole.g / geo.g, whole.tq / geo.tq};
 }
 
 int ring_trace_words(int n) { return kTraceHeaderWords + 2 * n; }

@@ -346,6 +346,7 @@ struct TraceState {
   std::vector<int64_t> len;
   std::vector<std::vector<int>> sources;  // per target, ring order
   int64_t blocks = 0;
+  int heads_div = 1, rows_div = 1;  // workgroups per 256-row query tile (short replays: several)
   int stride = 0;
 };
 thread_local TraceState g_trace;
@@ -373,7 +374,8 @@ void run_replay_fused(const hcp_ring_replay_desc* d, const ReplayPlan& p, hcp_ri
   L.lse_hs = p.seq;
   L.len = p.len.data();
   if (g_trace.buf != nullptr) {
-    const int64_t blocks = ring_fused_workgroups(L.hq, L.hkv, p.n, p.len.data());
+    const RingShape shape = ring_fused_shape(L.d, L.hq, L.hkv, p.n, p.len.data(), L.causal);
+    const int64_t blocks = shape.workgroups;
     const int stride = ring_trace_words(p.n);
     const size_t need = static_cast<size_t>(blocks) * stride * sizeof(uint32_t);
     require(g_trace.bytes >= need, "trace buffer too small: need " + std::to_string(need) + " bytes");
@@ -387,6 +389,8 @@ void run_replay_fused(const hcp_ring_replay_desc* d, const ReplayPlan& p, hcp_ri
     g_trace.len = p.len;
     g_trace.sources = p.sources;
     g_trace.blocks = blocks;
+    g_trace.heads_div = shape.heads_div;
+    g_trace.rows_div = shape.rows_div;
     g_trace.stride = stride;
   }
   timed(kTimedBlock, stream, [&] { launch_ring_fused(L, stream); });
@@ -484,6 +488,7 @@ void trace_stats(hipStream_t stream, std::vector<hcp_ring_trace_domain>& doms, h
   doms.assign(t.n, hcp_ring_trace_domain{});
   std::vector<uint64_t> d_first(t.n, UINT64_MAX), d_last(t.n, 0), d_ticks(t.n, 0), d_clk(t.n, 0);
   std::map<uint32_t, std::vector<std::pair<uint64_t, uint64_t>>> per_cu;
+  std::map<uint64_t, int32_t> tiles;
   L = hcp_ring_trace_launch{};
   uint64_t first = UINT64_MAX, last = 0, busy = 0, clk = 0, wmin = UINT64_MAX, wmax = 0;
   for (int64_t r = 0; r < t.blocks; ++r) {
@@ -492,8 +497,13 @@ void trace_stats(hipStream_t stream, std::vector<hcp_ring_trace_domain>& doms, h
     const int dom = static_cast<int>(hdr[10] & 0xffffu);
     require(t1 > t0 && dom < t.n, "incomplete trace record " + std::to_string(r));
     hcp_ring_trace_domain& D = doms[dom];
-    D.workgroups += 1;
-    D.key_tiles += hdr[12];
+    // the workgroups of one 256-row query tile count once, with the longest key range of them
+    int32_t& folded = tiles[(static_cast<uint64_t>(hdr[10]) & 0xffffu) << 48 |
+                            static_cast<uint64_t>((hdr[10] >> 16) / t.heads_div) << 32 | hdr[11] / t.rows_div];
+    D.workgroups += folded == 0;
+    L.workgroups += folded == 0;
+    D.key_tiles += std::max(static_cast<int32_t>(hdr[12]) - folded, 0);
+    folded = std::max(folded, static_cast<int32_t>(hdr[12]));
     uint64_t prev = t0, local = 0, peer = 0;
     for (int s = 0; s < t.n; ++s) {
       const uint64_t st = u64(r, 16 + 2 * s);
@@ -516,7 +526,6 @@ void trace_stats(hipStream_t stream, std::vector<hcp_ring_trace_domain>& doms, h
     wmin = std::min(wmin, t1 - t0);
     wmax = std::max(wmax, t1 - t0);
   }
-  L.workgroups = t.blocks;
   L.cus = static_cast<int32_t>(per_cu.size());
   L.span_ms = (last - first) / kTicksPerMs;
   L.busy_cu_ms = busy / kTicksPerMs;
@@ -1710,7 +1719,8 @@ int hcp_ring_trace_attach(void* buffer, size_t bytes) {
 size_t hcp_ring_trace_record_bytes(const hcp_ring_replay_desc* desc) {
   try {
     const ReplayPlan p = plan_replay(desc, false);
-    const int64_t wg = ring_fused_workgroups(desc->num_q_heads, desc->num_kv_heads, p.n, p.len.data());
+    const int64_t wg = ring_fused_shape(desc->head_dim, desc->num_q_heads, desc->num_kv_heads, p.n, p.len.data(),
+                                        desc->causal).workgroups;
     return static_cast<size_t>(wg) * ring_trace_words(p.n) * sizeof(uint32_t);
   } catch (...) {
     return 0;

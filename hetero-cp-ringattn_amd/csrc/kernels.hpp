@@ -70,8 +70,13 @@ struct RingLaunch {
 };
 bool ring_fused_applies(int dtype, int d);
 void launch_ring_fused(const RingLaunch& L, hipStream_t stream);
-// Workgroups of the fused ring launch for this head layout and chunk list.
-int64_t ring_fused_workgroups(int hq, int hkv, int n, const int64_t* len);
+// Workgroups of the fused ring launch for this head layout and chunk list, and how many of
+// them share a 256-row query tile: head groups (heads_div) times row blocks (rows_div).
+struct RingShape {
+  int64_t workgroups;
+  int heads_div, rows_div;
+};
+RingShape ring_fused_shape(int d, int hq, int hkv, int n, const int64_t* len, int causal);
 // 32-bit words of one trace record of an n-domain fused ring.
 int ring_trace_words(int n);
 

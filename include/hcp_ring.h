@@ -728,8 +728,9 @@ int hcp_ring_replay_timing_read(double* ms, int64_t* launches);
  * ------------------------------------------------------------------------------- */
 typedef struct hcp_ring_trace_domain {
   int32_t domain;
-  int32_t workgroups;
-  int64_t key_tiles;         /* 128-key tiles folded by the domain's workgroups */
+  int32_t workgroups;        /* 256-row query tiles of the domain, one workgroup each or, in a
+                                short replay, several smaller ones (recorded each, counted once) */
+  int64_t key_tiles;         /* 128-key tiles folded per query tile, summed over them */
   int64_t peer_chunks;       /* peer sources folded */
   int64_t kv_recv_bytes;
   int64_t kv_sent_bytes;
@@ -742,7 +743,7 @@ typedef struct hcp_ring_trace_domain {
 } hcp_ring_trace_domain;
 
 typedef struct hcp_ring_trace_launch {
-  int64_t workgroups;
+  int64_t workgroups;        /* query tiles of all domains, as above */
   int32_t cus;               /* distinct CUs that ran a workgroup */
   int32_t reserved0;
   double span_ms;            /* first workgroup start to last workgroup end */

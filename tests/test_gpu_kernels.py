@@ -1425,3 +1425,49 @@ def test_d64_token_major_and_head_major_layouts_agree(gpu, schedule):
         assert torch.equal(o3, o1)
         # 14 head groups of one query head, 256 rows per workgroup
         assert launch["workgroups"] == sum(-(-c // 256) for c in chunks) * 14
+
+
+# Short launches split every tile's keys over 2 or 4 waves (KW): per head layout the
+# smallest shapes (KW = 4) and one that leaves fewer CUs idle (KW = 2); key counts around a
+# part's 32 or 64 keys and a tile's 128, so that whole parts hold no visible key.
+SPLIT_KEY_CASES = [
+    # Hq, Hkv, D, dtype, Lq list, Lk list
+    (8, 1, 128, torch.bfloat16, (1, 33, 130), (1, 31, 33, 65, 129, 300)),
+    (8, 2, 128, torch.float16, (1, 64, 65), (32, 63, 97, 257)),
+    (4, 2, 64, torch.bfloat16, (31, 66), (1, 64, 96, 140)),
+    (3, 3, 96, torch.bfloat16, (63, 200), (33, 128, 161)),
+    (14, 2, 64, torch.bfloat16, (255, 129), (31, 127, 290)),
+    (32, 8, 128, torch.bfloat16, (1000,), (300,)),
+    (16, 8, 128, torch.bfloat16, (1500,), (200,)),
+    (16, 16, 64, torch.float16, (1600,), (130,)),
+]
+
+
+@pytest.mark.parametrize("case", SPLIT_KEY_CASES, ids=[f"{c[0]}q{c[1]}kv_d{c[2]}" for c in SPLIT_KEY_CASES])
+def test_split_key_parts_match_closed_form(gpu, case):
+    # Contiguous and explicit positions, with queries before, among and after the keys, and
+    # merged into a running state; rows that see no key stay (0, -inf).
+    hq, hkv, d, dt, lqs, lks = case
+    scale = 1 / math.sqrt(d)
+    for lq in lqs:
+        for lk in lks:
+            (q, k, v), (q32, k32, v32) = draw(lq + 3 * lk + d, [(lq, hq, d), (lk, hkv, d), (lk, hkv, d)], dt)
+            qv, kv, vv = (x.permute(1, 0, 2) for x in (q, k, v))
+            for qo in (-lq // 2, lk // 2, lk):
+                qp = torch.arange(qo + lq, 2 * lq + qo, device="cuda")
+                kp = torch.arange(lq, lq + lk, device="cuda")
+                ref_o, ref_l = C.attention_f64(q32, k32, v32, np.arange(qo, qo + lq), np.arange(lk), scale)
+                ref_o, ref_l = ref_o.transpose(1, 0, 2), ref_l.T
+                cont = H.block_partial(qv, kv, vv, qo + lq, lq, scale=scale)
+                pos = H.block_partial_positioned(qv, qp, kv, vv, kp, scale=scale)
+                o2, l2 = cont[0].clone(), cont[1].clone()
+                H.block_partial(qv, kv, vv, qo + lq, lq, scale=scale, o=o2, lse=l2, accumulate=True)
+                torch.cuda.synchronize()
+                fin = np.isfinite(ref_l)
+                for (o, l), shift in ((cont, 0.0), (pos, 0.0), ((o2, l2), math.log(2.0))):
+                    o, l = o.cpu().numpy(), l.cpu().numpy()
+                    assert np.array_equal(np.isfinite(l), fin), (lq, lk, qo)
+                    assert np.all(o[~fin] == 0)
+                    assert np.abs(o - ref_o).max() <= OUT_TOL, (lq, lk, qo)
+                    if fin.any():
+                        assert np.abs(l[fin] - ref_l[fin] - shift).max() <= LSE_TOL, (lq, lk, qo)
