@@ -1452,8 +1452,7 @@ static Geometry geometry(int hq, int hkv, int kw = 1) {
   return r;
 }
 
-// Compute units of the current device (256 when none can be queried).
-static int device_cus() {
+int device_cus() {
   static std::atomic<int> known[64];
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess) {

@@ -42,6 +42,9 @@ struct BlockLaunch {
   int64_t alt_hs = 0, alt_ss = 0;
 };
 
+// Compute units of the current device (256 when none can be queried).
+int device_cus();
+
 bool block_uses_mfma(int dtype, int d);
 // Whether an fp32 block runs on the fp32 matrix-core kernel (else the scalar one).
 bool block_uses_mfma_f32(const BlockLaunch& L);

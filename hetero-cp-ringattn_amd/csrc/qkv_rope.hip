@@ -378,6 +378,168 @@ __global__ __launch_bounds__(kQThreads, 1) void qkv_rope_kernel(QkvArgs a) {
   }
 }
 
+// Few tokens (a decode step, the tail of a prompt): the projection reads every weight for
+// a handful of rows, so it is bound by the weights' bytes, and the tiled kernel's few
+// workgroups (24 for a Llama-3-8B layer) leave most CUs idle.  Here a workgroup owns 32
+// features -- 16 and their RoPE partners D/2 above -- times 16 TB tokens, and its 8 waves
+// split the hidden dimension: each wave takes every eighth 64-value slice, streams its
+// weight and token fragments straight from memory into registers (a weight is used by one
+// wave only, so LDS would add nothing), and the eight partial tiles meet in LDS once, in a
+// fixed order.  v_mfma_f32_16x16x32: A = 16 weight rows, B = 16 token rows; a lane owns
+// one token and features 4 (lane / 16) .. + 3 of each 16.
+// Measured on the Llama-3-8B layer (50 MB of weights): 1 token 12.4 us (was 46), 64 tokens
+// 26 us (was 51).  At one token it is at the weights' 10 us; beyond, each workgroup also
+// takes in every token row (8 KiB a token), and the CUs' intake, about 35 GB/s each,
+// bounds it: whole 128-byte lines per load, a per-workgroup rotation of the slices and a
+// deeper weight prefetch all measured the same or slower.
+typedef float qf32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ qf32x4 mma16(bf16x8 a, bf16x8 b, qf32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ qf32x4 mma16(f16x8 a, f16x8 b, qf32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+template <int DT, int D, int TB>
+__global__ __launch_bounds__(kQThreads, 1) void qkv_few_tokens_kernel(QkvArgs a) {
+  using frag = typename QkvMfma<DT>::frag;
+  constexpr int kPerHead = D / 32;           // feature tiles per head
+  constexpr int SG = TB >= 8 ? 2 : 4;        // hidden steps (of 32) per load group
+  constexpr uint32_t kOut = 0x80000000u;     // past every descriptor's records: reads zeros
+  __shared__ __attribute__((aligned(16))) qf32x4 red[kQWaves][2][TB][64];
+
+  const int logical = xcd_remap(blockIdx.x, gridDim.x);  // token tiles of a feature tile share its XCD's L2
+  const int ft = logical / a.n_tiles_m;
+  const int tok0 = (logical - ft * a.n_tiles_m) * 16 * TB;
+  const int head = ft / kPerHead;            // over the q, k and v heads in turn
+  const int d0 = (ft - head * kPerHead) * 16;
+  const int nhq = a.nq / D, nhkv = a.nkv / D;
+  const int which = head < nhq ? 0 : head < nhq + nhkv ? 1 : 2;
+  const int lh = head - (which == 0 ? 0 : which == 1 ? nhq : nhq + nhkv);
+
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int col = lane & 15, grp = lane >> 4;
+
+  const uint16_t* wbase = a.w[which] + (static_cast<int64_t>(lh) * D + d0) * a.hidden;
+  const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(wbase), 0, (D / 2 + 16) * a.hidden * 2, 0x00020000);
+  const int rows = min(a.tokens - tok0, 16 * TB);
+  const uint16_t* xbase = a.x + static_cast<int64_t>(tok0) * a.x_ss;
+  const int x_rb = static_cast<int>(a.x_ss) * 2;
+  const auto xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(xbase), 0, (rows - 1) * x_rb + a.hidden * 2, 0x00020000);
+  const uint32_t w_off = static_cast<uint32_t>(col * a.hidden * 2 + grp * 16);
+  const uint32_t x_off = static_cast<uint32_t>(col * x_rb + grp * 16);
+
+  // Slice s of the hidden dimension is steps 2s and 2s + 1 (64 values, a 128-byte line of
+  // each row); this wave's j-th step is step 2 (wave + 8 (j / 2)) + j % 2.
+  const int n_st = a.hidden / kQK;
+  const int n_sl = (n_st + 1) / 2;
+  const int mine = wave < n_sl ? 2 * ((n_sl - wave + kQWaves - 1) / kQWaves) : 0;
+  struct Group {
+    u32x4 w[SG][2];
+    u32x4 x[SG][TB];
+  };
+  auto load = [&](int j0, Group& g) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < SG; ++j) {
+      const int st = 2 * (wave + kQWaves * ((j0 + j) / 2)) + (j & 1);
+      const uint32_t k = st < n_st ? static_cast<uint32_t>(st) * (kQK * 2) : kOut;
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        g.w[j][b] = __builtin_amdgcn_raw_buffer_load_b128(wr, w_off + k + static_cast<uint32_t>(b * (D / 2) * a.hidden * 2), 0, 0);
+#pragma unroll
+      for (int t = 0; t < TB; ++t)
+        g.x[j][t] = __builtin_amdgcn_raw_buffer_load_b128(xr, x_off + k + static_cast<uint32_t>(16 * t * x_rb), 0, 0);
+    }
+  };
+  qf32x4 acc[2][TB];
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int t = 0; t < TB; ++t) acc[b][t] = qf32x4{0.f, 0.f, 0.f, 0.f};
+  auto fold = [&](const Group& g) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < SG; ++j)
+#pragma unroll
+      for (int t = 0; t < TB; ++t)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+          acc[b][t] = mma16(__builtin_bit_cast(frag, g.w[j][b]), __builtin_bit_cast(frag, g.x[j][t]), acc[b][t]);
+  };
+  Group ga, gb;
+  load(0, ga);
+  for (int j0 = 0; j0 < mine; j0 += 2 * SG) {
+    load(j0 + SG, gb);
+    fold(ga);
+    load(j0 + 2 * SG, ga);
+    fold(gb);
+  }
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int t = 0; t < TB; ++t) red[wave][b][t][lane] = acc[b][t];
+  __syncthreads();
+
+  // ---- epilogue: wave t finishes token block t ----
+  if (wave >= TB) return;
+  const int t = tok0 + 16 * wave + col;
+  if (t >= a.tokens) return;
+  float v[2][4];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    qf32x4 sum = red[0][b][wave][lane];
+#pragma unroll
+    for (int w = 1; w < kQWaves; ++w) sum += red[w][b][wave][lane];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[b][i] = sum[i];
+  }
+  const int dh = d0 + 4 * grp;               // head dims dh .. + 3 and their partners + D/2
+  if (const uint16_t* bias = a.bias[which]) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[b][i] += ld16<DT>(bias + lh * D + dh + b * (D / 2) + i);
+  }
+  if (a.rope && which < 2) {
+    const int64_t p = a.pos[t];
+    if (p < 0 || p >= a.rope_rows) {
+      if (grp == 0) atomicOr(a.err, 4);
+    } else {
+      const float4 cs = *reinterpret_cast<const float4*>(a.rope_cos + p * (D / 2) + dh);
+      const float4 sn = *reinterpret_cast<const float4*>(a.rope_sin + p * (D / 2) + dh);
+      const float cc[4] = {cs.x, cs.y, cs.z, cs.w}, ss[4] = {sn.x, sn.y, sn.z, sn.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float x1 = v[0][i], x2 = v[1][i];
+        v[0][i] = x1 * cc[i] - x2 * ss[i];
+        v[1][i] = x1 * ss[i] + x2 * cc[i];
+      }
+    }
+  }
+  uint16_t* row;
+  if (which == 0 || a.pool == nullptr) {
+    row = a.out[which] + lh * a.out_hs[which] + static_cast<int64_t>(t) * a.out_ss[which];
+  } else {
+    const int64_t sp = a.t0 + t - a.table_off;  // position of this token in the table
+    const int64_t entry = sp / a.bs;
+    const int32_t blk = (sp >= 0 && entry < a.table_len) ? a.table[entry] : -1;
+    if (blk < 0 || blk >= a.num_blocks) {
+      if (grp == 0) atomicOr(a.err, 1);
+      return;
+    }
+    row = a.pool + (which == 2 ? a.plane_elems : 0) +
+          ((static_cast<int64_t>(blk) * a.bs + (sp - entry * a.bs)) * a.hkv + lh) * D;
+  }
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    u32x2 w;
+    w[0] = pack2<DT>(v[b][0], v[b][1]);
+    w[1] = pack2<DT>(v[b][2], v[b][3]);
+    *reinterpret_cast<u32x2*>(row + dh + b * (D / 2)) = w;
+  }
+}
+
 constexpr int kRopeThreads = 256;
 struct RopeArgs {
   float inv_freq[128];
@@ -424,10 +586,7 @@ void launch_rope_table(int d, int64_t rows, double base, float* cos, float* sin,
 // earlier model, 1.57 and whole rounds, missed 4096, 6144 and 24576 tokens by 7-12%).
 // Llama-3-8B at 12288 tokens: 768 tiles of 384 are 3 full rounds of 256 CUs.
 static int qkv_token_tile(int64_t tiles_f, int64_t tokens) {
-  int dev = 0, cus = 0;
-  HCP_HIP(hipGetDevice(&dev));
-  HCP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  if (cus <= 0) return 256;
+  const int cus = device_cus();
   const int tn[3] = {128, 256, 384};
   const double cost[3] = {0.62, 1.0, 1.41};
   int best = 1;
@@ -445,8 +604,46 @@ static int qkv_token_tile(int64_t tiles_f, int64_t tokens) {
   return tn[best];
 }
 
+template <int TB>
+static void launch_few_tokens(int dtype, int d, const QkvArgs& a, unsigned grid, hipStream_t stream) {
+  if (dtype == kBF16) {
+    if (d == 128) qkv_few_tokens_kernel<kBF16, 128, TB><<<grid, kQThreads, 0, stream>>>(a);
+    else qkv_few_tokens_kernel<kBF16, 64, TB><<<grid, kQThreads, 0, stream>>>(a);
+  } else {
+    if (d == 128) qkv_few_tokens_kernel<kF16, 128, TB><<<grid, kQThreads, 0, stream>>>(a);
+    else qkv_few_tokens_kernel<kF16, 64, TB><<<grid, kQThreads, 0, stream>>>(a);
+  }
+}
+
+// Token blocks (of 16) per workgroup of the few-tokens kernel, 0 where the tiled kernel is
+// the faster one.  The few-tokens kernel wins as long as its workgroups fit one round of
+// the CUs, or take one token tile: every further round costs another pass over the
+// weights.  Measured, tiled / few: 32/8 heads of 128, hidden 4096: 46 / 12 us at 1 token,
+// 47 / 19 at 32, 51 / 26 at 64, 55 / 41 at 128 (192 workgroups), 54 / 78 at 200; 16/2
+// heads, hidden 2048: 36 / 23 at 256 (160 workgroups), 35 / 43 at 400 (320); 14/2 heads of
+// 64, hidden 896: 23 / 14 at 512 (144), 24 / 25 at 1024 (288).  Its per-lane offsets are
+// 32-bit: the weight rows of a head and 128 token rows must span less than 2 GiB.
+static int few_token_blocks(int64_t n_feat, int64_t tokens, int d, int64_t hidden, int64_t x_ss, int cus) {
+  constexpr int64_t kSpan = int64_t(1) << 31;
+  if (d * hidden * 2 >= kSpan || x_ss >= kSpan / 256) return 0;
+  if (tokens > 128 && n_feat / 32 * ceil_div(tokens, 128) > cus) return 0;
+  return tokens <= 16 ? 1 : tokens <= 32 ? 2 : tokens <= 64 ? 4 : 8;
+}
+
 void launch_qkv_rope(int dtype, int d, QkvArgs& a, hipStream_t stream) {
   const int n_feat = a.nq + 2 * a.nkv;
+  if (a.tokens == 0) return;
+  if (const int tb = few_token_blocks(n_feat, a.tokens, d, a.hidden, a.x_ss, device_cus())) {
+    a.n_tiles_n = n_feat / 32;
+    a.n_tiles_m = static_cast<int32_t>(ceil_div(a.tokens, 16 * tb));
+    const unsigned grid = static_cast<unsigned>(a.n_tiles_n * a.n_tiles_m);
+    if (tb == 1) launch_few_tokens<1>(dtype, d, a, grid, stream);
+    else if (tb == 2) launch_few_tokens<2>(dtype, d, a, grid, stream);
+    else if (tb == 4) launch_few_tokens<4>(dtype, d, a, grid, stream);
+    else launch_few_tokens<8>(dtype, d, a, grid, stream);
+    HCP_HIP(hipGetLastError());
+    return;
+  }
   a.n_tiles_n = static_cast<int32_t>(ceil_div(n_feat, kQTileF));
   const int tn = qkv_token_tile(a.n_tiles_n, a.tokens);
   a.n_tiles_m = static_cast<int32_t>(ceil_div(a.tokens, tn));

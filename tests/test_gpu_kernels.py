@@ -1471,3 +1471,58 @@ def test_split_key_parts_match_closed_form(gpu, case):
                     assert np.abs(o - ref_o).max() <= OUT_TOL, (lq, lk, qo)
                     if fin.any():
                         assert np.abs(l[fin] - ref_l[fin] - shift).max() <= LSE_TOL, (lq, lk, qo)
+
+
+# The few-tokens projection at the edges of its 16-token blocks (1, 2, 4 or 8 of them per
+# workgroup, several token tiles), with one and three 32-value hidden steps, an odd and an
+# even number of 64-value slices, and more slices than waves; and the tiled one (the
+# workgroups of the last two no longer fit one round of the CUs) with a ragged last tile.
+QKV_EDGE_CASES = [
+    # tokens, hidden, Hq, Hkv, D, dtype, paged
+    (1, 32, 2, 1, 128, torch.bfloat16, False),
+    (15, 96, 4, 2, 64, torch.float16, True),
+    (17, 64, 8, 2, 128, torch.bfloat16, True),
+    (33, 544, 14, 2, 64, torch.bfloat16, False),
+    (64, 1152, 4, 4, 128, torch.float16, False),
+    (65, 160, 8, 2, 128, torch.bfloat16, True),
+    (129, 128, 2, 2, 64, torch.bfloat16, False),
+    (1300, 160, 8, 2, 128, torch.bfloat16, True),
+    (2100, 96, 14, 2, 64, torch.float16, False),
+]
+
+
+@pytest.mark.parametrize("case", QKV_EDGE_CASES, ids=[f"{c[0]}x{c[1]}_{c[2]}q{c[3]}kv_d{c[4]}" for c in QKV_EDGE_CASES])
+def test_qkv_rope_token_count_edges(gpu, case):
+    # Padded x rows hold NaN past the hidden dimension and after the last token: nothing
+    # outside x may reach a result.  Views 8- but not 16-byte aligned; against float64.
+    tokens, hidden, hq, hkv, d, dtype, paged = case
+    x, ws, bs = _qkv_inputs(tokens, hidden, hq, hkv, d, dtype, True, 400 + tokens)
+    xp = torch.full((tokens + 16, hidden + 24), float("nan"), dtype=dtype, device="cuda")
+    xp[:tokens, :hidden] = x.cuda()
+    xp = xp[:tokens, :hidden]
+    wd, bd = [w.cuda() for w in ws], [b.cuda() for b in bs]
+    table = H.rope_table(d, 4096, 10000.0)
+    pos = torch.arange(5, 5 + tokens, dtype=torch.int64, device="cuda")
+    q = torch.zeros(hq, tokens, d + 4, dtype=dtype, device="cuda")[:, :, 4:]
+    if paged:
+        nb = -(-(tokens + 3) // 16)
+        pool = torch.zeros(2, nb + 2, 16, hkv, d, dtype=dtype, device="cuda")
+        blocks = torch.arange(nb, -1, -1, dtype=torch.int32, device="cuda")
+        H.qkv_rope_project_paged(xp, *wd, hq, hkv, d, pool, blocks, 0, 3, positions=pos, table=table, bq=bd[0],
+                                 bk=bd[1], bv=bd[2], q_out=q)
+        k, v = H.paged_kv_gather(pool, blocks, 0, 3, 3 + tokens)
+    else:
+        k, v = (torch.zeros(hkv, tokens, d + 4, dtype=dtype, device="cuda")[:, :, 4:] for _ in range(2))
+        H.qkv_rope_project(xp, *wd, hq, hkv, d, positions=pos, table=table, bq=bd[0], bk=bd[1], bv=bd[2], q_out=q,
+                           k_out=k, v_out=v)
+    torch.cuda.synchronize()
+    assert H.fetch_device_errors() == 0
+    cos, sin = (table[i].cpu().double()[5: 5 + tokens] for i in range(2))
+    for i, (got, w, b) in enumerate(zip((q, k, v), ws, bs)):
+        y = (x.double() @ w.double().T + b.double()).view(tokens, -1, d).permute(1, 0, 2)
+        if i < 2:
+            y1, y2 = y[..., : d // 2], y[..., d // 2:]
+            y = torch.cat([y1 * cos - y2 * sin, y1 * sin + y2 * cos], -1)
+        # one rounding to the storage type (2^-8 bf16, 2^-11 fp16 of the value), fp32 sums below that
+        bound = y.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) + 1e-5 * y.abs().max()
+        assert bool(((got.cpu().double() - y).abs() <= bound).all()), i
