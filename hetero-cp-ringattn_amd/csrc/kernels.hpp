@@ -9,6 +9,8 @@
 
 namespace hcp {
 
+constexpr int kMaxDomains = 64;
+
 // One (query chunk, KV chunk) block partial; see block_attn.hip.
 struct BlockLaunch {
   int dtype;
@@ -105,16 +107,25 @@ void launch_paged_copy(bool gather, void* pool, int64_t num_blocks, int bs, int 
                        int64_t t1, void* k_buf, void* v_buf, int64_t head_stride, int64_t seq_stride,
                        int zero_tail, int* err, hipStream_t stream);
 
-size_t decode_workspace_bytes(int dtype, int batch, int hq, int hkv, int d, int64_t t0, int64_t t1);
+// One shard of every sequence's paged KV: tokens [t0, min(t1, seq_lens[b])) through row b
+// of its block tables.
+struct DecodeSpan {
+  const int32_t* tables;
+  int64_t table_stride, table_len;
+  const int32_t* seq_lens;  // or null
+  int64_t t0, t1;
+};
+// Workspace of launch_paged_decode for these shards.
+size_t decode_workspace_bytes(int dtype, int batch, int hq, int hkv, int d, int n, const DecodeSpan* spans);
+// Attention of one query per sequence over its n shards, merged: out[row * out_rs + d] in
+// out_dtype and lse[row] (fp32, may be null) for row = b * hq + head.
 void launch_paged_decode(int dtype, int batch, int hq, int hkv, int d, const void* q, int64_t q_bs,
-                         int64_t q_hs, const void* pool, int64_t num_blocks, int bs,
-                         const int32_t* tables, int64_t table_stride, int64_t table_len,
-                         const int32_t* seq_lens, int64_t t0, int64_t t1, float scale, float* o,
-                         float* lse, void* ws, size_t ws_bytes, int* err, hipStream_t stream);
+                         int64_t q_hs, const void* pool, int64_t num_blocks, int bs, int n,
+                         const DecodeSpan* spans, float scale, int out_dtype, void* out, int64_t out_rs, float* lse,
+                         void* ws, size_t ws_bytes, int* err, hipStream_t stream);
 
 // Scheduling strategies (strategy.rs:14-24) and their closed-form positions; see
 // positions.hip.
-constexpr int kMaxDomains = 64;
 enum Strategy : int32_t { kStrategyVanilla = 0, kStrategyStriped = 1, kStrategyZigZag = 2 };
 struct StrategySpec {
   int32_t strategy;

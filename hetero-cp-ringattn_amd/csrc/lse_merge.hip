@@ -39,6 +39,91 @@ __device__ __forceinline__ float4 nt_load4(const float* p) {
   return make_float4(x[0], x[1], x[2], x[3]);
 }
 
+// Four consecutive values of a merged row in the output type.
+template <int OUT_DT>
+__device__ __forceinline__ void store_row4(void* out, int64_t at, float4 x) {
+  if constexpr (OUT_DT == kF32) {
+    store16_nt_sc1(static_cast<float*>(out) + at, __builtin_bit_cast(u32x4, x));
+  } else {
+    u32x2 w;
+    if constexpr (OUT_DT == kBF16) {
+      w[0] = static_cast<uint32_t>(f32_to_bf16_bits(x.x)) | (static_cast<uint32_t>(f32_to_bf16_bits(x.y)) << 16);
+      w[1] = static_cast<uint32_t>(f32_to_bf16_bits(x.z)) | (static_cast<uint32_t>(f32_to_bf16_bits(x.w)) << 16);
+    } else {
+      w[0] = static_cast<uint32_t>(f32_to_f16_bits(x.x)) | (static_cast<uint32_t>(f32_to_f16_bits(x.y)) << 16);
+      w[1] = static_cast<uint32_t>(f32_to_f16_bits(x.z)) | (static_cast<uint32_t>(f32_to_f16_bits(x.w)) << 16);
+    }
+    store8_nt_sc1(static_cast<uint16_t*>(out) + at, w);
+  }
+}
+
+// Few rows, several partials (a decode step): one row per workgroup, whose 256 / lpr slots
+// take every so-manieth partial with all their loads in flight, and meet in LDS.  The
+// kernel below walks a row's partials in groups of 8, one memory latency each, on a handful
+// of workgroups: that chain, not the bytes, bounds it (19 partials of 64 rows: 9.4 us).
+// Decode steps with it and without: 4 sequences of 2085 tokens 18.9 / 23.7 us (32/8 heads),
+// 4 of 16384 28.0 / 34.1 us (16/2 heads).
+template <int OUT_DT>
+__global__ __launch_bounds__(256) void lse_merge_few_rows_kernel(MergeArgs a) {
+  constexpr int NP = 4;  // partials of a slot in flight together
+  __shared__ float4 acc_l[256];
+  __shared__ float m_l[256], den_l[256];
+  const int lpr = a.lanes_per_row;
+  const int slots = 256 / lpr;
+  const int64_t row = blockIdx.x;
+  const int slot = threadIdx.x / lpr;
+  const int c = threadIdx.x % lpr * 4;
+  const bool active = c < a.d;
+  float m = -INFINITY, den = 0.f;
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int base = slot; base < a.n; base += NP * slots) {
+    float l[NP];
+    float4 v[NP];
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      const int i = base + u * slots;
+      l[u] = i < a.n ? a.lse[i][row] : -INFINITY;
+      v[u] = i < a.n && active ? nt_load4(a.o[i] + row * a.d + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    float mn = m;
+#pragma unroll
+    for (int u = 0; u < NP; ++u) mn = fmaxf(mn, l[u]);
+    if (mn == -INFINITY) continue;  // every partial so far is empty
+    const float sc = __expf(m - mn);
+    den *= sc;
+    acc.x *= sc; acc.y *= sc; acc.z *= sc; acc.w *= sc;
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      const float w = __expf(l[u] - mn);
+      den += w;
+      acc.x += w * v[u].x; acc.y += w * v[u].y; acc.z += w * v[u].z; acc.w += w * v[u].w;
+    }
+    m = mn;
+  }
+  acc_l[threadIdx.x] = acc;
+  m_l[threadIdx.x] = m;
+  den_l[threadIdx.x] = den;
+  __syncthreads();
+  if (slot != 0) return;
+  float mt = -INFINITY;
+  for (int s = 0; s < slots; ++s) mt = fmaxf(mt, m_l[threadIdx.x + s * lpr]);
+  float dt = 0.f;
+  float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (mt != -INFINITY) {
+    for (int s = 0; s < slots; ++s) {
+      const float w = __expf(m_l[threadIdx.x + s * lpr] - mt);
+      const float4 x = acc_l[threadIdx.x + s * lpr];
+      dt += w * den_l[threadIdx.x + s * lpr];
+      o.x += w * x.x; o.y += w * x.y; o.z += w * x.z; o.w += w * x.w;
+    }
+  }
+  const float inv = dt > 0.f ? 1.f / dt : 0.f;
+  const int64_t h = row / a.q_len, t = row - h * a.q_len;
+  if (active)
+    store_row4<OUT_DT>(a.out, h * a.out_hs + t * a.out_ss + c, make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv));
+  if (a.lse_out != nullptr && threadIdx.x == 0) a.lse_out[h * a.lse_out_hs + t] = dt > 0.f ? mt + __logf(dt) : -INFINITY;
+}
+
 template <int OUT_DT, int NP, int R>
 __global__ __launch_bounds__(256) void lse_merge_kernel(MergeArgs a) {
   const int lpr = a.lanes_per_row;
@@ -109,27 +194,7 @@ __global__ __launch_bounds__(256) void lse_merge_kernel(MergeArgs a) {
     const float inv = (any && den[k] > 0.f) ? 1.f / den[k] : 0.f;
     if (active) {
       const int64_t base = h * a.out_hs + t * a.out_ss + c;
-      if constexpr (OUT_DT == kF32) {
-        store16_nt_sc1(static_cast<float*>(a.out) + base,
-                       __builtin_bit_cast(u32x4, make_float4(acc[k].x * inv, acc[k].y * inv, acc[k].z * inv, acc[k].w * inv)));
-      } else {
-        uint16_t b0, b1, b2, b3;
-        if constexpr (OUT_DT == kBF16) {
-          b0 = f32_to_bf16_bits(acc[k].x * inv);
-          b1 = f32_to_bf16_bits(acc[k].y * inv);
-          b2 = f32_to_bf16_bits(acc[k].z * inv);
-          b3 = f32_to_bf16_bits(acc[k].w * inv);
-        } else {
-          b0 = f32_to_f16_bits(acc[k].x * inv);
-          b1 = f32_to_f16_bits(acc[k].y * inv);
-          b2 = f32_to_f16_bits(acc[k].z * inv);
-          b3 = f32_to_f16_bits(acc[k].w * inv);
-        }
-        uint2 packed;
-        packed.x = static_cast<uint32_t>(b0) | (static_cast<uint32_t>(b1) << 16);
-        packed.y = static_cast<uint32_t>(b2) | (static_cast<uint32_t>(b3) << 16);
-        store8_nt_sc1(static_cast<uint16_t*>(a.out) + base, u32x2{packed.x, packed.y});
-      }
+      store_row4<OUT_DT>(a.out, base, make_float4(acc[k].x * inv, acc[k].y * inv, acc[k].z * inv, acc[k].w * inv));
     }
     if (a.lse_out != nullptr && lane_in_row == 0) {
       a.lse_out[h * a.lse_out_hs + t] = (any && den[k] > 0.f) ? m[k] + __logf(den[k]) : -INFINITY;
@@ -166,6 +231,21 @@ void launch_lse_merge(int n, const float* const* o_parts, const float* const* ls
   constexpr int R = HCP_MERGE_R;
   const int64_t threads = ceil_div(static_cast<int64_t>(heads) * q_len, R) * lpr;
   const dim3 grid(static_cast<unsigned>(ceil_div(threads, 256)));
+  const int64_t rows = static_cast<int64_t>(heads) * q_len;
+  // Up to four partials the kernel below has all loads of a row in flight too, and from
+  // 2048 rows on it has the workgroups (a decode step of 64 sequences x 32 heads: 165 us
+  // either way; of 16: 55 us with it, 52 with one row per workgroup).
+  if (n > 4 && rows <= 1024) {
+    const dim3 g(static_cast<unsigned>(rows));
+    switch (out_dtype) {
+      case kBF16: lse_merge_few_rows_kernel<kBF16><<<g, 256, 0, stream>>>(a); break;
+      case kF16: lse_merge_few_rows_kernel<kF16><<<g, 256, 0, stream>>>(a); break;
+      case kF32: lse_merge_few_rows_kernel<kF32><<<g, 256, 0, stream>>>(a); break;
+      default: throw Error(-6, "lse_merge: out_dtype must be BF16, F16 or F32");
+    }
+    HCP_HIP(hipGetLastError());
+    return;
+  }
   // Group size: all partials in one group up to 4, else groups of 8.
   auto go = [&](auto np) {
     constexpr int NP = decltype(np)::value;

@@ -7,12 +7,16 @@
 // sequence's block table -- no gather, no GQA expand copy.
 //
 // Work split (HBM-bound: every K/V byte is read exactly once):
-//   * grid = (splits, batch, ceil(Hkv / W)) with W = min(8, Hkv) waves per workgroup, so one
-//     workgroup reads whole pool token rows (4 waves: 0.7% slower on c4).
-//     A workgroup owns one sequence, a contiguous run of 16-token groups of the chunk
-//     and W kv heads: wave w handles kv head W*blockIdx.z + w, so per 16 tokens a wave
-//     reads 16 K rows and 16 V rows of its head (4 KiB each for D=128, bf16) straight
-//     from the pool.
+//   * One launch covers every shard of every sequence (a decode partial has one shard, the
+//     decode Q-ring one per domain).  A sequence's 16-token groups, shard after shard, are
+//     dealt out in equal contiguous runs to `parts` x `subs` waves, whatever its own
+//     length; grid = (parts, batch, ceil(Hkv / heads)), a workgroup holding `heads` kv
+//     heads x `subs` runs of one part.  The subs of a part meet in LDS, the parts in the
+//     LSE merge kernel.  The number of runs fills the chip once (see plan_decode): with a
+//     few sequences a run is down to one group.
+//   * Per 16 tokens a wave reads 16 K rows and 16 V rows of its head (4 KiB each for D=128,
+//     bf16) straight from the pool; with many sequences a workgroup reads whole pool token
+//     rows (heads = min(8, Hkv); 4 heads a workgroup: 0.7% slower on c4).
 //   * Scores: S^T = K Q^T on MFMA 16x16x32 (A = 16 key rows loaded from the pool, 16
 //     bytes per lane; B = the rep <= 16 query heads of the kv head -- the GQA group of
 //     repeat_decode_kv_heads, ring.rs:496-512 -- zero-padded to 16 columns, held in
@@ -21,13 +25,15 @@
 //     slot (broadcast reads) and PV runs on VALU with each lane owning 8 head-dim
 //     values of 4 of the 16 keys for R query heads (R = 4, 8 or 16, the smallest that
 //     holds rep; fp32 accumulators), reduced across lanes once at the end.
-//   * Each split writes (o, lse) to the workspace; the LSE merge kernel combines the
-//     splits of a sequence (heads = batch*Hq, q_len = 1).
+//   * Each part writes (o, lse) to the workspace; the LSE merge kernel combines the
+//     parts of a sequence (heads = batch*Hq, q_len = 1).
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <tuple>
 
 #include "kernels.hpp"
+#include "../../include/hcp_ring.h"
 
 namespace hcp {
 
@@ -38,21 +44,20 @@ struct DecodeArgs {
   int64_t plane_elems;
   int64_t num_blocks;
   int32_t bs, hkv, hq, rep;
-  const int32_t* tables;
-  int64_t table_stride, table_len;
-  const int32_t* seq_lens;
-  int64_t t0, t1;
-  int64_t g_begin;      // first 16-token group index (t0 / 16)
-  int32_t groups_per_split;
-  int32_t n_groups;     // total groups in [g_begin*16, t1)
+  DecodeSpan span[kMaxDomains];  // shards in merge order
+  int32_t n_spans;
+  int32_t heads, subs;  // kv heads and runs per workgroup
+  int32_t gpb;          // 16-token groups per block (bs / 16)
+  int32_t gpb_shift;    // its log2, or -1
   float scale_log2;
-  float* ws_o;          // [splits][batch*hq][D]
-  float* ws_lse;        // [splits][batch*hq]
+  float* ws_o;          // [parts][batch*hq][D]
+  float* ws_lse;        // [parts][batch*hq]
   int32_t batch;
   int* err;
   int32_t dn;           // head dim of the pool rows, q and the partials (the D=128 kernel:
                         // any multiple of 8 up to 128, columns past it read as zeros)
 };
+static_assert(sizeof(DecodeArgs) <= 4096, "kernel arguments are limited to 4 KiB");
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
@@ -77,9 +82,10 @@ __device__ __forceinline__ float hi_half(uint32_t w) {
   return DT == kBF16 ? __uint_as_float(w & 0xffff0000u) : f16_bits_to_f32(static_cast<uint16_t>(w >> 16));
 }
 
-constexpr int kDecWaves = 8;  // most kv heads per workgroup (one per wave)
+constexpr float kNoMax = -1.0e30f;
+constexpr int kDecWaves = 8;  // most waves per workgroup
 
-// One wave per kv head.  Per 16-key group the wave needs the head's 16 K rows and 16 V
+// One wave per kv head and run.  Per 16-key group the wave needs the head's 16 K rows and 16 V
 // rows (4 KiB each for D=128); the next group's loads are issued before a group is
 // computed, and the block ids come from one table load per 64 groups.
 template <int D, int DT, int R, bool PAD>
@@ -91,12 +97,16 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(DecodeArgs a) {
   constexpr int TPL = 16 * DCH / 64;  // keys per lane in PV (4 for D=128)
 
   __shared__ __attribute__((aligned(16))) float p_lds[kDecWaves][16][R];  // [wave][key][query col]
+  __shared__ __attribute__((aligned(16))) float o_lds[kDecWaves][R][D];   // subs > 1: the waves' O, m and l
+  __shared__ float m_lds[kDecWaves][R], l_lds[kDecWaves][R];
 
   const int b = blockIdx.y;
-  const int split = blockIdx.x;
+  const int part = blockIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kvh = blockIdx.z * (blockDim.x >> 6) + wave;
-  if (kvh >= a.hkv) return;  // no workgroup barriers below
+  const int sub = wave / a.heads;
+  const int kvh = blockIdx.z * a.heads + wave - sub * a.heads;
+  const bool idle = kvh >= a.hkv;
+  if (idle && a.subs == 1) return;  // no workgroup barrier below
   const int lane = threadIdx.x & 63;
   const int col = lane & 15;   // MFMA column = query head within the kv group
   const int grp = lane >> 4;   // MFMA k-group / key group
@@ -104,21 +114,30 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(DecodeArgs a) {
   const int pv_dc = lane % DCH;
   const int pv_tg = lane / DCH;
 
-  int64_t t_end = a.t1;
-  if (a.seq_lens != nullptr) t_end = min(t_end, static_cast<int64_t>(a.seq_lens[b]));
-  const int g0 = split * a.groups_per_split;
-  // Stop at this sequence's own last group: table entries past its length may be
-  // padding (ragged batches) and are neither read nor validated.
-  const int64_t g_seq = t_end > a.t0 ? (t_end + 15) / 16 - a.g_begin : 0;
-  const int g1 = static_cast<int>(min(static_cast<int64_t>(min(a.n_groups, g0 + a.groups_per_split)), g_seq));
-  const int32_t* table = a.tables + static_cast<int64_t>(b) * a.table_stride;
+  // Tokens and 16-token groups of this sequence in shard s: table entries past its own
+  // last group may be padding (ragged batches) and are neither read nor validated.
+  auto span_end = [&](int s) __attribute__((always_inline)) -> int64_t {
+    const DecodeSpan& sp = a.span[s];
+    if (sp.seq_lens == nullptr) return sp.t1;
+    return min(sp.t1, static_cast<int64_t>(__builtin_amdgcn_readfirstlane(sp.seq_lens[b])));
+  };
+  auto span_groups = [&](int s, int64_t t_end) __attribute__((always_inline)) {
+    const int64_t t0 = a.span[s].t0;
+    return t_end > t0 ? static_cast<int>((t_end + 15) / 16 - t0 / 16) : 0;
+  };
+  int total = 0;
+  for (int s = 0; s < a.n_spans; ++s) total += span_groups(s, span_end(s));
+  const int runs = gridDim.x * a.subs;
+  const int run_len = (total + runs - 1) / runs;
+  const int g0 = idle ? total : min((part * a.subs + sub) * run_len, total);
+  const int g1 = min(g0 + run_len, total);
 
   // Q^T fragments: lane (col, grp) holds Q[head kvh*rep + col][grp*8 + 32*s .. +8].
   u32x4 qf[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
     u32x4 v = {0, 0, 0, 0};
-    if (col < a.rep && (!PAD || grp * 8 + 32 * s < dn))
+    if (!idle && col < a.rep && (!PAD || grp * 8 + 32 * s < dn))
       v = *reinterpret_cast<const u32x4*>(a.q + b * a.q_bs + (kvh * a.rep + col) * a.q_hs + grp * 8 + 32 * s);
     qf[s] = v;
   }
@@ -129,43 +148,63 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(DecodeArgs a) {
   for (int c = 0; c < R; ++c)
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[c][e] = 0.f;
-  float m_run = -1.0e30f, l_run = 0.f;
+  float m_run = kNoMax, l_run = 0.f;
 
   const int64_t row_elems = static_cast<int64_t>(a.hkv) * dn;  // one slot, all heads
 
   struct Group {
     u32x4 k[KS];
     u32x4 v[TPL];
-    int64_t tok0;
+    int lo, hi;  // keys [lo, hi) of the group count
     bool ok;
   };
-  // Block ids of the split's groups, 64 at a time: lane i holds the table entry of
-  // group ids_base + i, read back with readlane, so no group waits on a table load.
-  // Keys tok0 .. tok0+15 of group g lie in table entry tok0 / bs (bs is a multiple of 16).
-  int ids = -1, ids_base = g0 - 64;
-  auto block_of = [&](int g, int64_t entry) __attribute__((always_inline)) {
+  // Cursor over the shards: groups [s_begin, s_end) of the sequence lie in shard s.
+  int s = -1, s_begin = 0, s_end = 0;
+  int64_t t_end = 0, t_beg = 0;
+  int g_first = 0;                  // first group of the shard (t0 / 16)
+  const int32_t* table = nullptr;
+  int64_t table_len = 0;
+  // Block ids of the run's groups, 64 at a time: lane i holds the table entry of group
+  // ids_base + i, read back with readlane, so no group waits on a table load.  Keys of a
+  // group lie in one table entry (bs is a multiple of 16).
+  int ids = -1, ids_base = -64;
+  auto load_group = [&](int g, Group& G) {
+    if (g >= s_end) {
+      do {
+        ++s;
+        s_begin = s_end;
+        t_end = span_end(s);
+        s_end += span_groups(s, t_end);
+      } while (g >= s_end);
+      const DecodeSpan& sp = a.span[s];
+      t_beg = sp.t0;
+      g_first = static_cast<int>(t_beg / 16);
+      table = sp.tables + static_cast<int64_t>(b) * sp.table_stride;
+      table_len = sp.table_len;
+      ids_base = g - 64;
+    }
     if (g - ids_base >= 64) {
       ids_base = g;
-      const int64_t e = (a.g_begin + g + lane) * 16 / a.bs;
-      ids = g + lane < g1 && e < a.table_len ? table[e] : -1;
+      const int gl = g_first + g - s_begin + lane;
+      const int e = a.gpb_shift >= 0 ? gl >> a.gpb_shift : gl / a.gpb;
+      ids = g + lane < min(g1, s_end) && e < table_len ? table[e] : -1;
     }
     const int32_t blk = __builtin_amdgcn_readlane(ids, g - ids_base);
-    return entry < a.table_len ? blk : -1;
-  };
-  auto load_group = [&](int g, Group& G) {
-    G.tok0 = (a.g_begin + g) * 16;
-    const int64_t entry = G.tok0 / a.bs;
-    const int32_t blk = block_of(g, entry);
+    const int gl = g_first + g - s_begin;
+    const int entry = a.gpb_shift >= 0 ? gl >> a.gpb_shift : gl / a.gpb;
+    const int64_t tok0 = static_cast<int64_t>(gl) * 16;
+    G.lo = __builtin_amdgcn_readfirstlane(static_cast<int>(t_beg > tok0 ? t_beg - tok0 : 0));
+    G.hi = __builtin_amdgcn_readfirstlane(static_cast<int>(min(t_end - tok0, static_cast<int64_t>(16))));
     G.ok = blk >= 0 && blk < a.num_blocks;
     if (!G.ok) {
-      if (lane == 0 && entry < a.table_len) atomicOr(a.err, 1);
+      if (lane == 0 && entry < table_len) atomicOr(a.err, 1);
 #pragma unroll
       for (int s = 0; s < KS; ++s) G.k[s] = u32x4{0, 0, 0, 0};
 #pragma unroll
       for (int j = 0; j < TPL; ++j) G.v[j] = u32x4{0, 0, 0, 0};
       return;
     }
-    const int slot0 = static_cast<int>(G.tok0 - entry * a.bs);
+    const int slot0 = (gl - entry * a.gpb) * 16;
     const uint16_t* kslot = a.pool + (static_cast<int64_t>(blk) * a.bs + slot0) * row_elems + kvh * dn;
     const uint16_t* krow = kslot + col * row_elems + grp * 8;
 #pragma unroll
@@ -189,8 +228,8 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(DecodeArgs a) {
     float sv[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int64_t t = G.tok0 + grp * 4 + i;
-      const bool ok = t >= a.t0 && t < t_end;
+      const int t = grp * 4 + i;
+      const bool ok = t >= G.lo && t < G.hi;
       sv[i] = ok ? s4[i] * a.scale_log2 : -INFINITY;
       tmax = fmaxf(tmax, sv[i]);
     }
@@ -220,8 +259,7 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(DecodeArgs a) {
 #pragma unroll
     for (int j = 0; j < TPL; ++j) {
       const int key = pv_tg * TPL + j;
-      const int64_t t = G.tok0 + key;
-      const bool ok = t >= a.t0 && t < t_end;
+      const bool ok = key >= G.lo && key < G.hi;
       const u32x4 vv = ok ? G.v[j] : u32x4{0, 0, 0, 0};
       float vf[8];
 #pragma unroll
@@ -254,8 +292,8 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(DecodeArgs a) {
     if (g + 1 < g1) compute_group(gb);
   }
 
-  // ---- epilogue: reduce over key subgroups, normalise, write split partial ----
-  const int64_t ws_row_base = static_cast<int64_t>(split) * a.batch * a.hq + static_cast<int64_t>(b) * a.hq;
+  // ---- epilogue: reduce over key subgroups, normalise, write the part ----
+  const int64_t ws_row_base = static_cast<int64_t>(part) * a.batch * a.hq + static_cast<int64_t>(b) * a.hq;
   float l = l_run;
   l += __shfl_xor(l, 16);
   l += __shfl_xor(l, 32);  // lanes with the same col now hold the total over keys
@@ -268,6 +306,44 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(DecodeArgs a) {
       for (int off = DCH; off < 64; off *= 2) v += __shfl_xor(v, off);
       acc[c][e] = v;
     }
+  if (a.subs > 1) {
+    // The runs of a part meet in LDS; wave `sub` of a kv head finishes its query heads
+    // sub, sub + subs, ...
+    if (pv_tg == 0) {
+#pragma unroll
+      for (int c = 0; c < R; ++c)
+#pragma unroll
+        for (int e = 0; e < 8; e += 4)
+          *reinterpret_cast<float4*>(&o_lds[wave][c][pv_dc * 8 + e]) =
+              make_float4(acc[c][e], acc[c][e + 1], acc[c][e + 2], acc[c][e + 3]);
+    }
+    if (lane < R) {
+      m_lds[wave][lane] = m_run;
+      l_lds[wave][lane] = l;
+    }
+    __syncthreads();
+    if (idle) return;
+    const int w0 = wave - sub * a.heads;
+    for (int c = sub; c < a.rep; c += a.subs) {
+      float m = kNoMax;
+      for (int i = 0; i < a.subs; ++i) m = fmaxf(m, m_lds[w0 + i * a.heads][c]);
+      float o[D / 64] = {}, den = 0.f;
+      for (int i = 0; i < a.subs; ++i) {
+        const int w = w0 + i * a.heads;
+        const float f = exp2f(m_lds[w][c] - m);
+        den += f * l_lds[w][c];
+#pragma unroll
+        for (int k = 0; k < D / 64; ++k) o[k] += f * o_lds[w][c][lane + 64 * k];
+      }
+      const float inv = den > 0.f ? 1.f / den : 0.f;
+      const int64_t row = ws_row_base + kvh * a.rep + c;
+#pragma unroll
+      for (int k = 0; k < D / 64; ++k)
+        if (!PAD || lane + 64 * k < dn) a.ws_o[row * dn + lane + 64 * k] = o[k] * inv;
+      if (lane == 0) a.ws_lse[row] = den > 0.f ? (m + __log2f(den)) * kLn2 : -INFINITY;
+    }
+    return;
+  }
   float lc[R];
 #pragma unroll
   for (int c = 0; c < R; ++c) lc[c] = __shfl(l, c);
@@ -290,17 +366,11 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(DecodeArgs a) {
 }
 
 struct DecodePlan {
-  int splits;
-  int groups_per_split;
-  int n_groups;
-  int64_t g_begin;
+  int parts, heads, subs;
 };
 
 // Query heads per kv head the PV accumulators hold: the smallest of 4, 8, 16 >= rep.
 int decode_width(int rep) { return rep <= 4 ? 4 : rep <= 8 ? 8 : 16; }
-// Waves (kv heads) per workgroup.
-int decode_waves(int hkv) { return std::min(hkv, kDecWaves); }
-
 template <int D, int DT, bool PAD = false>
 const void* decode_fn(int r) {
   switch (r) {
@@ -308,6 +378,15 @@ const void* decode_fn(int r) {
     case 8: return reinterpret_cast<const void*>(&paged_decode_kernel<D, DT, 8, PAD>);
     default: return reinterpret_cast<const void*>(&paged_decode_kernel<D, DT, 16, PAD>);
   }
+}
+
+constexpr int kMaxParts = 64;  // partials of one LSE merge
+
+size_t align_up256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
+// Workspace of `parts` partials of every (sequence, head): o, then lse.
+size_t parts_bytes(int parts, int batch, int hq, int d) {
+  const size_t rows = static_cast<size_t>(parts) * batch * hq;
+  return align_up256(rows * d * sizeof(float)) + align_up256(rows * sizeof(float));
 }
 
 // Workgroups of the decode kernel resident at once on the current device (CUs x
@@ -343,31 +422,46 @@ int decode_slots(int d, int dtype, int r, int waves) {
   return slots;
 }
 
-DecodePlan plan_decode(int batch, int hq, int hkv, int d, int dtype, int64_t t0, int64_t t1) {
-  DecodePlan p;
-  p.g_begin = t0 / 16;
-  const int64_t g_end = t1 > t0 ? (t1 + 15) / 16 : p.g_begin;
-  p.n_groups = static_cast<int>(g_end - p.g_begin);
-  // grid = splits x batch x kv-head groups.  One round of resident workgroups: a
-  // partial second round leaves most CUs idle for its whole length (a measured 13-25%
-  // loss at c4), and fewer splits also mean fewer partials to merge.  At least 4 groups
-  // (64 keys) per split.
-  const int waves = decode_waves(hkv);
-  const int rows = std::max(batch, 1) * ((hkv + waves - 1) / waves);
-  int splits = std::max(1, decode_slots(d, dtype, decode_width(hq / hkv), waves) / rows);
-  splits = std::min(splits, 64);
-  int gps = static_cast<int>(ceil_div(std::max(p.n_groups, 1), splits));
-  gps = std::max(gps, 4);
-  p.groups_per_split = gps;
-  p.splits = static_cast<int>(ceil_div(std::max(p.n_groups, 1), gps));
+// Runs per sequence and kv head: as many as fill the chip once -- a partial second round of
+// workgroups leaves most CUs idle for its whole length (a measured 13-25% loss at c4) --
+// and at most one per 16-token group.  A workgroup holds whole token rows (all kv heads,
+// up to 8) while that leaves at most 16 parts to merge, else half the heads and twice the
+// runs, and so on.  Decode steps of 64 / 16 / 4 / 1 sequences of 16384 tokens over three
+// shards: 634 / 169 / 56 / 26 us with 32/8 heads of 128, 195 / 57 / 28 / 26 us with 16/2
+// (one launch and merge per shard, at most 64 runs, at least 4 groups each: 660 / 205 /
+// 126 / 116 and 231 / 140 / 114 / 111 us).  The parts' bytes are kept within the static
+// scratch of the entry point that uses it.
+DecodePlan plan_decode(int batch, int hq, int hkv, int d, int dtype, int n, const DecodeSpan* spans) {
+  int64_t groups = 0;
+  for (int i = 0; i < n; ++i)
+    if (spans[i].t1 > spans[i].t0) groups += (spans[i].t1 + 15) / 16 - spans[i].t0 / 16;
+  require(groups <= INT32_MAX / 16, "paged_decode: too many tokens");
+  groups = std::max<int64_t>(groups, 1);
+  const int z = static_cast<int>(ceil_div(hkv, kDecWaves));
+  DecodePlan p{};
+  const int r = decode_width(hq / hkv);
+  for (int heads = static_cast<int>(ceil_div(hkv, z));; heads = (heads + 1) / 2) {
+    const int64_t rows = static_cast<int64_t>(batch) * ceil_div(hkv, heads);
+    p.heads = heads;
+    p.subs = kDecWaves / heads;
+    int64_t slots = decode_slots(d, dtype, r, heads * p.subs);
+    // half-size workgroups where more waves are resident that way (three a SIMD, say)
+    // and the tokens are enough to use them: 64 x 16384 tokens of 14/2 heads of 64 dims
+    // 106 us, 122 with whole ones
+    const int64_t half = heads * 2 <= kDecWaves ? decode_slots(d, dtype, r, heads * (p.subs / 2)) : 0;
+    if (half > 2 * slots && groups * rows >= half * (p.subs / 2)) {
+      p.subs /= 2;
+      slots = half;
+    }
+    p.parts = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({slots / rows, ceil_div(groups, p.subs), kMaxParts})));
+    if (p.parts <= 16 || heads == 1) break;
+  }
+  while (p.parts > 1 && parts_bytes(p.parts, batch, hq, d) > HCP_DECODE_STATIC_SCRATCH_BYTES) --p.parts;
   return p;
 }
 
-size_t decode_workspace_bytes(int dtype, int batch, int hq, int hkv, int d, int64_t t0, int64_t t1) {
-  const DecodePlan p = plan_decode(batch, hq, hkv, d, dtype, t0, t1);
-  const size_t rows = static_cast<size_t>(p.splits) * batch * hq;
-  auto al = [](size_t x) { return (x + 255) & ~static_cast<size_t>(255); };
-  return al(rows * d * sizeof(float)) + al(rows * sizeof(float));
+size_t decode_workspace_bytes(int dtype, int batch, int hq, int hkv, int d, int n, const DecodeSpan* spans) {
+  return parts_bytes(plan_decode(batch, hq, hkv, d, dtype, n, spans).parts, batch, hq, d);
 }
 
 template <int D, int DT, bool PAD = false>
@@ -380,20 +474,19 @@ static void launch_decode_kernel(int r, dim3 grid, int waves, const DecodeArgs& 
 }
 
 void launch_paged_decode(int dtype, int batch, int hq, int hkv, int d, const void* q, int64_t q_bs,
-                         int64_t q_hs, const void* pool, int64_t num_blocks, int bs,
-                         const int32_t* tables, int64_t table_stride, int64_t table_len,
-                         const int32_t* seq_lens, int64_t t0, int64_t t1, float scale, float* o,
-                         float* lse, void* ws, size_t ws_bytes, int* err, hipStream_t stream) {
+                         int64_t q_hs, const void* pool, int64_t num_blocks, int bs, int n,
+                         const DecodeSpan* spans, float scale, int out_dtype, void* out, int64_t out_rs, float* lse,
+                         void* ws, size_t ws_bytes, int* err, hipStream_t stream) {
   require(hq % hkv == 0 && hq / hkv <= 16, "paged_decode: num_q_heads/num_kv_heads must be <= 16");
   require(bs % 16 == 0, "paged_decode: block_size must be a multiple of 16");
   require(d > 0 && d <= 128 && d % 8 == 0, "paged_decode: head_dim must be a multiple of 8 up to 128");
   require(dtype == kBF16 || dtype == kF16, "paged_decode: dtype must be BF16 or F16");
-  const DecodePlan p = plan_decode(batch, hq, hkv, d, dtype, t0, t1);
-  require(ws_bytes >= decode_workspace_bytes(dtype, batch, hq, hkv, d, t0, t1), "paged_decode: workspace too small");
-  auto al = [](size_t x) { return (x + 255) & ~static_cast<size_t>(255); };
-  const size_t rows = static_cast<size_t>(p.splits) * batch * hq;
+  require(n >= 1 && n <= kMaxDomains, "paged_decode: 1 to 64 shards");
+  const DecodePlan p = plan_decode(batch, hq, hkv, d, dtype, n, spans);
+  require(ws_bytes >= parts_bytes(p.parts, batch, hq, d), "paged_decode: workspace too small");
+  const size_t rows = static_cast<size_t>(p.parts) * batch * hq;
   float* ws_o = static_cast<float*>(ws);
-  float* ws_lse = reinterpret_cast<float*>(static_cast<char*>(ws) + al(rows * d * sizeof(float)));
+  float* ws_lse = reinterpret_cast<float*>(static_cast<char*>(ws) + align_up256(rows * d * sizeof(float)));
 
   DecodeArgs a;
   a.q = static_cast<const uint16_t*>(q);
@@ -406,25 +499,22 @@ void launch_paged_decode(int dtype, int batch, int hq, int hkv, int d, const voi
   a.hkv = hkv;
   a.hq = hq;
   a.rep = hq / hkv;
-  a.tables = tables;
-  a.table_stride = table_stride;
-  a.table_len = table_len;
-  a.seq_lens = seq_lens;
-  a.t0 = t0;
-  a.t1 = t1;
-  a.g_begin = p.g_begin;
-  a.groups_per_split = p.groups_per_split;
-  a.n_groups = p.n_groups;
+  a.n_spans = n;
+  for (int i = 0; i < n; ++i) a.span[i] = spans[i];
+  a.heads = p.heads;
+  a.subs = p.subs;
+  a.gpb = bs / 16;
+  a.gpb_shift = (a.gpb & (a.gpb - 1)) == 0 ? __builtin_ctz(a.gpb) : -1;
   a.scale_log2 = scale * kLog2e;
   a.ws_o = ws_o;
   a.ws_lse = ws_lse;
   a.batch = batch;
   a.err = err;
   a.dn = d;
-  const int waves = decode_waves(hkv);
+  const int waves = p.heads * p.subs;
   const int r = decode_width(a.rep);
-  const dim3 grid(static_cast<unsigned>(p.splits), static_cast<unsigned>(batch),
-                  static_cast<unsigned>((hkv + waves - 1) / waves));
+  const dim3 grid(static_cast<unsigned>(p.parts), static_cast<unsigned>(batch),
+                  static_cast<unsigned>(ceil_div(hkv, p.heads)));
   // head dim 64: its own kernel; other multiples of 8 up to 128: the D=128 kernel with
   // the columns past d zero-padded
   if (dtype == kBF16) {
@@ -437,14 +527,14 @@ void launch_paged_decode(int dtype, int batch, int hq, int hkv, int d, const voi
     else launch_decode_kernel<128, kF16, true>(r, grid, waves, a, stream);
   }
   HCP_HIP(hipGetLastError());
-  // Merge the splits of every (sequence, head): rows = batch*hq, one token each.
-  const float* o_parts[64];
-  const float* l_parts[64];
-  for (int s = 0; s < p.splits; ++s) {
-    o_parts[s] = ws_o + static_cast<size_t>(s) * batch * hq * d;
-    l_parts[s] = ws_lse + static_cast<size_t>(s) * batch * hq;
+  // Merge the parts of every (sequence, head): rows = batch*hq, one token each.
+  const float* o_parts[kMaxParts];
+  const float* l_parts[kMaxParts];
+  for (int i = 0; i < p.parts; ++i) {
+    o_parts[i] = ws_o + static_cast<size_t>(i) * batch * hq * d;
+    l_parts[i] = ws_lse + static_cast<size_t>(i) * batch * hq;
   }
-  launch_lse_merge(p.splits, o_parts, l_parts, batch * hq, 1, d, kF32, o, d, d, lse, 1, stream);
+  launch_lse_merge(p.parts, o_parts, l_parts, batch * hq, 1, d, out_dtype, out, out_rs, out_rs, lse, 1, stream);
 }
 
 }  // namespace hcp

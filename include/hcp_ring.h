@@ -339,8 +339,8 @@ int hcp_paged_decode_partial_static(const hcp_paged_decode_desc* desc, const hcp
  * seed+1, seed+2, ... (mod N), each domain merging its shard into the accumulator
  * (decode_merge_packet, ring.rs:647-663).  After N-1 hops the accumulator is the
  * layer's attention output; the seed only fixes the merge order.
- * This entry replays the whole journey on one GPU: one hcp_paged_decode_partial-style
- * pass per shard, then the closed-form merge in journey order into out (q dtype,
+ * This entry replays the whole journey on one GPU: one paged decode launch over all
+ * shards in journey order, then the closed-form merge of its parts into out (q dtype,
  * [batch, Hq, D] as a view with head_stride / seq_stride = batch stride) and lse_out
  * ([batch, Hq] fp32, may be NULL).  An empty shard passes the packet through
  * unchanged (lse + log 1).  desc->t0/t1 are ignored: shard s covers tokens

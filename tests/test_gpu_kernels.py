@@ -1526,3 +1526,64 @@ def test_qkv_rope_token_count_edges(gpu, case):
         # one rounding to the storage type (2^-8 bf16, 2^-11 fp16 of the value), fp32 sums below that
         bound = y.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) + 1e-5 * y.abs().max()
         assert bool(((got.cpu().double() - y).abs() <= bound).all()), i
+
+
+# Runs that cross shard boundaries, end inside a group, leave waves without a group or a kv
+# head, and meet in LDS (2 to 8 runs per workgroup) or as many parts: one long sequence, few
+# short ones, many shards, kv head counts off the wave counts, blocks of 1, 2 and 3 groups,
+# a first token inside a group.
+DECODE_RUN_CASES = [
+    # Hq, Hkv, D, block_size, tokens of every sequence per shard, first token of the one-shard call
+    (32, 8, 128, 16, [[5003]], 21),
+    (8, 2, 128, 48, [[1], [0]], 0),
+    (14, 2, 64, 32, [[700, 33, 0, 95]], 5),
+    (12, 3, 64, 16, [[17, 16, 15], [300, 1, 64]], 3),
+    (24, 12, 96, 16, [[130, 40], [16, 128]], 0),
+    (16, 1, 128, 48, [[400, 31]], 47),
+    (16, 2, 128, 16, [[i % 5 * 7 for i in range(40)]], 0),
+    (32, 8, 128, 16, [[90 + 11 * i, 13 * i] for i in range(24)], 0),
+]
+
+
+@pytest.mark.parametrize("case", DECODE_RUN_CASES, ids=[f"{c[0]}q{c[1]}kv_d{c[2]}_bs{c[3]}" for c in DECODE_RUN_CASES])
+def test_decode_runs_over_shards(gpu, case):
+    hq, hkv, d, bs, lens, t0 = case
+    b, n = len(lens), len(lens[0])
+    width = [max(1, -(-max(row[s] for row in lens) // bs)) for s in range(n)]
+    nb = b * sum(width) + 2
+    (q, pool), (q32, pool32) = draw(900 + hq + b, [(b, hq, d), (2, nb, bs, hkv, d)], torch.bfloat16)
+    perm, cur = I.permuted_block_table(91, nb), 0
+    shards, rows = [], [[] for _ in range(b)]
+    for s in range(n):
+        tab = np.full((b, width[s]), -1, dtype=np.int32)  # padding past a sequence's own tokens is never read
+        for i in range(b):
+            used = -(-lens[i][s] // bs)
+            tab[i, :used] = perm[cur: cur + used]
+            cur += used
+            rows[i] += [tab[i, t // bs] * bs + t % bs for t in range(lens[i][s])]
+        shards.append((torch.from_numpy(tab).cuda(), torch.tensor([r[s] for r in lens], dtype=torch.int32).cuda(),
+                       max(r[s] for r in lens)))
+    flat = pool32.reshape(2, nb * bs, hkv, d)
+    scale = 1 / math.sqrt(d)
+
+    def check(o, lse, i, tokens):
+        if not tokens:
+            assert np.all(o == 0) and np.all(np.isneginf(lse))
+            return
+        ref_o, ref_l = C.attention_f64(q32[i:i + 1], flat[0, tokens], flat[1, tokens], np.zeros(1),
+                                       np.zeros(len(tokens)), scale, causal=False)
+        assert np.abs(o - ref_o[0]).max() <= OUT_TOL, i
+        assert np.abs(lse - ref_l[0]).max() <= LSE_TOL, i
+
+    for seed in range(min(n, 3)):
+        out, lse = H.decode_ring_replay(q, pool, shards, seed)
+        torch.cuda.synchronize()
+        for i in range(b):
+            check(out[i].float().cpu().numpy(), lse[i].cpu().numpy(), i, rows[i])
+    tables, seq_lens, max_len = shards[0]
+    if max_len > t0:
+        o, lse = H.decode_local_compact_partial(q, pool, tables, t0, max_len, seq_lens=seq_lens)
+        torch.cuda.synchronize()
+        for i in range(b):
+            check(o[i].cpu().numpy(), lse[i].cpu().numpy(), i, rows[i][t0: lens[i][0]])
+    assert H.fetch_device_errors() == 0
