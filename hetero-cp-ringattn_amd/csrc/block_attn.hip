@@ -1177,6 +1177,10 @@ __global__ __launch_bounds__(kGenRows) void general_block_kernel(GenArgs a) {
 // k-steps 4t .. 4t+3 of a lane half are adjacent.  Element i of a 32x32
 // accumulator holds row 8 (i / 4) + 4 half + (i mod 4), column lane mod 32 -- the
 // layout of the head-dim-128 kernel's O^T, whose epilogue indexing this one shares.
+// The fp32 matrix rate bounds it (64 MFMAs of 64 cycles per 32 keys and wave at 64 dims),
+// so a short sequence, whose few workgroups leave SIMDs idle, runs a split form (KW = 2 or
+// 4): 128 / KW rows a workgroup, 32 KW keys a step, a wave folding 32 of them for its
+// 32-row block; the parts meet in LDS at the end (f32_key_parts: when, and by how much).
 // Masking, the online softmax (base 2, scale folded into the exponent), the running-
 // state merge (accumulate) and the final-row mode are those of general_block_kernel.
 // ----------------------------------------------------------------------------------
@@ -1185,17 +1189,20 @@ constexpr int kF32Threads = 64 * kF32Waves;
 constexpr int kF32Rows = 32 * kF32Waves;
 constexpr int kF32BK = 32;
 
-template <int DP>
+template <int DP, int KW>
 __global__ __launch_bounds__(kF32Threads) void mfma_f32_block_kernel(GenArgs a) {
   static_assert(DP % 32 == 0 && DP <= 128, "padded head dim");
+  static_assert(kF32Waves % KW == 0, "key parts");
+  constexpr int RB = kF32Waves / KW;   // 32-row blocks per workgroup
+  constexpr int BK = kF32BK * KW;      // keys staged per step, kF32BK for each part
   constexpr int DB = DP / 32;
   constexpr int KS = DP / 2;
   constexpr int KLS = DP + 4;          // K row stride (floats), 16-byte aligned
   constexpr int VLS = kF32BK + 4;      // V^T row stride (floats), 16-byte aligned
-  constexpr int NV4 = kF32BK * DP / 4 / kF32Threads;  // float4 of K (and of V) per thread per tile
-  static_assert(NV4 >= 1 && kF32BK * DP % (4 * kF32Threads) == 0, "tile split");
-  __shared__ __attribute__((aligned(16))) float ks[kF32BK * KLS];
-  __shared__ __attribute__((aligned(16))) float vt[DP * VLS];
+  constexpr int NV4 = BK * DP / 4 / kF32Threads;  // float4 of K (and of V) per thread per step
+  static_assert(NV4 >= 1 && BK * DP % (4 * kF32Threads) == 0, "tile split");
+  __shared__ __attribute__((aligned(16))) float ks[BK * KLS];
+  __shared__ __attribute__((aligned(16))) float vt[KW * DP * VLS];
   __shared__ int red[kF32Waves];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1203,7 +1210,7 @@ __global__ __launch_bounds__(kF32Threads) void mfma_f32_block_kernel(GenArgs a) 
   const int lcol = lane & 31, half = lane >> 5;
   // work item: heads innermost, query tiles from the last (the most keys under causal
   // masking) to the first, so every head's heaviest tiles start first
-  const int n_qt = (a.lq + kF32Rows - 1) / kF32Rows;
+  const int n_qt = (a.lq + 32 * RB - 1) / (32 * RB);
   const int head = blockIdx.x % a.hq;
   const int qt = n_qt - 1 - static_cast<int>(blockIdx.x / a.hq);
   const int kvh = head / a.rep;
@@ -1215,9 +1222,10 @@ __global__ __launch_bounds__(kF32Threads) void mfma_f32_block_kernel(GenArgs a) 
   }
   const float* kf = static_cast<const float*>(a.k) + kvh * a.k_hs;
   const float* vf = static_cast<const float*>(a.v) + kvh * a.v_hs;
-  const int tq0 = qt * kF32Rows;
-  const int row = tq0 + 32 * wave + lcol;
+  const int tq0 = qt * 32 * RB;
+  const int row = tq0 + 32 * (wave % RB) + lcol;
   const bool live = row < a.lq;
+  const int part = wave / RB;              // this wave's 32 keys of every step
 
   // Q^T fragments: k-step s, this lane's row, dim 8 (s / 4) + 4 half + (s mod 4) (zero
   // past the head dim)
@@ -1247,7 +1255,7 @@ __global__ __launch_bounds__(kF32Threads) void mfma_f32_block_kernel(GenArgs a) 
       n_kv = hi;
     } else {
       row_lim = a.q_off + row + 1 - a.k_off;
-      const int last = min(a.lq, tq0 + kF32Rows) - 1;
+      const int last = min(a.lq, tq0 + 32 * RB) - 1;
       const int64_t lim = a.q_off + last + 1 - a.k_off;
       n_kv = static_cast<int>(lim <= 0 ? 0 : (lim < a.lk ? lim : a.lk));
     }
@@ -1281,10 +1289,11 @@ __global__ __launch_bounds__(kF32Threads) void mfma_f32_block_kernel(GenArgs a) 
       const int e = tid + j * kF32Threads;
       const int r = e / (DP / 4), c4 = 4 * (e % (DP / 4));
       *reinterpret_cast<float4*>(&ks[r * KLS + c4]) = kr[j];
-      vt[(c4 + 0) * VLS + r] = vr[j].x;
-      vt[(c4 + 1) * VLS + r] = vr[j].y;
-      vt[(c4 + 2) * VLS + r] = vr[j].z;
-      vt[(c4 + 3) * VLS + r] = vr[j].w;
+      float* const vp = vt + (r / kF32BK * DP + c4) * VLS + r % kF32BK;
+      vp[0] = vr[j].x;
+      vp[VLS] = vr[j].y;
+      vp[2 * VLS] = vr[j].z;
+      vp[3 * VLS] = vr[j].w;
     }
   };
 
@@ -1297,17 +1306,18 @@ __global__ __launch_bounds__(kF32Threads) void mfma_f32_block_kernel(GenArgs a) 
   float m_run = -INFINITY, l_run = 0.f;
 
   if (n_kv > 0) load_tile(0);
-  for (int kv0 = 0; kv0 < n_kv; kv0 += kF32BK) {
-    __syncthreads();  // the previous tile's reads are done
+  for (int step = 0; step < n_kv; step += BK) {
+    __syncthreads();  // the previous step's reads are done
     store_tile();
     __syncthreads();
-    if (kv0 + kF32BK < n_kv) load_tile(kv0 + kF32BK);  // in flight while this tile is folded
+    if (step + BK < n_kv) load_tile(step + BK);  // in flight while this step is folded
+    const int kv0 = step + part * kF32BK;
     if (kv0 >= wave_hi) continue;  // no key of this tile is visible to the wave's rows
     // S^T in two accumulators (even / odd groups of four k-steps), summed after
     f32x16 sa, sb;
 #pragma unroll
     for (int r = 0; r < 16; ++r) sa[r] = sb[r] = 0.f;
-    const float* kl = &ks[lcol * KLS + 4 * half];
+    const float* kl = &ks[(part * kF32BK + lcol) * KLS + 4 * half];
 #pragma unroll
     for (int u = 0; u < KS / 4; ++u) {
       const float4 k4 = *reinterpret_cast<const float4*>(kl + 8 * u);
@@ -1363,7 +1373,7 @@ __global__ __launch_bounds__(kF32Threads) void mfma_f32_block_kernel(GenArgs a) 
       float4 v4[DB];
 #pragma unroll
       for (int b = 0; b < DB; ++b)
-        v4[b] = *reinterpret_cast<const float4*>(&vt[(32 * b + lcol) * VLS + 8 * t + 4 * half]);
+        v4[b] = *reinterpret_cast<const float4*>(&vt[(part * DP + 32 * b + lcol) * VLS + 8 * t + 4 * half]);
 #pragma unroll
       for (int b = 0; b < DB; ++b) oacc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(v4[b].x, p[4 * t + 0], oacc[b], 0, 0, 0);
 #pragma unroll
@@ -1381,6 +1391,43 @@ __global__ __launch_bounds__(kF32Threads) void mfma_f32_block_kernel(GenArgs a) 
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
     }
     __builtin_amdgcn_sched_group_barrier(0x008, 4 * DB, 1);
+  }
+  if constexpr (KW > 1) {
+    // The key parts of a row block meet in LDS, over the K / V^T tiles: parts 1 .. KW - 1
+    // leave (O, m, l), part 0 folds them in and writes the rows.
+    static_assert((KW - 1) * RB * DB * 1024 <= KW * DP * VLS && 2 * (KW - 1) * RB * 64 <= BK * KLS, "parts fit");
+    f32x4* const os = reinterpret_cast<f32x4*>(vt);
+    __syncthreads();  // every wave is past its last read of the tiles
+    if (part > 0) {
+      const int at = wave - RB;
+      ks[2 * at * 64 + lane] = m_run;
+      ks[(2 * at + 1) * 64 + lane] = l_run;
+#pragma unroll
+      for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          os[((at * DB + b) * 4 + j) * 64 + lane] =
+              f32x4{oacc[b][4 * j], oacc[b][4 * j + 1], oacc[b][4 * j + 2], oacc[b][4 * j + 3]};
+    }
+    __syncthreads();
+    if (part > 0) return;
+#pragma unroll 1
+    for (int at = wave; at < (KW - 1) * RB; at += RB) {
+      const float m2 = ks[2 * at * 64 + lane], l2 = ks[(2 * at + 1) * 64 + lane];
+      const float m_new = fmaxf(m_run, m2);
+      const bool none = m_new == -INFINITY;  // no key visible to the row in either
+      const float a1 = none ? 1.f : exp2f(m_run - m_new), a2 = none ? 1.f : exp2f(m2 - m_new);
+      l_run = l_run * a1 + l2 * a2;
+      m_run = m_new;
+#pragma unroll
+      for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const f32x4 o2 = os[((at * DB + b) * 4 + j) * 64 + lane];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) oacc[b][4 * j + e] = oacc[b][4 * j + e] * a1 + o2[e] * a2;
+        }
+    }
   }
   const float l_tot = l_run + __shfl_xor(l_run, 32);
   if (!live) return;
@@ -1472,14 +1519,24 @@ int device_cus() {
 
 static bool half_width_d(int d);
 
+// Modelled time of a launch: its longest workgroup and its whole work spread over the CUs,
+// joined as a 4-norm (the workgroups of a causal launch neither all run at once nor queue
+// evenly).
+static double launch_time(double chain, double spread) {
+  return std::pow(std::pow(chain, 4) + std::pow(spread, 4), 0.25);
+}
+// 1, 2 or 4 parts for the modelled times of each; a split has to be 6% ahead.
+static int fewest_parts(const double (&t)[3]) {
+  if (std::min(t[1], t[2]) * 1.06 >= t[0]) return 1;
+  return t[1] <= t[2] ? 2 : 4;
+}
+
 // Key parts (KW) of a launch.  A workgroup of 256 / KW rows splits every tile's keys over
 // KW waves: KW times the workgroups, each with a shorter chain of tiles, for launches that
 // leave CUs idle; but every workgroup still brings whole K / V tiles to LDS, so on a full
-// chip it costs more.  Modelled time: the longest workgroup (its tiles alone on a CU) and
-// the whole work over the CUs (tiles with every CU busy: lower clock, shared L2), joined as
-// a 4-norm since the workgroups of a causal launch neither all run at once nor queue
-// evenly; a split form has to be 6% ahead.  Per KW = 1, 2, 4, in us: `own` per workgroup
-// (first loads, rows written), `alone` and `full` per 128-key tile, fitted on MI355X to 74
+// chip it costs more.  The modelled times take, per KW = 1, 2, 4, in us: `own` per
+// workgroup (first loads, rows written), `alone` and `full` per 128-key tile on an idle and
+// on a full chip (lower clock, shared L2), fitted on MI355X to 74
 // launches: blocks of 16-4096 queries against 256-16384 keys, causal rings of 512-8192
 // tokens and ZigZag ones, with 32/8, 16/2, 16/16 heads of 128 and 14/2 of 64 dims.  There
 // it costs at most 3% against KW = 1 and saves up to 59% (512 x 16384, 32/8 heads: 271 us
@@ -1493,21 +1550,14 @@ static int key_parts(double pairs, double rows, int blocks, double n_max, int hq
   static const double full[2][3] = {{3.26, 1.77, 1.07}, {2.22, 1.20, 0.55}};
   const int w = half_width_d(d) ? 1 : 0;
   const double cus = device_cus();
-  int best = 1;
-  double best_t = 0.0;
+  double t[3];
   for (int i = 0; i < 3; ++i) {
     const Geometry geo = geometry(hq, hkv, 1 << i);
     const double items = geo.n_groups * (rows / geo.tq + 0.5 * blocks);
     const double tiles = geo.n_groups * (pairs / kBK3 + 0.5 * rows) / geo.tq;
-    const double chain = own[i] + n_max * alone[w][i];
-    const double spread = (items * own[i] + tiles * full[w][i]) / cus;
-    const double t = (i == 0 ? 1.0 : 1.06) * std::pow(std::pow(chain, 4) + std::pow(spread, 4), 0.25);
-    if (i == 0 || t < best_t) {
-      best = 1 << i;
-      best_t = t;
-    }
+    t[i] = launch_time(own[i] + n_max * alone[w][i], (items * own[i] + tiles * full[w][i]) / cus);
   }
-  return best;
+  return fewest_parts(t);
 }
 
 // The head-dim-128 kernels form buffer descriptors with 32-bit row arithmetic: a tile of
@@ -1606,18 +1656,21 @@ static double block_work(const BlockLaunch& L) {
   return w;
 }
 
+// 128-key tiles that the last row of a block sees (explicit positions: some row may see
+// every key).
+static double block_tiles(const BlockLaunch& L) {
+  int64_t keys = L.lk;
+  if (L.causal && L.q_lim == nullptr) keys = std::max<int64_t>(0, std::min(L.lk, L.q_off + L.lq - L.k_off));
+  return static_cast<double>(ceil_div(keys, kBK3));
+}
+
 // Decomposition of a launch over the blocks Ls[0 .. n) (same heads and head dim).
 static Geometry block_geometry(const BlockLaunch* const* Ls, int n) {
   double pairs = 0.0, rows = 0.0, n_max = 0.0;
   for (int i = 0; i < n; ++i) {
-    const BlockLaunch& L = *Ls[i];
-    pairs += block_work(L);
-    rows += static_cast<double>(L.lq);
-    // keys that the last row sees (explicit positions: some row may see all of them)
-    int64_t keys = L.lk;
-    if (L.causal && L.q_lim == nullptr)
-      keys = std::max<int64_t>(0, std::min(L.lk, L.q_off + L.lq - L.k_off));
-    n_max = std::max(n_max, static_cast<double>(ceil_div(keys, kBK3)));
+    pairs += block_work(*Ls[i]);
+    rows += static_cast<double>(Ls[i]->lq);
+    n_max = std::max(n_max, block_tiles(*Ls[i]));
   }
   return geometry(Ls[0]->hq, Ls[0]->hkv, key_parts(pairs, rows, n, n_max, Ls[0]->hq, Ls[0]->hkv, Ls[0]->d));
 }
@@ -1684,18 +1737,47 @@ bool block_uses_mfma_f32(const BlockLaunch& L) {
   return true;
 }
 
-static void launch_mfma_f32(const BlockLaunch& L, hipStream_t stream) {
-  const GenArgs a = make_gen_args(L);
-  const int64_t items = ceil_div(L.lq, kF32Rows) * static_cast<int64_t>(L.hq);
-  require(items <= INT32_MAX, "fp32 block: too many work items");
+template <int KW>
+static void launch_mfma_f32_k(const GenArgs& a, int64_t items, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>(items));
   const dim3 block(kF32Threads);
-  switch ((L.d + 31) / 32) {
-    case 1: mfma_f32_block_kernel<32><<<grid, block, 0, stream>>>(a); break;
-    case 2: mfma_f32_block_kernel<64><<<grid, block, 0, stream>>>(a); break;
-    case 3: mfma_f32_block_kernel<96><<<grid, block, 0, stream>>>(a); break;
-    default: mfma_f32_block_kernel<128><<<grid, block, 0, stream>>>(a); break;
+  switch ((a.d + 31) / 32) {
+    case 1: mfma_f32_block_kernel<32, KW><<<grid, block, 0, stream>>>(a); break;
+    case 2: mfma_f32_block_kernel<64, KW><<<grid, block, 0, stream>>>(a); break;
+    case 3: mfma_f32_block_kernel<96, KW><<<grid, block, 0, stream>>>(a); break;
+    default: mfma_f32_block_kernel<128, KW><<<grid, block, 0, stream>>>(a); break;
   }
+}
+
+// Key parts of the fp32 kernel: 128 / KW rows a workgroup, as key_parts.  Per KW = 1, 2, 4
+// and 32, 64, 96, 128 padded dims, in us per 128 keys of a workgroup (96 dims between its
+// neighbours), fitted to causal sequences of 128-8192 tokens and blocks of 32-1024 queries
+// against 1024-4096 keys.  1024 tokens, 8 heads of 64 dims: 107 us with KW = 1, 64 with 2,
+// 43 with 4; 4096 tokens: 404, 285, 312; 32/8 heads of 128 dims, 4096 tokens: 1603, 1931,
+// 2717.
+static int f32_key_parts(const BlockLaunch& L) {
+  static const double alone[4][3] = {{7.4, 4.1, 2.3}, {12.3, 6.95, 4.25}, {18.0, 10.5, 6.9}, {23.5, 14.1, 9.5}};
+  static const double full[4][3] = {{6.0, 3.3, 1.75}, {11.0, 6.4, 4.5}, {17.6, 10.5, 7.4}, {24.3, 14.6, 10.3}};
+  constexpr double own = 5.0;
+  const int w = (L.d + 31) / 32 - 1;
+  const double cus = device_cus(), lq = static_cast<double>(L.lq), pairs = block_work(L), n_max = block_tiles(L);
+  double t[3];
+  for (int i = 0; i < 3; ++i) {
+    const double wgs = L.hq * std::ceil(lq / (kF32Rows >> i));
+    const double tiles = L.hq * (pairs / kBK3 + 0.25 * lq) / (kF32Rows >> i);
+    t[i] = launch_time(own + n_max * alone[w][i], (wgs * own + tiles * full[w][i]) / cus);
+  }
+  return fewest_parts(t);
+}
+
+static void launch_mfma_f32(const BlockLaunch& L, hipStream_t stream) {
+  const GenArgs a = make_gen_args(L);
+  const int kw = f32_key_parts(L);
+  const int64_t items = ceil_div(L.lq, kF32Rows / kw) * static_cast<int64_t>(L.hq);
+  require(items <= INT32_MAX, "fp32 block: too many work items");
+  if (kw == 4) launch_mfma_f32_k<4>(a, items, stream);
+  else if (kw == 2) launch_mfma_f32_k<2>(a, items, stream);
+  else launch_mfma_f32_k<1>(a, items, stream);
 }
 
 void launch_block_partial(const BlockLaunch& L, hipStream_t stream) {

@@ -1587,3 +1587,44 @@ def test_decode_runs_over_shards(gpu, case):
         for i in range(b):
             check(o[i].cpu().numpy(), lse[i].cpu().numpy(), i, rows[i][t0: lens[i][0]])
     assert H.fetch_device_errors() == 0
+
+
+# The fp32 kernel's split forms (2 or 4 waves share a 32-row block and fold 32 of every 64
+# or 128 keys each): one and several steps, parts with no visible key, each padded width, and
+# a shape per number of parts.
+F32_SPLIT_CASES = [
+    # Hq, Hkv, D, Lq list, Lk list
+    (4, 2, 64, (1, 33, 100), (1, 31, 64, 129, 300)),
+    (2, 2, 32, (40,), (33, 95)),
+    (4, 1, 96, (65,), (32, 161)),
+    (3, 1, 128, (31, 96), (97, 256)),
+    (32, 8, 128, (320,), (300,)),
+    (16, 16, 64, (1100,), (200,)),
+]
+
+
+@pytest.mark.parametrize("case", F32_SPLIT_CASES, ids=[f"{c[0]}q{c[1]}kv_d{c[2]}" for c in F32_SPLIT_CASES])
+def test_fp32_split_key_parts_match_closed_form(gpu, case):
+    hq, hkv, d, lqs, lks = case
+    scale = 1 / math.sqrt(d)
+    for lq in lqs:
+        for lk in lks:
+            (q, k, v), (q32, k32, v32) = draw(lq + 5 * lk + d, [(lq, hq, d), (lk, hkv, d), (lk, hkv, d)], torch.float32)
+            qv, kv, vv = (x.permute(1, 0, 2) for x in (q, k, v))
+            for qo in (-lq // 2, lk // 2, lk):
+                ref_o, ref_l = C.attention_f64(q32, k32, v32, np.arange(qo, qo + lq), np.arange(lk), scale)
+                ref_o, ref_l = ref_o.transpose(1, 0, 2), ref_l.T
+                cont = H.block_partial(qv, kv, vv, qo + lq, lq, scale=scale)
+                assert H.last_path() == "mfma_f32"
+                pos = H.block_partial_positioned(qv, torch.arange(qo + lq, 2 * lq + qo, device="cuda"), kv, vv,
+                                                 torch.arange(lq, lq + lk, device="cuda"), scale=scale)
+                o2, l2 = cont[0].clone(), cont[1].clone()
+                H.block_partial(qv, kv, vv, qo + lq, lq, scale=scale, o=o2, lse=l2, accumulate=True)
+                torch.cuda.synchronize()
+                fin = np.isfinite(ref_l)
+                for (o, l), shift in ((cont, 0.0), (pos, 0.0), ((o2, l2), math.log(2.0))):
+                    o, l = o.cpu().numpy(), l.cpu().numpy()
+                    assert np.array_equal(np.isfinite(l), fin) and np.all(o[~fin] == 0), (lq, lk, qo)
+                    assert np.abs(o - ref_o).max() <= 1e-4, (lq, lk, qo)
+                    if fin.any():
+                        assert np.abs(l[fin] - ref_l[fin] - shift).max() <= 1e-4, (lq, lk, qo)
