@@ -1488,6 +1488,10 @@ QKV_EDGE_CASES = [
     (129, 128, 2, 2, 64, torch.bfloat16, False),
     (1300, 160, 8, 2, 128, torch.bfloat16, True),
     (2100, 96, 14, 2, 64, torch.float16, False),
+    # 384 x 256 tiles: full, with a ragged last tile of features, and with head dim 64
+    (4090, 96, 32, 8, 128, torch.bfloat16, True),
+    (3580, 64, 30, 8, 128, torch.bfloat16, False),
+    (4000, 64, 64, 16, 64, torch.float16, False),
 ]
 
 
