@@ -9,13 +9,14 @@
 //
 //   * C^T = W X^T on v_mfma_f32_32x32x16 (A = weight rows, B = token rows, both
 //     hidden-contiguous), so a lane owns one token and 16 features of each 32-feature
-//     block.  A workgroup computes 256 features x 128, 256 or 384 tokens or 384 features
-//     x 256 tokens (chosen per launch) with 8 waves of 64 features x half the tokens or
-//     192 x a quarter: a wave's features come in pairs of 32-feature blocks at d and
+//     block.  A workgroup computes 256 features x 128, 256 or 384 tokens, 384 features
+//     x 256 tokens or 128 x 128 (chosen per launch) with 8 waves of 64 features x half
+//     the tokens, 192 x a quarter or 64 x a quarter: a wave's features come in pairs of 32-feature blocks at d and
 //     d + D/2 of one head, so each RoPE partner pair sits in the same lane and register
 //     slot of the wave's two blocks -- the rotation needs no data exchange.
 //   * Weight and token tiles of 32 hidden values reach LDS through buffer_load ... lds
-//     (four buffers, three stages in flight, one barrier per stage); chunk p of tile row
+//     (four buffers, three stages in flight, eight and seven for 128 x 128 tiles; one
+//     barrier per stage); chunk p of tile row
 //     r holds global chunk p ^ ((r >> 2) & 3), which keeps the fragment reads free of
 //     bank conflicts.  The loop is software-pipelined: a stage's DMA instructions are
 //     spread through the MFMAs of the stage three before it, the second K half's
@@ -44,7 +45,6 @@ constexpr int kQWaves = 8;
 constexpr int kQThreads = kQWaves * 64;
 constexpr int kQK = 32;                      // hidden values per stage
 constexpr int kQRow = kQK * 2;               // bytes per tile row in LDS
-constexpr int kQBufs = 4;
 constexpr int kQGroupM = 4;                  // token tiles per placement group
 
 template <int DT>
@@ -80,27 +80,29 @@ __device__ __forceinline__ float ld16(const uint16_t* p) {
 // TF features x TN tokens per workgroup.  Each wave owns 2 x OB blocks of 32 x 32: with
 // TF = 256 the features fbase and fbase + D/2 of one head (RoPE partners; group wf = w & 3)
 // times the TN/2 tokens of half wt = w >> 2; with TF = 384 three such pairs 128 features
-// apart (group wf = w & 1) times the 64 tokens of quarter wt = w >> 1.  The side with more
+// apart (group wf = w & 1) times the 64 tokens of quarter wt = w >> 1; with TF = 128 one
+// pair (group w & 1) times the 32 tokens of quarter w >> 1.  The side with more
 // blocks is the outer one of the MFMA order, each of its fragments used for two MFMAs.
 template <int DT, int D, int TF, int TN>
 __global__ __launch_bounds__(kQThreads, 1) void qkv_rope_kernel(QkvArgs a) {
   using Ops = QkvMfma<DT>;
   using frag = typename Ops::frag;
-  static_assert(TF == 256 || (TF == 384 && TN == 256), "tile shapes");
+  static_assert(TF == 256 || (TF == 384 && TN == 256) || (TF == 128 && TN == 128), "tile shapes");
   constexpr bool kFeatOuter = TF == 384;
-  constexpr int OB = kFeatOuter ? 6 : TN / 64;  // outer 32-blocks per wave (2 inner ones)
+  constexpr int WF = TF == 256 ? 4 : 2;         // feature groups of waves
+  constexpr int WT = kQWaves / WF;              // token groups
+  constexpr int OB = kFeatOuter ? 6 : TN / WT / 32;  // outer 32-blocks per wave (2 inner ones)
   constexpr int NP = kFeatOuter ? 3 : 1;        // RoPE pairs per wave
   constexpr int NT = kFeatOuter ? 2 : OB;       // 32-token blocks per wave
-  constexpr int WF = kFeatOuter ? 2 : 4;        // feature groups of waves
-  constexpr int WT = kQWaves / WF;              // token groups
   constexpr int WJ = TF / 128;                  // weight-row DMA instructions per wave per stage
   constexpr int XJ = TN / 128;                  // token-row DMA instructions per wave per stage
   constexpr int kOperandW = TF * kQRow;
   constexpr int kOperandX = TN * kQRow;
   constexpr int kStage = kOperandW + kOperandX;
+  constexpr int NB = TF == 128 ? 8 : 4;         // stage buffers, NB - 1 stages in flight
   constexpr int kPerStage = WJ + XJ;            // DMA instructions per wave per stage
   constexpr int kPair = D / 64;                 // pairs per head
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[kQBufs * kStage];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[NB * kStage];
 
   // ---- placement: groups of kQGroupM token tiles x every feature tile ----
   const int logical = xcd_remap(blockIdx.x, gridDim.x);
@@ -198,16 +200,18 @@ __global__ __launch_bounds__(kQThreads, 1) void qkv_rope_kernel(QkvArgs a) {
       for (int r = 0; r < 16; ++r) acc[i][o][r] = 0.f;
 
   const int n_st = a.hidden / kQK;
-  if (n_st > 0) issue(0, 0);
-  if (n_st > 1) issue(1, 1);
-  if (n_st > 2) issue(2, 2);
+#pragma unroll
+  for (int st = 0; st < NB - 1; ++st)
+    if (st < n_st) issue(st, st);
 
   // Stage st resident for every wave: this wave's DMA of it done (at most the stages
   // issued after it still in flight), this wave's reads of older stages done, then the
   // barrier.
   auto sync_stage = [&](int st) __attribute__((always_inline)) {
-    const int after = min(2, max(0, n_st - 1 - st));
-    if (after >= 2) wait_vmcnt<2 * kPerStage>();
+    const int after = min(NB - 2, max(0, n_st - 1 - st));
+    if (after == NB - 2) wait_vmcnt<(NB - 2) * kPerStage>();
+    else if (NB > 4 && after >= 4) wait_vmcnt<4 * kPerStage>();
+    else if (NB > 4 && after >= 2) wait_vmcnt<2 * kPerStage>();
     else if (after == 1) wait_vmcnt<kPerStage>();
     else wait_vmcnt<0>();
     wait_lgkmcnt0();
@@ -218,11 +222,15 @@ __global__ __launch_bounds__(kQThreads, 1) void qkv_rope_kernel(QkvArgs a) {
   };
   // MFMA (flat index over the stage) after which the next stage's barrier sits: after the
   // last DMA instruction and at least two outer blocks into the second K half.
-  constexpr int kMidA = 3 * (kPerStage - 1) + 1 > 2 * OB + 3 ? 3 * (kPerStage - 1) + 1 : 2 * OB + 3;
+  constexpr int kGap = OB == 1 ? 1 : 3;    // one DMA instruction after every third MFMA from the second
+  constexpr int kOff = OB == 1 ? 0 : 1;    // (128 x 128 tiles: after each from the first)
+  constexpr int kLast = kGap * (kPerStage - 1) + kOff;
+  constexpr int kMidB = OB == 1 ? 3 : 2 * OB + 3;
+  constexpr int kMidA = kLast > kMidB ? kLast : kMidB;
   constexpr int kMid = kMidA % 2 ? kMidA : kMidA + 1;
   constexpr int kMidO = (kMid - 2 * OB) / 2;  // last second-half outer block before it
   static_assert(kMid < 4 * OB, "barrier inside the stage");
-  static_assert(3 * (kPerStage - 1) + 1 < 4 * OB, "every DMA instruction issued inside the stage");
+  static_assert(kLast < 4 * OB, "every DMA instruction issued inside the stage");
 
   frag in0[2], out0[OB];  // first-half fragments of the current stage, read ahead
   if (n_st > 0) {
@@ -232,18 +240,17 @@ __global__ __launch_bounds__(kQThreads, 1) void qkv_rope_kernel(QkvArgs a) {
 #pragma unroll
     for (int o = 0; o < OB; ++o) out0[o] = rd(0, out_at(0, o));
   }
-  // compute(st, bufc): the MFMAs of stage st (buffer bufc).  The DMA of stage st + 3 (into
-  // buffer (bufc + 3) & 3, last read in stage st - 1, before this stage's barrier) is
-  // spread through them, one instruction after every third MFMA from the second, so the
-  // waves' address traffic does not queue at the stage start.
+  // compute(st, bufc): the MFMAs of stage st (buffer bufc).  The DMA of stage st + NB - 1
+  // (into buffer bufc - 1, last read in stage st - 1, before this stage's barrier) is
+  // spread through them, so the waves' address traffic does not queue at the stage start.
   auto compute = [&](int st, auto bufc) __attribute__((always_inline)) {
     constexpr int bf = decltype(bufc)::value;
-    constexpr int nb = (bf + 1) & 3;
-    const int pf = st + 3 < n_st ? st + 3 : -1;
+    constexpr int nb = (bf + 1) % NB;
+    const int pf = st + NB - 1 < n_st ? st + NB - 1 : -1;
     auto dma_after = [&](int m) __attribute__((always_inline)) {
-      if (m % 3 == 1 && m / 3 < kPerStage && pf >= 0) {
+      if (m % kGap == kOff % kGap && m / kGap < kPerStage && pf >= 0) {
         __builtin_amdgcn_sched_barrier(0);
-        issue_one(pf, (bf + 3) & 3, m / 3);
+        issue_one(pf, (bf + NB - 1) % NB, m / kGap);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
@@ -279,11 +286,17 @@ __global__ __launch_bounds__(kQThreads, 1) void qkv_rope_kernel(QkvArgs a) {
       if (o > kMidO) out0[o] = rd(nb, out_at(0, o));
     }
   };
-  for (int st = 0; st < n_st; st += kQBufs) {
+  for (int st = 0; st < n_st; st += NB) {
     compute(st, IntC<0>{});
     if (st + 1 < n_st) compute(st + 1, IntC<1>{});
     if (st + 2 < n_st) compute(st + 2, IntC<2>{});
     if (st + 3 < n_st) compute(st + 3, IntC<3>{});
+    if constexpr (NB == 8) {
+      if (st + 4 < n_st) compute(st + 4, IntC<4>{});
+      if (st + 5 < n_st) compute(st + 5, IntC<5>{});
+      if (st + 6 < n_st) compute(st + 6, IntC<6>{});
+      if (st + 7 < n_st) compute(st + 7, IntC<7>{});
+    }
   }
 
   // ---- epilogue ----
@@ -597,24 +610,28 @@ void launch_rope_table(int d, int64_t rows, double base, float* cos, float* sin,
   HCP_HIP(hipGetLastError());
 }
 
-// Tile (features x tokens) of 256 x 128, 256 x 256, 256 x 384 or 384 x 256: the one with
-// the least modelled time, i.e. rounds of workgroups over the device's compute units times
-// the time one tile of that size takes relative to 256 x 256 (0.62 and 1.41: bigger tiles
-// reuse each LDS fragment more), a partly filled last round counted as 0.5 + 0.5 x its fill
-// (it runs at a higher clock with part of the chip idle).  Fitted to a sweep of the
-// Llama-3-8B projection over 1024-24576 tokens on MI355X.  That layer at 12288 tokens:
-// 768 tiles of 256 x 384 are 3 full rounds of 256 CUs; at 4096 tokens 256 of 384 x 256 are
-// one, 177 us (384 of 256 x 256, one round and a half: 232); at 8192 tokens 354 against 376.
+// Tile (features x tokens) of 256 x 128, 256 x 256, 256 x 384, 384 x 256 or 128 x 128: the
+// one with the least modelled time, i.e. rounds of workgroups over the device's compute
+// units times the time one tile of that size takes relative to 256 x 256 (bigger tiles reuse
+// each LDS fragment more), a partly filled last round counted as 0.5 + 0.5 x its fill (it
+// runs at a higher clock with part of the chip idle).  Fitted to a sweep of the Llama-3-8B
+// projection over 1024-24576 tokens on MI355X, the 128 x 128 tile to 150-8192 tokens of it
+// and of Qwen2.5-3B's and Qwen2-0.5B's.  Llama-3-8B at 12288 tokens: 768 tiles of 256 x 384
+// are 3 full rounds of 256 CUs; at 4096 tokens 256 of 384 x 256 are one, 177 us (384 of
+// 256 x 256, one round and a half: 232); at 8192 tokens 354 against 376.  128 x 128 spreads a
+// launch that fills less than a round over twice the CUs of 256 x 128: 256 tokens of
+// Llama-3-8B 36 us against 55, 1024 of Qwen2.5-3B 25 against 37, 2048 of Qwen2-0.5B 17
+// against 25; over more than a round it is the slower one (768 of Llama-3-8B: 74 against 72).
 struct QkvTile {
   int tf, tn;
 };
 static QkvTile qkv_tile(int64_t n_feat, int64_t tokens) {
   const int cus = device_cus();
-  const QkvTile tiles[4] = {{256, 256}, {256, 128}, {256, 384}, {384, 256}};
-  const double cost[4] = {1.0, 0.62, 1.41, 1.41};
+  const QkvTile tiles[5] = {{256, 256}, {256, 128}, {256, 384}, {384, 256}, {128, 128}};
+  const double cost[5] = {1.0, 0.62, 1.41, 1.41, 0.42};
   int best = 0;
   double best_t = 0.0;
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < 5; ++i) {
     const int64_t n = ceil_div(n_feat, tiles[i].tf) * ceil_div(tokens, tiles[i].tn);
     const int64_t full = n / cus;
     const double fill = static_cast<double>(n - full * cus) / cus;
@@ -682,6 +699,7 @@ void launch_qkv_rope(int dtype, int d, QkvArgs& a, hipStream_t stream) {
     }
   };
   if (tile.tf == 384) go(IntC<384>{}, IntC<256>{});
+  else if (tile.tf == 128) go(IntC<128>{}, IntC<128>{});
   else if (tile.tn == 128) go(IntC<256>{}, IntC<128>{});
   else if (tile.tn == 384) go(IntC<256>{}, IntC<384>{});
   else go(IntC<256>{}, IntC<256>{});

@@ -1488,6 +1488,9 @@ QKV_EDGE_CASES = [
     (129, 128, 2, 2, 64, torch.bfloat16, False),
     (1300, 160, 8, 2, 128, torch.bfloat16, True),
     (2100, 96, 14, 2, 64, torch.float16, False),
+    # 128 x 128 tiles above; ragged 256 x 128 and 256 x 256 ones
+    (2100, 64, 16, 2, 128, torch.bfloat16, False),
+    (4100, 64, 16, 2, 128, torch.bfloat16, True),
     # 384 x 256 tiles: full, with a ragged last tile of features, and with head dim 64
     (4090, 96, 32, 8, 128, torch.bfloat16, True),
     (3580, 64, 30, 8, 128, torch.bfloat16, False),
@@ -1505,7 +1508,7 @@ def test_qkv_rope_token_count_edges(gpu, case):
     xp[:tokens, :hidden] = x.cuda()
     xp = xp[:tokens, :hidden]
     wd, bd = [w.cuda() for w in ws], [b.cuda() for b in bs]
-    table = H.rope_table(d, 4096, 10000.0)
+    table = H.rope_table(d, 4200, 10000.0)
     pos = torch.arange(5, 5 + tokens, dtype=torch.int64, device="cuda")
     q = torch.zeros(hq, tokens, d + 4, dtype=dtype, device="cuda")[:, :, 4:]
     if paged:
