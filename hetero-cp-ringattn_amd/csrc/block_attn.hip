@@ -1821,7 +1821,11 @@ void launch_block_partial(const BlockLaunch& L, hipStream_t stream) {
   if (!L.force_general && block_uses_mfma(L.dtype, L.d)) {
     if (L.dtype == kBF16) launch_mfma<kBF16>(L, stream);
     else launch_mfma<kF16>(L, stream);
-  } else if (block_uses_mfma_f32(L)) {
+    HCP_HIP(hipGetLastError());
+    return;
+  }
+  require(L.q_rows == nullptr, "block_partial: a query row map needs the 16-bit matrix-core kernel");
+  if (block_uses_mfma_f32(L)) {
     launch_mfma_f32(L, stream);
   } else {
     switch (L.dtype) {

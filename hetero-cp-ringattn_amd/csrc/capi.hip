@@ -312,7 +312,7 @@ ReplayPlan plan_replay(const hcp_ring_replay_desc* d, bool paged) {
     size_t c = paged ? 2 * p.fused_stage_bytes : 0;
     const size_t n8 = align256(static_cast<size_t>(p.seq) * sizeof(int64_t));
     const size_t n4 = align256(static_cast<size_t>(p.seq) * sizeof(int32_t));
-    c += n8 + 256;  // part of the reported size from when positions and a flag were stored; unused
+    c += n8 + 256;  // room below the arrays, at least 256 bytes, for run_replay_fused_positioned to align them
     p.fp_rows = c;
     c += n4;
     p.fp_kc = c;
@@ -448,13 +448,17 @@ void run_replay_fused_positioned(const hcp_ring_replay_desc* d, const ReplayPlan
   g.k_ss_bytes = k.seq_stride * es;
   g.v_hs_bytes = v.head_stride * es;
   g.v_ss_bytes = v.seq_stride * es;
-  g.kc = base + p.fp_kc;
-  g.vc = base + p.fp_vc;
-  g.lim = reinterpret_cast<int32_t*>(base + p.fp_lim);
+  // The workspace may start at any address, but the matrix-core kernels read the copies in
+  // 16-byte columns: the arrays start at 256-byte boundaries, up to 255 bytes into the room
+  // that the layout leaves below them.
+  char* const fp = base - reinterpret_cast<uintptr_t>(base) % 256;
+  g.kc = fp + p.fp_kc;
+  g.vc = fp + p.fp_vc;
+  g.lim = reinterpret_cast<int32_t*>(fp + p.fp_lim);
   // The 16-bit kernels also take the query rows in position order, so a tile's rows see
   // keys up to a common diagonal and the last tiles are the heaviest; the fp32 one takes
   // them as stored.
-  g.rows = d->dtype == kF32 ? nullptr : reinterpret_cast<int32_t*>(base + p.fp_rows);
+  g.rows = d->dtype == kF32 ? nullptr : reinterpret_cast<int32_t*>(fp + p.fp_rows);
   timed(kTimedGather, stream, [&] { launch_strategy_gather(g, stream); });
   const int64_t hs = p.seq * d->head_dim;
   BlockLaunch L = whole_sequence_launch(d, p, q, hcp_ring_view{g.kc, hs, d->head_dim},

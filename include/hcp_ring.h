@@ -419,7 +419,8 @@ int hcp_decode_ring_replay(const hcp_paged_decode_desc* desc, const hcp_paged_po
  * Workspace: hcp_ring_replay_workspace_size reports the need of the requested schedule
  * (AUTO: the larger of the two).  FUSED needs none unpaged with VANILLA positions; with
  * STRIPED / ZIGZAG it holds the row of each position, K/V in position order
- * (2 * Hkv * S * head_dim elements) and the per-row key limits.
+ * (2 * Hkv * S * head_dim elements), the per-row key limits, and 8 * S + 256 bytes in
+ * which these are aligned.  A workspace may start at any address.
  * ------------------------------------------------------------------------------- */
 enum hcp_ring_schedule {
   HCP_SCHEDULE_AUTO = 0,

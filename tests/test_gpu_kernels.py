@@ -1668,3 +1668,40 @@ def test_strategy_replay_rows_in_position_order(gpu, case, strategy):
     assert np.abs(lse.cpu().numpy() - ref_l.T).max() <= (1e-4 if f32 else LSE_TOL)
     ob[:, 2: 2 + s, :d] = 7.0
     assert bool((ob == 7.0).all())
+
+
+@pytest.mark.parametrize("paged", [False, True], ids=["views", "paged"])
+@pytest.mark.parametrize("strategy", ["striped", "zigzag"])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "f16", "f32"])
+def test_strategy_replay_workspace_at_any_address(gpu, dt, strategy, paged):
+    # A workspace of exactly the reported size anywhere in a byte buffer: the same bits as
+    # with an aligned one, the closed form's values, and nothing written outside it.
+    chunks, hq, hkv, d, bs = [97, 40, 130], 4, 2, 64, 16
+    s = sum(chunks)
+    nb = -(-s // bs)
+    (q, pool), (q32, pool32) = draw(810, [(s, hq, d), (2, nb, bs, hkv, d)], dt)
+    table = torch.from_numpy(I.permuted_block_table(17, nb).astype(np.int32))
+    kv32 = pool32[:, table.numpy()].reshape(2, nb * bs, hkv, d)[:, :s]
+    k, v = pool[:, table.long().cuda()].reshape(2, nb * bs, hkv, d)[:, :s].permute(0, 2, 1, 3).contiguous()
+    pos = np.array(sum(_strategy_rows(chunks, strategy)[0], []))
+    need = H.replay_workspace_size(dt, hq, hkv, d, chunks, paged=paged, strategy=strategy)
+    results = []
+    for offset in (0, 4, 8, 252):
+        buf = torch.full((need + 512,), 0xA5, dtype=torch.uint8, device="cuda")
+        assert buf.data_ptr() % 256 == 0
+        ws = buf[offset: offset + need]
+        if paged:
+            got = H.ring_attention_replay_paged(q.permute(1, 0, 2), pool, table.cuda(), chunks, strategy=strategy,
+                                                workspace=ws)
+        else:
+            got = H.ring_attention_replay(q.permute(1, 0, 2), k, v, chunks, strategy=strategy, workspace=ws)
+        torch.cuda.synchronize()
+        assert bool((buf[:offset] == 0xA5).all()) and bool((buf[offset + need:] == 0xA5).all()), offset
+        results.append(got)
+    assert H.fetch_device_errors() == 0
+    ref_o, ref_l = C.attention_f64(q32, kv32[0], kv32[1], pos, pos, 1 / math.sqrt(d))
+    f32 = dt == torch.float32
+    for o, l in results:
+        assert np.abs(o.float().cpu().numpy() - ref_o.transpose(1, 0, 2)).max() <= (1e-4 if f32 else OUT_TOL)
+        assert np.abs(l.cpu().numpy() - ref_l.T).max() <= (1e-4 if f32 else LSE_TOL)
+        assert torch.equal(o, results[0][0]) and torch.equal(l, results[0][1])
