@@ -1,7 +1,8 @@
 // LSE merge of ring-step partials (closed form of the re-entry merge in
 // positioned_merge_compact_partial / decode_merge_packet, ring.rs:574-603, :647-663):
 //   m = max_i lse_i,  w_i = e^(lse_i - m),
-//   o = sum_i w_i o_i / sum_i w_i,  lse = m + ln sum_i w_i,  all -inf -> (0, -inf).
+//   o = sum_i w_i o_i / sum_i w_i,  lse = m + ln sum_i w_i,  all -inf -> (0, -inf);
+// a NaN LSE makes the row NaN.
 //
 // Layout: each partial is o [H, L, D] fp32 and lse [H, L] fp32 (as the block kernel
 // writes them).  One row (h, t) = D fp32 is handled by D/4 lanes with 16-byte loads,
@@ -37,6 +38,12 @@ __device__ __forceinline__ float4 nt_load4(const float* p) {
   typedef float f4 __attribute__((ext_vector_type(4)));
   const f4 x = __builtin_nontemporal_load(reinterpret_cast<const f4*>(p));
   return make_float4(x[0], x[1], x[2], x[3]);
+}
+
+// LSE of a row from its largest partial LSE and the sum of the weights against it: -inf
+// for a row of empty partials (sum 0), NaN where a partial's is.
+__device__ __forceinline__ float merged_lse(float m, float den) {
+  return den > 0.f ? m + __logf(den) : den == 0.f ? -INFINITY : den;
 }
 
 // Four consecutive values of a merged row in the output type.
@@ -88,13 +95,15 @@ __global__ __launch_bounds__(256) void lse_merge_few_rows_kernel(MergeArgs a) {
     float mn = m;
 #pragma unroll
     for (int u = 0; u < NP; ++u) mn = fmaxf(mn, l[u]);
-    if (mn == -INFINITY) continue;  // every partial so far is empty
-    const float sc = __expf(m - mn);
+    // While every partial of the slot is empty the weights are taken against 0: an empty
+    // one adds nothing, a NaN stays (the row's other slots may hold finite partials).
+    const float ref = mn == -INFINITY ? 0.f : mn;
+    const float sc = __expf(m - ref);
     den *= sc;
     acc.x *= sc; acc.y *= sc; acc.z *= sc; acc.w *= sc;
 #pragma unroll
     for (int u = 0; u < NP; ++u) {
-      const float w = __expf(l[u] - mn);
+      const float w = __expf(l[u] - ref);
       den += w;
       acc.x += w * v[u].x; acc.y += w * v[u].y; acc.z += w * v[u].z; acc.w += w * v[u].w;
     }
@@ -105,23 +114,23 @@ __global__ __launch_bounds__(256) void lse_merge_few_rows_kernel(MergeArgs a) {
   den_l[threadIdx.x] = den;
   __syncthreads();
   if (slot != 0) return;
+  const int used = min(slots, a.n);  // slots past the last partial hold nothing
   float mt = -INFINITY;
-  for (int s = 0; s < slots; ++s) mt = fmaxf(mt, m_l[threadIdx.x + s * lpr]);
+  for (int s = 0; s < used; ++s) mt = fmaxf(mt, m_l[threadIdx.x + s * lpr]);
   float dt = 0.f;
   float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (mt != -INFINITY) {
-    for (int s = 0; s < slots; ++s) {
-      const float w = __expf(m_l[threadIdx.x + s * lpr] - mt);
-      const float4 x = acc_l[threadIdx.x + s * lpr];
-      dt += w * den_l[threadIdx.x + s * lpr];
-      o.x += w * x.x; o.y += w * x.y; o.z += w * x.z; o.w += w * x.w;
-    }
+  for (int s = 0; s < used; ++s) {
+    const float w = mt == -INFINITY ? 1.f : __expf(m_l[threadIdx.x + s * lpr] - mt);
+    dt += w * den_l[threadIdx.x + s * lpr];
+    if (mt == -INFINITY) continue;  // no finite LSE: (0, -inf), or NaN with a NaN one
+    const float4 x = acc_l[threadIdx.x + s * lpr];
+    o.x += w * x.x; o.y += w * x.y; o.z += w * x.z; o.w += w * x.w;
   }
-  const float inv = dt > 0.f ? 1.f / dt : 0.f;
+  const float inv = dt > 0.f ? 1.f / dt : dt;
   const int64_t h = row / a.q_len, t = row - h * a.q_len;
   if (active)
     store_row4<OUT_DT>(a.out, h * a.out_hs + t * a.out_ss + c, make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv));
-  if (a.lse_out != nullptr && threadIdx.x == 0) a.lse_out[h * a.lse_out_hs + t] = dt > 0.f ? mt + __logf(dt) : -INFINITY;
+  if (a.lse_out != nullptr && threadIdx.x == 0) a.lse_out[h * a.lse_out_hs + t] = merged_lse(mt, dt);
 }
 
 template <int OUT_DT, int NP, int R>
@@ -165,7 +174,11 @@ __global__ __launch_bounds__(256) void lse_merge_kernel(MergeArgs a) {
 #pragma unroll
       for (int u = 1; u < NP; ++u) mg = fmaxf(mg, l[k][u]);
       const float mn = fmaxf(m[k], mg);
-      if (mn == -INFINITY) continue;  // every partial so far is empty
+      if (mn == -INFINITY) {  // every partial so far is empty, or its LSE a NaN, which the sum keeps
+#pragma unroll
+        for (int u = 0; u < NP; ++u) den[k] += __expf(l[k][u]);
+        continue;
+      }
       const float sc = __expf(m[k] - mn);  // 0 while m = -inf
       den[k] *= sc;
       acc[k].x *= sc;
@@ -190,14 +203,13 @@ __global__ __launch_bounds__(256) void lse_merge_kernel(MergeArgs a) {
     if (row >= rows) break;
     const int64_t h = row / a.q_len;
     const int64_t t = row - h * a.q_len;
-    const bool any = m[k] != -INFINITY;
-    const float inv = (any && den[k] > 0.f) ? 1.f / den[k] : 0.f;
+    const float inv = den[k] > 0.f ? 1.f / den[k] : den[k];  // 0: empty; NaN stays
     if (active) {
       const int64_t base = h * a.out_hs + t * a.out_ss + c;
       store_row4<OUT_DT>(a.out, base, make_float4(acc[k].x * inv, acc[k].y * inv, acc[k].z * inv, acc[k].w * inv));
     }
     if (a.lse_out != nullptr && lane_in_row == 0) {
-      a.lse_out[h * a.lse_out_hs + t] = (any && den[k] > 0.f) ? m[k] + __logf(den[k]) : -INFINITY;
+      a.lse_out[h * a.lse_out_hs + t] = merged_lse(m[k], den[k]);
     }
   }
 }

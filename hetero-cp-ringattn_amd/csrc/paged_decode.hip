@@ -340,7 +340,7 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(DecodeArgs a) {
 #pragma unroll
       for (int k = 0; k < D / 64; ++k)
         if (!PAD || lane + 64 * k < dn) a.ws_o[row * dn + lane + 64 * k] = o[k] * inv;
-      if (lane == 0) a.ws_lse[row] = den > 0.f ? (m + __log2f(den)) * kLn2 : -INFINITY;
+      if (lane == 0) a.ws_lse[row] = den == 0.f ? -INFINITY : (m + __log2f(den)) * kLn2;  // NaN stays
     }
     return;
   }
@@ -360,8 +360,9 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(DecodeArgs a) {
     }
   }
   if (lane < a.rep && lane < R) {
-    const float lt = l;  // lane c holds column c's total
-    a.ws_lse[ws_row_base + kvh * a.rep + lane] = lt > 0.f ? (m_run + __log2f(lt)) * kLn2 : -INFINITY;
+    // lane c holds column c's total; a NaN one (a NaN key) stays, so the merge cannot take
+    // the part for an empty one
+    a.ws_lse[ws_row_base + kvh * a.rep + lane] = l == 0.f ? -INFINITY : (m_run + __log2f(l)) * kLn2;
   }
 }
 

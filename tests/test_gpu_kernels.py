@@ -1705,3 +1705,75 @@ def test_strategy_replay_workspace_at_any_address(gpu, dt, strategy, paged):
         assert np.abs(o.float().cpu().numpy() - ref_o.transpose(1, 0, 2)).max() <= (1e-4 if f32 else OUT_TOL)
         assert np.abs(l.cpu().numpy() - ref_l.T).max() <= (1e-4 if f32 else LSE_TOL)
         assert torch.equal(o, results[0][0]) and torch.equal(l, results[0][1])
+
+
+# A NaN key of one sequence reaches every output row that sees it, whatever the runs, parts
+# and merge the step takes: one part, runs that meet in LDS, few and many rows to merge.
+DECODE_NAN_CASES = [
+    # batch, Hq, Hkv, D, tokens per shard, NaN token of sequence 0 (over its shards in turn)
+    (1, 8, 8, 128, [10], 3),
+    (2, 8, 1, 128, [100], 37),
+    (1, 32, 8, 128, [5, 90], 60),
+    (3, 14, 2, 64, [300, 45], 310),
+    (2, 16, 2, 128, [700, 700], 0),
+    (64, 32, 8, 128, [150, 40], 170),
+]
+
+
+@pytest.mark.parametrize("case", DECODE_NAN_CASES, ids=[f"{c[0]}x{sum(c[4])}_{c[1]}q{c[2]}kv_d{c[3]}" for c in DECODE_NAN_CASES])
+def test_decode_nan_key_reaches_its_rows(gpu, case):
+    b, hq, hkv, d, lens, bad = case
+    bs, rep = 16, hq // hkv
+    blocks = [-(-n // bs) for n in lens]
+    nb = b * sum(blocks)
+    (q, pool), _ = draw(1200 + hq, [(b, hq, d), (2, nb, bs, hkv, d)], torch.bfloat16)
+    tables = torch.arange(nb, dtype=torch.int32, device="cuda").view(b, -1)
+    shards, at = [], 0
+    for n, w in zip(lens, blocks):
+        shards.append((tables[:, at: at + w].contiguous(), torch.full((b,), n, dtype=torch.int32, device="cuda"), n))
+        at += w
+    clean, clean_l = H.decode_ring_replay(q, pool, shards, 0)
+    part = 0
+    while bad >= lens[part]:
+        bad -= lens[part]
+        part += 1
+    blk = sum(blocks[:part]) + bad // bs  # sequence 0's table
+    kvh = hkv - 1
+    pool[0, blk, bad % bs, kvh] = float("nan")
+    rows = slice(kvh * rep, hq)
+    for seed in range(len(shards)):
+        out, lse = H.decode_ring_replay(q, pool, shards, seed)
+        torch.cuda.synchronize()
+        assert bool(torch.isnan(out[0, rows]).all()) and bool(torch.isnan(lse[0, rows]).all()), seed
+        if seed == 0:
+            out[0, rows], lse[0, rows] = clean[0, rows], clean_l[0, rows]
+            assert torch.equal(out, clean) and torch.equal(lse, clean_l)  # no other row changed
+    tables0, lens0, n0 = shards[part]
+    o, l = H.decode_local_compact_partial(q, pool, tables0, 0, n0, seq_lens=lens0)
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(o[0, rows]).all()) and bool(torch.isnan(l[0, rows]).all())
+
+
+@pytest.mark.parametrize("rows", [3, 1500], ids=["few_rows", "many_rows"])
+@pytest.mark.parametrize("n", [2, 5, 11, 40])
+def test_lse_merge_nan_partial(gpu, n, rows):
+    # One NaN partial among finite and empty ones: its row is NaN; an all-empty row stays
+    # (0, -inf) whatever its partials' o hold.
+    for d, where in ((128, 0), (64, n - 1), (128, n // 2)):
+        for nan_lse in (True, False):
+            o = torch.ones(n, 2, rows, d, dtype=torch.float32, device="cuda")
+            l = torch.zeros(n, 2, rows, dtype=torch.float32, device="cuda")
+            l[1:, 0, 1] = -math.inf                      # one finite partial left in this row
+            l[:, 1, 2] = -math.inf                       # no partial sees a key
+            o[:, 1, 2] = float("nan")
+            o[where, 0, 0] = float("nan")                # as a kernel leaves a NaN sum:
+            l[where, 0, 0] = float("nan") if nan_lse else -math.inf
+            out, lse = H.lse_merge(list(o), list(l), out_dtype=torch.float32)
+            torch.cuda.synchronize()
+            assert bool(torch.isnan(out[0, 0]).all()), (d, where, nan_lse)
+            assert bool(torch.isnan(lse[0, 0])) == nan_lse
+            assert bool((out[1, 2] == 0).all()) and float(lse[1, 2]) == -math.inf
+            out[0, 0], lse[0, 0] = 1.0, math.log(n)
+            out[1, 2], lse[1, 2] = 1.0, math.log(n)
+            lse[0, 1] += math.log(n)
+            assert float((out - 1).abs().max()) < 1e-6 and float((lse - math.log(n)).abs().max()) < 1e-5
