@@ -1382,13 +1382,15 @@ __global__ __launch_bounds__(kF32Threads) void mfma_f32_block_kernel(GenArgs a) 
     }
     mx = fmaxf(mx, __shfl_xor(mx, 32));
     const float m_new = fmaxf(m_run, mx);
-    // a row with no visible key so far keeps m = -inf, p = 0 and its (zero) state
+    // a row with no visible key so far keeps m = -inf, p = 0 and its (zero) state; a NaN
+    // score leaves no maximum but stays in p
     const bool none = m_new == -INFINITY;
     const float alpha = none ? 1.f : exp2f(m_run - m_new);
+    const float ref = none ? 0.f : m_new;
     float ls = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      p[i] = none ? 0.f : exp2f(p[i] - m_new);
+      p[i] = exp2f(p[i] - ref);
       ls += p[i];
     }
     l_run = l_run * alpha + ls;

@@ -1777,3 +1777,32 @@ def test_lse_merge_nan_partial(gpu, n, rows):
             out[1, 2], lse[1, 2] = 1.0, math.log(n)
             lse[0, 1] += math.log(n)
             assert float((out - 1).abs().max()) < 1e-6 and float((lse - math.log(n)).abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("positioned", [False, True], ids=["contiguous", "positions"])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_nan_key_alone_in_a_key_part(gpu, dt, positioned):
+    # Keys of which a whole part (32 or more of a step's) or all that a part's rows see are
+    # NaN: rows that see one are NaN, rows that see none are as without it.
+    lq, hq, hkv, d = 40, 4, 2, 64
+    for lk, bad in ((33, [32]), (97, [96]), (129, [128]), (160, list(range(32, 64))), (8, [0])):
+        (q, k, v), _ = draw(lk, [(lq, hq, d), (lk, hkv, d), (lk, hkv, d)], dt)
+        qv, kv, vv = (x.permute(1, 0, 2) for x in (q, k, v))
+        qo = max(bad) - lq // 2                          # half of the rows see every NaN key
+        ref = None
+        for nan in (False, True):
+            if nan:
+                k[bad] = float("nan")
+            if positioned:
+                got = H.block_partial_positioned(qv, torch.arange(qo + lq, qo + 2 * lq, device="cuda"), kv, vv,
+                                                 torch.arange(lq, lq + lk, device="cuda"))
+            else:
+                got = H.block_partial(qv, kv, vv, qo + lq, lq)
+            torch.cuda.synchronize()
+            ref = got if ref is None else ref
+        sees = torch.arange(qo, qo + lq, device="cuda") >= min(bad)
+        assert bool(torch.isnan(got[0][:, sees]).all()), lk
+        # (a NaN row may make its wave take a tile's maximum anew: other bits, the same value)
+        tol = OUT_TOL if dt == torch.bfloat16 else 1e-5
+        for x, y in zip(got, ref):
+            assert torch.allclose(x[:, ~sees], y[:, ~sees], rtol=0, atol=tol), lk
