@@ -119,12 +119,15 @@ __global__ __launch_bounds__(256) void lse_merge_few_rows_kernel(MergeArgs a) {
   for (int s = 0; s < used; ++s) mt = fmaxf(mt, m_l[threadIdx.x + s * lpr]);
   float dt = 0.f;
   float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int s = 0; s < used; ++s) {
-    const float w = mt == -INFINITY ? 1.f : __expf(m_l[threadIdx.x + s * lpr] - mt);
-    dt += w * den_l[threadIdx.x + s * lpr];
-    if (mt == -INFINITY) continue;  // no finite LSE: (0, -inf), or NaN with a NaN one
-    const float4 x = acc_l[threadIdx.x + s * lpr];
-    o.x += w * x.x; o.y += w * x.y; o.z += w * x.z; o.w += w * x.w;
+  if (mt != -INFINITY) {
+    for (int s = 0; s < used; ++s) {
+      const float w = __expf(m_l[threadIdx.x + s * lpr] - mt);
+      const float4 x = acc_l[threadIdx.x + s * lpr];
+      dt += w * den_l[threadIdx.x + s * lpr];
+      o.x += w * x.x; o.y += w * x.y; o.z += w * x.z; o.w += w * x.w;
+    }
+  } else {  // no finite LSE: 0, or NaN with a NaN one
+    for (int s = 0; s < used; ++s) dt += den_l[threadIdx.x + s * lpr];
   }
   const float inv = dt > 0.f ? 1.f / dt : dt;
   const int64_t h = row / a.q_len, t = row - h * a.q_len;
