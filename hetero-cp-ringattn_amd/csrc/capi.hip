@@ -1139,9 +1139,6 @@ int hcp_decode_ring_replay(const hcp_paged_decode_desc* desc, const hcp_paged_po
             "descriptor does not match the pool");
     require(pool->elem_bytes == 2, "paged decode needs a 16-bit pool");
     require(desc->scale > 0.f, "scale must be positive");
-    const size_t need = ring_workspace(desc, spans);
-    require(workspace != nullptr && workspace_bytes >= need,
-            "workspace too small: need " + std::to_string(need) + " bytes");
     check_view(q, "q", 1);
     require(mfma_layout_ok(q), "q must be 16-byte aligned with strides multiple of 8");
     check_view(out, "out", 1);

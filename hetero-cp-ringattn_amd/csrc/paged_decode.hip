@@ -382,6 +382,7 @@ const void* decode_fn(int r) {
 }
 
 constexpr int kMaxParts = 64;  // partials of one LSE merge
+constexpr int kFewParts = 16;  // parts that need no further halving of the heads
 
 size_t align_up256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 // Workspace of `parts` partials of every (sequence, head): o, then lse.
@@ -423,6 +424,36 @@ int decode_slots(int d, int dtype, int r, int waves) {
   return slots;
 }
 
+// 16-token groups of the longest sequence that the spans allow.
+int64_t span_groups(int n, const DecodeSpan* spans) {
+  int64_t groups = 0;
+  for (int i = 0; i < n; ++i)
+    if (spans[i].t1 > spans[i].t0) groups += (spans[i].t1 + 15) / 16 - spans[i].t0 / 16;
+  require(groups <= INT32_MAX / 16, "paged_decode: too many tokens");
+  return std::max<int64_t>(groups, 1);
+}
+
+// Most kv heads of a workgroup: all of them, or an even share of the waves.
+int whole_heads(int hkv) { return static_cast<int>(ceil_div(hkv, ceil_div(hkv, kDecWaves))); }
+
+// Rows of workgroups (sequences x head groups) of `heads` kv heads, and how many workgroups
+// are resident at once, with kDecWaves / heads runs each and with half of them (0: odd).
+struct DecodeSlots {
+  int64_t rows, whole, half;
+};
+DecodeSlots decode_level(int batch, int hq, int hkv, int d, int dtype, int heads) {
+  const int r = decode_width(hq / hkv), subs = kDecWaves / heads;
+  return {static_cast<int64_t>(batch) * ceil_div(hkv, heads), decode_slots(d, dtype, r, heads * subs),
+          heads * 2 <= kDecWaves ? decode_slots(d, dtype, r, heads * (subs / 2)) : 0};
+}
+
+// Parts whose bytes stay within the static scratch of the entry point that uses it (at
+// least one).
+int scratch_parts(int parts, int batch, int hq, int d) {
+  while (parts > 1 && parts_bytes(parts, batch, hq, d) > HCP_DECODE_STATIC_SCRATCH_BYTES) --parts;
+  return parts;
+}
+
 // Runs per sequence and kv head: as many as fill the chip once -- a partial second round of
 // workgroups leaves most CUs idle for its whole length (a measured 13-25% loss at c4) --
 // and at most one per 16-token group.  A workgroup holds whole token rows (all kv heads,
@@ -430,39 +461,43 @@ int decode_slots(int d, int dtype, int r, int waves) {
 // runs, and so on.  Decode steps of 64 / 16 / 4 / 1 sequences of 16384 tokens over three
 // shards: 634 / 169 / 56 / 26 us with 32/8 heads of 128, 195 / 57 / 28 / 26 us with 16/2
 // (one launch and merge per shard, at most 64 runs, at least 4 groups each: 660 / 205 /
-// 126 / 116 and 231 / 140 / 114 / 111 us).  The parts' bytes are kept within the static
-// scratch of the entry point that uses it.
+// 126 / 116 and 231 / 140 / 114 / 111 us).
 DecodePlan plan_decode(int batch, int hq, int hkv, int d, int dtype, int n, const DecodeSpan* spans) {
-  int64_t groups = 0;
-  for (int i = 0; i < n; ++i)
-    if (spans[i].t1 > spans[i].t0) groups += (spans[i].t1 + 15) / 16 - spans[i].t0 / 16;
-  require(groups <= INT32_MAX / 16, "paged_decode: too many tokens");
-  groups = std::max<int64_t>(groups, 1);
-  const int z = static_cast<int>(ceil_div(hkv, kDecWaves));
+  const int64_t groups = span_groups(n, spans);
   DecodePlan p{};
-  const int r = decode_width(hq / hkv);
-  for (int heads = static_cast<int>(ceil_div(hkv, z));; heads = (heads + 1) / 2) {
-    const int64_t rows = static_cast<int64_t>(batch) * ceil_div(hkv, heads);
+  for (int heads = whole_heads(hkv);; heads = (heads + 1) / 2) {
+    const DecodeSlots s = decode_level(batch, hq, hkv, d, dtype, heads);
     p.heads = heads;
     p.subs = kDecWaves / heads;
-    int64_t slots = decode_slots(d, dtype, r, heads * p.subs);
+    int64_t slots = s.whole;
     // half-size workgroups where more waves are resident that way (three a SIMD, say)
     // and the tokens are enough to use them: 64 x 16384 tokens of 14/2 heads of 64 dims
     // 106 us, 122 with whole ones
-    const int64_t half = heads * 2 <= kDecWaves ? decode_slots(d, dtype, r, heads * (p.subs / 2)) : 0;
-    if (half > 2 * slots && groups * rows >= half * (p.subs / 2)) {
+    if (s.half > 2 * s.whole && groups * s.rows >= s.half * (p.subs / 2)) {
       p.subs /= 2;
-      slots = half;
+      slots = s.half;
     }
-    p.parts = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({slots / rows, ceil_div(groups, p.subs), kMaxParts})));
-    if (p.parts <= 16 || heads == 1) break;
+    p.parts = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({slots / s.rows, ceil_div(groups, p.subs), kMaxParts})));
+    if (p.parts <= kFewParts || heads == 1) break;
   }
-  while (p.parts > 1 && parts_bytes(p.parts, batch, hq, d) > HCP_DECODE_STATIC_SCRATCH_BYTES) --p.parts;
+  p.parts = scratch_parts(p.parts, batch, hq, d);
   return p;
 }
 
+// Covers these spans and every shorter ones (a workspace sized once for the longest context
+// serves all of them), although fewer tokens can take more parts: a plan stops halving the
+// heads at kFewParts parts, so 11 sequences of 256 tokens, 32/8 heads, take 16, of 16384
+// tokens 11.  A plan that never halves has at most its first level's parts, any other at most
+// kFewParts or one kv head's, and none more than its groups.
 size_t decode_workspace_bytes(int dtype, int batch, int hq, int hkv, int d, int n, const DecodeSpan* spans) {
-  return parts_bytes(plan_decode(batch, hq, hkv, d, dtype, n, spans).parts, batch, hq, d);
+  auto most_at = [&](int heads) {
+    const DecodeSlots s = decode_level(batch, hq, hkv, d, dtype, heads);
+    return (s.half > 2 * s.whole ? s.half : s.whole) / s.rows;
+  };
+  int64_t most = most_at(whole_heads(hkv));
+  if (most > kFewParts) most = std::max<int64_t>(kFewParts, most_at(1));
+  most = std::max<int64_t>(1, std::min<int64_t>({most, span_groups(n, spans), kMaxParts}));
+  return parts_bytes(scratch_parts(static_cast<int>(most), batch, hq, d), batch, hq, d);
 }
 
 template <int D, int DT, bool PAD = false>
@@ -484,7 +519,8 @@ void launch_paged_decode(int dtype, int batch, int hq, int hkv, int d, const voi
   require(dtype == kBF16 || dtype == kF16, "paged_decode: dtype must be BF16 or F16");
   require(n >= 1 && n <= kMaxDomains, "paged_decode: 1 to 64 shards");
   const DecodePlan p = plan_decode(batch, hq, hkv, d, dtype, n, spans);
-  require(ws_bytes >= parts_bytes(p.parts, batch, hq, d), "paged_decode: workspace too small");
+  const size_t need = parts_bytes(p.parts, batch, hq, d);
+  require(ws != nullptr && ws_bytes >= need, "workspace too small: need " + std::to_string(need) + " bytes");
   const size_t rows = static_cast<size_t>(p.parts) * batch * hq;
   float* ws_o = static_cast<float*>(ws);
   float* ws_lse = reinterpret_cast<float*>(static_cast<char*>(ws) + align_up256(rows * d * sizeof(float)));

@@ -278,7 +278,8 @@ int hcp_paged_kv_gather_batch(const hcp_paged_pool* pool, int32_t num_ranges,
  *     o [batch, num_q_heads, head_dim], lse [batch, num_q_heads] (-inf, o = 0 when the
  *     range is empty).
  * The chunk is split across workgroups; workspace holds the split partials
- * (hcp_paged_decode_workspace_size bytes, 256-byte aligned).
+ * (hcp_paged_decode_workspace_size bytes, 256-byte aligned; they cover every shorter
+ * [t0, t1) of the same batch and heads, too).
  * dtype BF16 or F16, head_dim a multiple of 8 up to 128 (64: its own kernel; others run
  * the head-dim-128 kernel with the columns past head_dim zero-padded), block_size a
  * multiple of 16, and at most 16

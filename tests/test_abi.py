@@ -39,6 +39,24 @@ def test_positioned_workspace_size_covers_the_key_sort(hcp):
     assert hcp.lib().hcp_ring_block_partial_positioned_workspace_size(ctypes.byref(d)) == 0
 
 
+@pytest.mark.parametrize("heads", [(32, 8, 128), (16, 2, 128), (14, 2, 64), (24, 12, 96), (8, 1, 128), (40, 5, 64)])
+@pytest.mark.parametrize("batch", [1, 3, 11, 40, 300])
+def test_decode_workspace_covers_every_shorter_context(hcp, batch, heads):
+    # A workspace sized for the longest context serves shorter ones: the reported size never
+    # falls as the tokens grow, for one range and for a ring's shards.
+    hq, hkv, d = heads
+    pool = hcp.PagedPool(256, 1 << 16, 16, hkv, d, 2)
+    sizes, rings = [], []
+    for tokens in [*range(1, 1200, 13), 2048, 4099, 16384, 131072]:
+        desc = hcp.DecodeDesc(2, batch, hq, hkv, d, 0, 0, tokens, 1 << 14, 1 << 14, 0.1)
+        sizes.append(hcp.lib().hcp_paged_decode_workspace_size(ctypes.byref(desc), ctypes.byref(pool)))
+        shards = (hcp.DecodeShard * 3)(*[hcp.DecodeShard(256, 1 << 14, 1 << 14, None, t)
+                                         for t in (tokens, tokens // 2, tokens // 7)])
+        rings.append(hcp.lib().hcp_decode_ring_workspace_size(ctypes.byref(desc), ctypes.byref(pool), 3, shards))
+    for s in (sizes, rings):
+        assert s[0] > 0 and all(a <= b for a, b in zip(s, s[1:])), (batch, heads)
+
+
 def test_null_descriptor_is_invalid(hcp):
     v = hcp.View(0, 0, 1)
     rc = hcp.lib().hcp_ring_block_partial(None, v, v, v, None, None, None)

@@ -1806,3 +1806,20 @@ def test_nan_key_alone_in_a_key_part(gpu, dt, positioned):
         tol = OUT_TOL if dt == torch.bfloat16 else 1e-5
         for x, y in zip(got, ref):
             assert torch.allclose(x[:, ~sees], y[:, ~sees], rtol=0, atol=tol), lk
+
+
+@pytest.mark.parametrize("heads", [(32, 8, 128), (16, 2, 128), (14, 2, 64), (8, 1, 96)])
+@pytest.mark.parametrize("batch", [1, 5, 11, 36])
+def test_decode_workspace_sized_once_serves_shorter_contexts(gpu, batch, heads):
+    hq, hkv, d = heads
+    blocks = 70
+    (q, pool), _ = draw(1500 + batch, [(batch, hq, d), (2, blocks, 16, hkv, d)], torch.bfloat16)
+    table = torch.arange(blocks, dtype=torch.int32, device="cuda").expand(batch, blocks).contiguous()
+    ws = torch.empty(H.decode_ring_workspace_size(q, pool, [(table, None, 16 * blocks)]), dtype=torch.uint8, device="cuda")
+    for tokens in (1, 16, 17, 65, 130, 250, 256, 257, 400, 600, 16 * blocks):
+        out, lse = H.decode_ring_replay(q, pool, [(table, None, tokens)], 0, workspace=ws)
+        ref, ref_l = H.decode_ring_replay(q, pool, [(table, None, tokens)], 0)
+        o, l = H.decode_local_compact_partial(q, pool, table, 0, tokens, workspace=ws)
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref) and torch.equal(lse, ref_l) and torch.equal(l, ref_l), tokens
+        assert float((o - ref.float()).abs().max()) <= OUT_TOL
