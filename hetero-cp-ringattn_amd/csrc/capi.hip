@@ -1031,7 +1031,7 @@ int hcp_paged_kv_gather_batch(const hcp_paged_pool* pool, int32_t num_ranges, co
 namespace {
 size_t partial_workspace(const hcp_paged_decode_desc* d) {
   const DecodeSpan span{nullptr, 0, 0, nullptr, d->t0, d->t1};
-  return decode_workspace_bytes(d->dtype, d->batch, d->num_q_heads, d->num_kv_heads, d->head_dim, 1, &span);
+  return decode_workspace_bytes(d->batch, d->num_q_heads, d->head_dim, 1, &span);
 }
 }  // namespace
 extern "C" {
@@ -1106,8 +1106,7 @@ std::vector<DecodeSpan> ring_spans(const hcp_paged_decode_desc* desc, int n, con
   return spans;
 }
 size_t ring_workspace(const hcp_paged_decode_desc* d, const std::vector<DecodeSpan>& spans) {
-  return decode_workspace_bytes(d->dtype, d->batch, d->num_q_heads, d->num_kv_heads, d->head_dim,
-                                static_cast<int>(spans.size()), spans.data());
+  return decode_workspace_bytes(d->batch, d->num_q_heads, d->head_dim, static_cast<int>(spans.size()), spans.data());
 }
 }  // namespace
 extern "C" {

@@ -119,7 +119,7 @@ struct DecodeSpan {
   int64_t t0, t1;
 };
 // Workspace of launch_paged_decode for these shards, and for any shorter ones.
-size_t decode_workspace_bytes(int dtype, int batch, int hq, int hkv, int d, int n, const DecodeSpan* spans);
+size_t decode_workspace_bytes(int batch, int hq, int d, int n, const DecodeSpan* spans);
 // Attention of one query per sequence over its n shards, merged: out[row * out_rs + d] in
 // out_dtype and lse[row] (fp32, may be null) for row = b * hq + head.
 void launch_paged_decode(int dtype, int batch, int hq, int hkv, int d, const void* q, int64_t q_bs,

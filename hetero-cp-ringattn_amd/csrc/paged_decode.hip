@@ -12,8 +12,8 @@
 //     dealt out in equal contiguous runs to `parts` x `subs` waves, whatever its own
 //     length; grid = (parts, batch, ceil(Hkv / heads)), a workgroup holding `heads` kv
 //     heads x `subs` runs of one part.  The subs of a part meet in LDS, the parts in the
-//     LSE merge kernel.  The number of runs fills the chip once (see plan_decode): with a
-//     few sequences a run is down to one group.
+//     LSE merge kernel.  plan_decode picks the three by modelled time: with a few sequences
+//     a run is down to one group.
 //   * Per 16 tokens a wave reads 16 K rows and 16 V rows of its head (4 KiB each for D=128,
 //     bf16) straight from the pool; with many sequences a workgroup reads whole pool token
 //     rows (heads = min(8, Hkv); 4 heads a workgroup: 0.7% slower on c4).
@@ -28,9 +28,6 @@
 //   * Each part writes (o, lse) to the workspace; the LSE merge kernel combines the
 //     parts of a sequence (heads = batch*Hq, q_len = 1).
 #include <algorithm>
-#include <map>
-#include <mutex>
-#include <tuple>
 
 #include "kernels.hpp"
 #include "../../include/hcp_ring.h"
@@ -97,8 +94,12 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(DecodeArgs a) {
   constexpr int TPL = 16 * DCH / 64;  // keys per lane in PV (4 for D=128)
 
   __shared__ __attribute__((aligned(16))) float p_lds[kDecWaves][16][R];  // [wave][key][query col]
-  __shared__ __attribute__((aligned(16))) float o_lds[kDecWaves][R][D];   // subs > 1: the waves' O, m and l
-  __shared__ float m_lds[kDecWaves][R], l_lds[kDecWaves][R];
+  // subs > 1: the waves' O, m and l (meet_bytes; a launch whose runs do not meet holds none of
+  // it, and small workgroups stay as many to a CU as their registers allow)
+  extern __shared__ __attribute__((aligned(16))) float meet_lds[];
+  float (*const o_lds)[R][D] = reinterpret_cast<float (*)[R][D]>(meet_lds);
+  float (*const m_lds)[R] = reinterpret_cast<float (*)[R]>(meet_lds + kDecWaves * R * D);
+  float (*const l_lds)[R] = m_lds + kDecWaves;
 
   const int b = blockIdx.y;
   const int part = blockIdx.x;
@@ -372,17 +373,7 @@ struct DecodePlan {
 
 // Query heads per kv head the PV accumulators hold: the smallest of 4, 8, 16 >= rep.
 int decode_width(int rep) { return rep <= 4 ? 4 : rep <= 8 ? 8 : 16; }
-template <int D, int DT, bool PAD = false>
-const void* decode_fn(int r) {
-  switch (r) {
-    case 4: return reinterpret_cast<const void*>(&paged_decode_kernel<D, DT, 4, PAD>);
-    case 8: return reinterpret_cast<const void*>(&paged_decode_kernel<D, DT, 8, PAD>);
-    default: return reinterpret_cast<const void*>(&paged_decode_kernel<D, DT, 16, PAD>);
-  }
-}
-
 constexpr int kMaxParts = 64;  // partials of one LSE merge
-constexpr int kFewParts = 16;  // parts that need no further halving of the heads
 
 size_t align_up256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 // Workspace of `parts` partials of every (sequence, head): o, then lse.
@@ -391,37 +382,9 @@ size_t parts_bytes(int parts, int batch, int hq, int d) {
   return align_up256(rows * d * sizeof(float)) + align_up256(rows * sizeof(float));
 }
 
-// Workgroups of the decode kernel resident at once on the current device (CUs x
-// occupancy); 256 CUs x 3 when no device can be queried.
-int decode_slots(int d, int dtype, int r, int waves) {
-  static std::mutex mu;
-  static std::map<std::tuple<int, int, int, int, int>, int> cache;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) {
-    (void)hipGetLastError();
-    return 768;
-  }
-  std::lock_guard<std::mutex> lock(mu);
-  // the instantiation the launch takes: head dims other than 64 and 128 run the
-  // zero-padding (PAD) build of the 128 kernel, whose register use may differ
-  const bool pad = d != 64 && d != 128;
-  const int dk = d == 64 ? 64 : pad ? -1 : 128;
-  const auto key = std::make_tuple(dev, dk, dtype, r, waves);
-  auto it = cache.find(key);
-  if (it != cache.end()) return it->second;
-  int cus = 0, per_cu = 0;
-  const void* fn = dtype == kBF16
-                       ? (d == 64 ? decode_fn<64, kBF16>(r) : pad ? decode_fn<128, kBF16, true>(r) : decode_fn<128, kBF16>(r))
-                       : (d == 64 ? decode_fn<64, kF16>(r) : pad ? decode_fn<128, kF16, true>(r) : decode_fn<128, kF16>(r));
-  int slots = 768;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64 * waves, 0) == hipSuccess && cus > 0 &&
-      per_cu > 0)
-    slots = cus * per_cu;
-  else
-    (void)hipGetLastError();
-  cache[key] = slots;
-  return slots;
+// LDS in which the runs of a workgroup meet.
+size_t meet_bytes(int d, int r, int subs) {
+  return subs > 1 ? static_cast<size_t>(kDecWaves) * r * ((d == 64 ? 64 : 128) + 2) * sizeof(float) : 0;
 }
 
 // 16-token groups of the longest sequence that the spans allow.
@@ -433,79 +396,97 @@ int64_t span_groups(int n, const DecodeSpan* spans) {
   return std::max<int64_t>(groups, 1);
 }
 
-// Most kv heads of a workgroup: all of them, or an even share of the waves.
-int whole_heads(int hkv) { return static_cast<int>(ceil_div(hkv, ceil_div(hkv, kDecWaves))); }
-
-// Rows of workgroups (sequences x head groups) of `heads` kv heads, and how many workgroups
-// are resident at once, with kDecWaves / heads runs each and with half of them (0: odd).
-struct DecodeSlots {
-  int64_t rows, whole, half;
-};
-DecodeSlots decode_level(int batch, int hq, int hkv, int d, int dtype, int heads) {
-  const int r = decode_width(hq / hkv), subs = kDecWaves / heads;
-  return {static_cast<int64_t>(batch) * ceil_div(hkv, heads), decode_slots(d, dtype, r, heads * subs),
-          heads * 2 <= kDecWaves ? decode_slots(d, dtype, r, heads * (subs / 2)) : 0};
-}
-
-// Parts whose bytes stay within the static scratch of the entry point that uses it (at
-// least one).
-int scratch_parts(int parts, int batch, int hq, int d) {
+// Most parts of a plan: what one merge takes, no more than the groups, and within the static
+// scratch of the entry point that uses it (at least one).  Never fewer for more groups.
+int most_parts(int batch, int hq, int d, int64_t groups) {
+  int parts = static_cast<int>(std::min<int64_t>(groups, kMaxParts));
   while (parts > 1 && parts_bytes(parts, batch, hq, d) > HCP_DECODE_STATIC_SCRATCH_BYTES) --parts;
   return parts;
 }
 
-// Runs per sequence and kv head: as many as fill the chip once -- a partial second round of
-// workgroups leaves most CUs idle for its whole length (a measured 13-25% loss at c4) --
-// and at most one per 16-token group.  A workgroup holds whole token rows (all kv heads,
-// up to 8) while that leaves at most 16 parts to merge, else half the heads and twice the
-// runs, and so on.  Decode steps of 64 / 16 / 4 / 1 sequences of 16384 tokens over three
-// shards: 634 / 169 / 56 / 26 us with 32/8 heads of 128, 195 / 57 / 28 / 26 us with 16/2
-// (one launch and merge per shard, at most 64 runs, at least 4 groups each: 660 / 205 /
-// 126 / 116 and 231 / 140 / 114 / 111 us).
-DecodePlan plan_decode(int batch, int hq, int hkv, int d, int dtype, int n, const DecodeSpan* spans) {
+// The plan with the least modelled time, in us, over 1, 2, 4 or 8 runs a workgroup, all kv
+// heads of it (up to 8), half of them and so on, and parts that make short runs (up to 8
+// groups) or that give every CU 1, 2, 3, ... workgroups:
+//   * the fullest CU's share of the groups at a CU's rate (`group` per 16 tokens of a kv head
+//     of 128 dims), or the groups of a run one after another (`chain` each) times the rounds
+//     of resident workgroups, whichever is longer.  A CU takes in at most its own rate, so a
+//     workgroup count that does not divide over the CUs costs its whole last round: 130
+//     sequences of 700 tokens, 24/4 heads, took 64.7 us as 390 workgroups of 8 waves, 45 as
+//     1560 of one.  Workgroups that read part of a token's row cost 2.5% more, and if their
+//     runs lie apart as well (runs that meet) up to a third: 32 sequences of 8000 tokens,
+//     32/8 heads, 190 us as 8 runs of one head a workgroup, 164 as 8 parts of whole rows;
+//   * `meet` where runs meet in LDS, the more the wider the accumulators: one sequence of 40
+//     tokens, 32/2 heads of 64 dims, 20.0 us with four runs that meet, 13.6 as three parts;
+//   * the parts written and read again, the merge's chain over them and its batches of
+//     loads in flight (32 parts of 128 dims, 64 of 64);
+//   * the start of every workgroup.
+// Per accumulator width R = 4, 8, 16 and head dim 128, 64.  Fitted on MI355X to 602 calls: 12
+// head layouts (8/1 to 64/8 heads of 64, 96 and 128 dims), 1-400 sequences of 40-16384
+// tokens, some 70 plans each: the model's choice among them is 1.6% above the fastest on
+// average.  Against as many runs as fill the chip once, the heads halved while more than 16
+// parts resulted, these calls take 8% less on average; 32/8, 16/2 and 14/2 heads, 1-64
+// sequences: none more than 6% longer; the worst, 16 sequences of 6000 tokens of 64/8 heads,
+// 89 us against 77.
+DecodePlan plan_decode(int batch, int hq, int hkv, int d, int n, const DecodeSpan* spans) {
+  static const double group[3][2] = {{0.181, 0.157}, {0.229, 0.146}, {0.281, 0.322}};
+  static const double chain[3][2] = {{1.09, 0.84}, {1.37, 0.78}, {1.97, 1.36}};
+  static const double meet[3] = {1.1, 1.95, 6.9};
+  static const int waves_per_cu[3][2] = {{12, 16}, {8, 12}, {8, 8}};  // resident, by registers
+  constexpr double kPartRows = 0.025, kApart = 0.047;
+  constexpr double kPartValue = 4.4e-6, kPart = 0.029, kPartBatch = 0.8, kStart = 0.05;
   const int64_t groups = span_groups(n, spans);
-  DecodePlan p{};
-  for (int heads = whole_heads(hkv);; heads = (heads + 1) / 2) {
-    const DecodeSlots s = decode_level(batch, hq, hkv, d, dtype, heads);
-    p.heads = heads;
-    p.subs = kDecWaves / heads;
-    int64_t slots = s.whole;
-    // half-size workgroups where more waves are resident that way (three a SIMD, say)
-    // and the tokens are enough to use them: 64 x 16384 tokens of 14/2 heads of 64 dims
-    // 106 us, 122 with whole ones
-    if (s.half > 2 * s.whole && groups * s.rows >= s.half * (p.subs / 2)) {
-      p.subs /= 2;
-      slots = s.half;
+  const int r = decode_width(hq / hkv), w = r <= 4 ? 0 : r <= 8 ? 1 : 2, h = d == 64 ? 1 : 0;
+  const int cus = device_cus(), most = most_parts(batch, hq, d, groups);
+  const int whole = static_cast<int>(ceil_div(hkv, ceil_div(hkv, kDecWaves)));
+  const double part = kPartValue * batch * hq * d + kPart;
+  DecodePlan best{1, whole, 1};
+  double best_t = 0.0;
+  for (int heads = whole;; heads = (heads + 1) / 2) {
+    const int64_t rows = static_cast<int64_t>(batch) * ceil_div(hkv, heads);
+    for (int subs = 1; heads * subs <= kDecWaves; subs *= 2) {
+      const int waves = heads * subs, resident = std::max(1, waves_per_cu[w][h] / waves);
+      const double apart = subs > 1 ? kApart * (static_cast<double>(whole) / heads - 1.0) : 0.0;
+      const double unit = group[w][h] * d / 128 * waves * (1.0 + (heads < whole ? kPartRows : 0.0) + apart);
+      const int64_t shares = std::min<int64_t>(ceil_div(groups, subs), most);  // most parts
+      auto consider = [&](int64_t want) {
+        const int64_t len = ceil_div(groups, subs * std::min(std::max<int64_t>(want, 1), shares));  // groups of a run
+        const int64_t parts = ceil_div(groups, subs * len), per_cu = ceil_div(rows * parts, cus);
+        const double run = static_cast<double>(len);
+        const double t = std::max(unit * per_cu * run, chain[w][h] * run * ceil_div(per_cu, resident)) +
+                         (subs > 1 ? meet[w] : 0.0) + part * parts + kPartBatch * ((parts - 1) / (h ? 64 : 32)) +
+                         kStart * per_cu;
+        if (best_t == 0.0 || t < best_t) {
+          best = DecodePlan{static_cast<int>(parts), heads, subs};
+          best_t = t;
+        }
+      };
+      for (int64_t len : {1, 2, 3, 4, 6, 8}) consider(ceil_div(groups, subs * len));
+      if (rows >= cus)
+        for (int64_t parts : {1, 2, 3, 4, 6, 8, 12}) consider(parts);
+      else
+        for (int64_t k : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16}) {
+          consider(k * cus / rows);
+          if (k * cus / rows >= shares) break;
+        }
     }
-    p.parts = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({slots / s.rows, ceil_div(groups, p.subs), kMaxParts})));
-    if (p.parts <= kFewParts || heads == 1) break;
+    if (heads == 1) break;
   }
-  p.parts = scratch_parts(p.parts, batch, hq, d);
-  return p;
+  return best;
 }
 
-// Covers these spans and every shorter ones (a workspace sized once for the longest context
-// serves all of them), although fewer tokens can take more parts: a plan stops halving the
-// heads at kFewParts parts, so 11 sequences of 256 tokens, 32/8 heads, take 16, of 16384
-// tokens 11.  A plan that never halves has at most its first level's parts, any other at most
-// kFewParts or one kv head's, and none more than its groups.
-size_t decode_workspace_bytes(int dtype, int batch, int hq, int hkv, int d, int n, const DecodeSpan* spans) {
-  auto most_at = [&](int heads) {
-    const DecodeSlots s = decode_level(batch, hq, hkv, d, dtype, heads);
-    return (s.half > 2 * s.whole ? s.half : s.whole) / s.rows;
-  };
-  int64_t most = most_at(whole_heads(hkv));
-  if (most > kFewParts) most = std::max<int64_t>(kFewParts, most_at(1));
-  most = std::max<int64_t>(1, std::min<int64_t>({most, span_groups(n, spans), kMaxParts}));
-  return parts_bytes(scratch_parts(static_cast<int>(most), batch, hq, d), batch, hq, d);
+// Covers these spans and any shorter ones: a workspace sized once for the longest context
+// serves all of them.
+size_t decode_workspace_bytes(int batch, int hq, int d, int n, const DecodeSpan* spans) {
+  return parts_bytes(most_parts(batch, hq, d, span_groups(n, spans)), batch, hq, d);
 }
 
 template <int D, int DT, bool PAD = false>
 static void launch_decode_kernel(int r, dim3 grid, int waves, const DecodeArgs& a, hipStream_t stream) {
+  const size_t lds = meet_bytes(D, r, a.subs);
   switch (r) {
-    case 4: paged_decode_kernel<D, DT, 4, PAD><<<grid, 64 * waves, 0, stream>>>(a); break;
-    case 8: paged_decode_kernel<D, DT, 8, PAD><<<grid, 64 * waves, 0, stream>>>(a); break;
-    default: paged_decode_kernel<D, DT, 16, PAD><<<grid, 64 * waves, 0, stream>>>(a); break;
+    case 4: paged_decode_kernel<D, DT, 4, PAD><<<grid, 64 * waves, lds, stream>>>(a); break;
+    case 8: paged_decode_kernel<D, DT, 8, PAD><<<grid, 64 * waves, lds, stream>>>(a); break;
+    default: paged_decode_kernel<D, DT, 16, PAD><<<grid, 64 * waves, lds, stream>>>(a); break;
   }
 }
 
@@ -518,7 +499,7 @@ void launch_paged_decode(int dtype, int batch, int hq, int hkv, int d, const voi
   require(d > 0 && d <= 128 && d % 8 == 0, "paged_decode: head_dim must be a multiple of 8 up to 128");
   require(dtype == kBF16 || dtype == kF16, "paged_decode: dtype must be BF16 or F16");
   require(n >= 1 && n <= kMaxDomains, "paged_decode: 1 to 64 shards");
-  const DecodePlan p = plan_decode(batch, hq, hkv, d, dtype, n, spans);
+  const DecodePlan p = plan_decode(batch, hq, hkv, d, n, spans);
   const size_t need = parts_bytes(p.parts, batch, hq, d);
   require(ws != nullptr && ws_bytes >= need, "workspace too small: need " + std::to_string(need) + " bytes");
   const size_t rows = static_cast<size_t>(p.parts) * batch * hq;

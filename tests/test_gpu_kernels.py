@@ -1823,3 +1823,34 @@ def test_decode_workspace_sized_once_serves_shorter_contexts(gpu, batch, heads):
         torch.cuda.synchronize()
         assert torch.equal(out, ref) and torch.equal(lse, ref_l) and torch.equal(l, ref_l), tokens
         assert float((o - ref.float()).abs().max()) <= OUT_TOL
+
+
+@pytest.mark.parametrize("heads", [(32, 8, 128), (14, 2, 64), (24, 4, 128), (8, 1, 96), (12, 12, 64), (40, 20, 128)])
+@pytest.mark.parametrize("batch", [1, 7, 60, 130, 300])
+def test_decode_plans_over_batches_match_closed_form(gpu, batch, heads):
+    # Few to many workgroups per CU, one to eight runs a workgroup, kv heads that do not fill
+    # the last workgroup; ragged sequences over one and two shards, sampled rows in float64.
+    hq, hkv, d = heads
+    blocks, bs = 40, 16
+    (q, pool), (q32, pool32) = draw(1600 + batch + hq, [(batch, hq, d), (2, blocks, bs, hkv, d)], torch.bfloat16)
+    flat = pool32.reshape(2, blocks * bs, hkv, d)
+    rng = np.random.default_rng(batch + hq)
+    tables = [np.stack([rng.permutation(blocks)[:w] for _ in range(batch)]).astype(np.int32) for w in (33, 7)]
+    for max_lens in ((5,), (16 * 33 - 3,), (16 * 20 + 1, 16 * 7)):
+        lens = [rng.integers(0, m + 1, batch) for m in max_lens]
+        lens[0][0] = max_lens[0]
+        shards = [(torch.from_numpy(t).cuda(), torch.tensor(n, dtype=torch.int32, device="cuda"), m)
+                  for t, n, m in zip(tables, lens, max_lens)]
+        out, lse = H.decode_ring_replay(q, pool, shards, len(shards) - 1)
+        torch.cuda.synchronize()
+        out, lse = out.float().cpu().numpy(), lse.cpu().numpy()
+        for i in {0, batch // 2, batch - 1}:
+            tokens = [t[i, j // bs] * bs + j % bs for t, n in zip(tables, lens) for j in range(n[i])]
+            if not tokens:
+                assert np.all(out[i] == 0) and np.all(np.isneginf(lse[i]))
+                continue
+            ref_o, ref_l = C.attention_f64(q32[i:i + 1], flat[0, tokens], flat[1, tokens], np.zeros(1),
+                                           np.zeros(len(tokens)), 1 / math.sqrt(d), causal=False)
+            assert np.abs(out[i] - ref_o[0]).max() <= OUT_TOL, (max_lens, i)
+            assert np.abs(lse[i] - ref_l[0]).max() <= LSE_TOL, (max_lens, i)
+    assert H.fetch_device_errors() == 0
