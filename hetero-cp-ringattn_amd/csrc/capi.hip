@@ -1063,7 +1063,11 @@ int hcp_paged_decode_partial(const hcp_paged_decode_desc* desc, const hcp_paged_
     require(desc->scale > 0.f, "scale must be positive");
     check_view(q, "q", 1);
     require(mfma_layout_ok(q), "q must be 16-byte aligned with strides multiple of 8");
-    const DecodeSpan span{block_tables, desc->table_stride, desc->table_len, seq_lens, desc->t0, desc->t1};
+    const bool any = desc->t1 > desc->t0;
+    const int64_t skip = any ? desc->t0 / pool->block_size : 0;  // whole blocks before t0
+    const int64_t off = skip * pool->block_size;
+    const DecodeSpan span{block_tables + skip, desc->table_stride, desc->table_len - skip, seq_lens,
+                          any ? desc->t0 - off : 0, any ? desc->t1 - off : 0, off};
     launch_paged_decode(desc->dtype, desc->batch, desc->num_q_heads, desc->num_kv_heads, desc->head_dim, q.data,
                         q.seq_stride, q.head_stride, pool->data, pool->num_blocks, pool->block_size, 1, &span,
                         desc->scale, kF32, o, desc->head_dim, lse, workspace, workspace_bytes, device_error_flags(),

@@ -110,13 +110,16 @@ void launch_paged_copy(bool gather, void* pool, int64_t num_blocks, int bs, int 
                        int64_t t1, void* k_buf, void* v_buf, int64_t head_stride, int64_t seq_stride,
                        int zero_tail, int* err, hipStream_t stream);
 
-// One shard of every sequence's paged KV: tokens [t0, min(t1, seq_lens[b])) through row b
-// of its block tables.
+// One shard of every sequence's paged KV: tokens [t0, min(t1, seq_lens[b] - len_off)) through
+// row b of its block tables.  t0 lies in the first block (16-token groups are counted in 32
+// bits from the table's start): a range further on comes with the tables' later entries and
+// the tokens skipped as len_off.
 struct DecodeSpan {
   const int32_t* tables;
   int64_t table_stride, table_len;
   const int32_t* seq_lens;  // or null
   int64_t t0, t1;
+  int64_t len_off = 0;
 };
 // Workspace of launch_paged_decode for these shards, and for any shorter ones.
 size_t decode_workspace_bytes(int batch, int hq, int d, int n, const DecodeSpan* spans);

@@ -120,7 +120,7 @@ __global__ __launch_bounds__(512) void paged_decode_kernel(DecodeArgs a) {
   auto span_end = [&](int s) __attribute__((always_inline)) -> int64_t {
     const DecodeSpan& sp = a.span[s];
     if (sp.seq_lens == nullptr) return sp.t1;
-    return min(sp.t1, static_cast<int64_t>(__builtin_amdgcn_readfirstlane(sp.seq_lens[b])));
+    return min(sp.t1, static_cast<int64_t>(__builtin_amdgcn_readfirstlane(sp.seq_lens[b])) - sp.len_off);
   };
   auto span_groups = [&](int s, int64_t t_end) __attribute__((always_inline)) {
     const int64_t t0 = a.span[s].t0;
@@ -392,7 +392,7 @@ int64_t span_groups(int n, const DecodeSpan* spans) {
   int64_t groups = 0;
   for (int i = 0; i < n; ++i)
     if (spans[i].t1 > spans[i].t0) groups += (spans[i].t1 + 15) / 16 - spans[i].t0 / 16;
-  require(groups <= INT32_MAX / 16, "paged_decode: too many tokens");
+  require(groups <= INT32_MAX / 2, "paged_decode: too many tokens");  // the kernel counts them in 32 bits
   return std::max<int64_t>(groups, 1);
 }
 
@@ -499,6 +499,7 @@ void launch_paged_decode(int dtype, int batch, int hq, int hkv, int d, const voi
   require(d > 0 && d <= 128 && d % 8 == 0, "paged_decode: head_dim must be a multiple of 8 up to 128");
   require(dtype == kBF16 || dtype == kF16, "paged_decode: dtype must be BF16 or F16");
   require(n >= 1 && n <= kMaxDomains, "paged_decode: 1 to 64 shards");
+  for (int i = 0; i < n; ++i) require(spans[i].t0 >= 0 && spans[i].t0 < bs, "paged_decode: a span starts in its first block");
   const DecodePlan p = plan_decode(batch, hq, hkv, d, n, spans);
   const size_t need = parts_bytes(p.parts, batch, hq, d);
   require(ws != nullptr && ws_bytes >= need, "workspace too small: need " + std::to_string(need) + " bytes");

@@ -1854,3 +1854,28 @@ def test_decode_plans_over_batches_match_closed_form(gpu, batch, heads):
             assert np.abs(out[i] - ref_o[0]).max() <= OUT_TOL, (max_lens, i)
             assert np.abs(lse[i] - ref_l[0]).max() <= LSE_TOL, (max_lens, i)
     assert H.fetch_device_errors() == 0
+
+
+def test_decode_partial_far_into_a_long_table(gpu):
+    # A range that starts 2^35 tokens into the table (large blocks, so the table stays small):
+    # 16-token groups before it are past 32 bits.  77 tokens over the end of one block and the
+    # start of the next, against float64; with sequence lengths that end before it, none.
+    bs, far, hq, hkv, d = 1 << 20, 1 << 35, 4, 1, 8
+    pool = torch.zeros(2, 2, bs, hkv, d, dtype=torch.bfloat16, device="cuda")
+    (q, kv), (q32, kv32) = draw(1700, [(1, hq, d), (2, 77, hkv, d)], torch.bfloat16)
+    pool[:, 1, bs - 37:], pool[:, 0, :40] = kv[:, :37], kv[:, 37:]
+    table = torch.full((1, far // bs + 2), -1, dtype=torch.int32)
+    table[0, far // bs], table[0, far // bs + 1] = 1, 0
+    t0 = far + bs - 37
+    o, lse = H.decode_local_compact_partial(q, pool, table.cuda(), t0, t0 + 77)
+    torch.cuda.synchronize()
+    assert H.fetch_device_errors() == 0
+    ref_o, ref_l = C.attention_f64(q32, kv32[0], kv32[1], np.zeros(1), np.zeros(77), 1 / math.sqrt(d), causal=False)
+    assert np.abs(o.cpu().numpy() - ref_o).max() <= OUT_TOL and np.abs(lse.cpu().numpy() - ref_l).max() <= LSE_TOL
+    lens = torch.tensor([2 ** 31 - 1], dtype=torch.int32, device="cuda")
+    o, lse = H.decode_local_compact_partial(q, pool, table.cuda(), t0, t0 + 77, seq_lens=lens)
+    torch.cuda.synchronize()
+    assert bool((o == 0).all()) and bool(torch.isneginf(lse).all())
+    o, lse = H.decode_local_compact_partial(q, pool, table.cuda(), t0, t0, seq_lens=lens)
+    torch.cuda.synchronize()
+    assert bool((o == 0).all()) and bool(torch.isneginf(lse).all()) and H.fetch_device_errors() == 0
