@@ -656,17 +656,23 @@ static void launch_few_tokens(int dtype, int d, const QkvArgs& a, unsigned grid,
 }
 
 // Token blocks (of 16) per workgroup of the few-tokens kernel, 0 where the tiled kernel is
-// the faster one.  The few-tokens kernel wins as long as its workgroups fit one round of
-// the CUs, or take one token tile: every further round costs another pass over the
-// weights.  Measured, tiled / few: 32/8 heads of 128, hidden 4096: 46 / 12 us at 1 token,
-// 47 / 19 at 32, 51 / 26 at 64, 55 / 41 at 128 (192 workgroups), 54 / 78 at 200; 16/2
-// heads, hidden 2048: 36 / 23 at 256 (160 workgroups), 35 / 43 at 400 (320); 14/2 heads of
-// 64, hidden 896: 23 / 14 at 512 (144), 24 / 25 at 1024 (288).  Its per-lane offsets are
-// 32-bit: the weight rows of a head and 128 token rows must span less than 2 GiB.
+// the faster one.  Its workgroups each take in every token row beside their weights, and past
+// one round of the CUs that is paid again; the tiled kernel's time hardly depends on the
+// tokens.  In us, few / tiled:
+//   one round (up to 256 workgroups), up to 128 tokens: 32/8 heads of 128, hidden 4096: 1
+//     token 13 / 32, 32 19 / 33, 64 27 / 34, 96 36 / 35, 128 41 / 36; 16/2, hidden 2048: 64
+//     15 / 19, 128 22 / 20; 40/8, hidden 5120: 64 34 / 51, 128 50 / 56; and more tokens while
+//     their tiles fit it too: 14/2 of 64, hidden 896: 160 12.7 / 12.3;
+//   two rounds, up to 24: 64/8, hidden 8192 (320 workgroups): 1 41 / 58, 24 56 / 59, 33 70 /
+//     59, 64 91 / 60, 128 148 / 65; 32/32, hidden 4096 (384): 24 31 / 33, 33 39 / 34, 128 79 / 37;
+//   three, up to 16: 128/8, hidden 16384 (576): 1 130 / 153, 16 172 / 169, 64 313 / 190.
+// Its per-lane offsets are 32-bit: the weight rows of a head and 128 token rows must span
+// less than 2 GiB.
 static int few_token_blocks(int64_t n_feat, int64_t tokens, int d, int64_t hidden, int64_t x_ss, int cus) {
   constexpr int64_t kSpan = int64_t(1) << 31;
   if (d * hidden * 2 >= kSpan || x_ss >= kSpan / 256) return 0;
-  if (tokens > 128 && n_feat / 32 * ceil_div(tokens, 128) > cus) return 0;
+  const int64_t rounds = ceil_div(n_feat / 32 * ceil_div(tokens, 128), cus);
+  if (rounds > 1 && tokens > 48 / rounds) return 0;
   return tokens <= 16 ? 1 : tokens <= 32 ? 2 : tokens <= 64 ? 4 : 8;
 }
 

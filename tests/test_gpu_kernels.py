@@ -1879,3 +1879,19 @@ def test_decode_partial_far_into_a_long_table(gpu):
     o, lse = H.decode_local_compact_partial(q, pool, table.cuda(), t0, t0, seq_lens=lens)
     torch.cuda.synchronize()
     assert bool((o == 0).all()) and bool(torch.isneginf(lse).all()) and H.fetch_device_errors() == 0
+
+
+# Layers of more than one and two rounds of the few-tokens kernel's workgroups, at the token
+# counts where they turn to the tiled one.
+QKV_WIDE_CASES = [
+    (24, 64, 64, 8, 128, torch.bfloat16, False),
+    (25, 64, 64, 8, 128, torch.bfloat16, True),
+    (100, 96, 64, 64, 64, torch.float16, False),
+    (16, 64, 128, 8, 128, torch.bfloat16, True),
+    (17, 32, 128, 8, 128, torch.float16, False),
+]
+
+
+@pytest.mark.parametrize("case", QKV_WIDE_CASES, ids=[f"{c[0]}x{c[1]}_{c[2]}q{c[3]}kv_d{c[4]}" for c in QKV_WIDE_CASES])
+def test_qkv_rope_wide_layer_token_counts(gpu, case):
+    test_qkv_rope_token_count_edges(gpu, case)
