@@ -172,6 +172,12 @@ def last_path() -> str:
     return PATHS[lib().hcp_ring_last_path()]
 
 
+def last_key_parts() -> int:
+    """Waves that split each tile's keys in this thread's last block or replay launch (1, 2
+    or 4), hcp_ring_last_key_parts."""
+    return lib().hcp_ring_last_key_parts()
+
+
 def strategy_code(strategy) -> int:
     if isinstance(strategy, int):
         return strategy
@@ -197,6 +203,7 @@ def lib() -> ctypes.CDLL:
         "hcp_ring_last_error": ([], ctypes.c_char_p),
         "hcp_ring_abi_version": ([], ctypes.c_int),
         "hcp_ring_last_path": ([], ctypes.c_int),
+        "hcp_ring_last_key_parts": ([], ctypes.c_int),
         "hcp_ring_device_count": ([ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
         "hcp_ring_fetch_device_errors": ([vp, ctypes.POINTER(ctypes.c_int)], ctypes.c_int),
         "hcp_ring_block_partial": ([ctypes.POINTER(BlockDesc), View, View, View, vp, vp, vp],

@@ -37,8 +37,10 @@
 // K/V tiles staged in LDS as fp32.
 #include <algorithm>
 #include <atomic>
+#include <climits>
 #include <cmath>
 #include <cstdlib>
+#include <limits>
 #include <vector>
 
 #include "kernels.hpp"
@@ -1556,43 +1558,94 @@ int device_cus() {
 
 static bool half_width_d(int d);
 
-// Modelled time of a launch: its longest workgroup and its whole work spread over the CUs,
-// joined as a 4-norm (the workgroups of a causal launch neither all run at once nor queue
-// evenly).
-static double launch_time(double chain, double spread) {
-  return std::pow(std::pow(chain, 4) + std::pow(spread, 4), 0.25);
+static thread_local int g_key_parts = 0;
+int last_key_parts() { return g_key_parts; }
+
+// Key parts (KW) of a launch.  A workgroup of 1 / KW the rows splits every tile's keys over
+// KW waves: KW times the workgroups, each with a shorter chain of steps, for launches that
+// leave CUs idle; but every workgroup still brings whole K / V tiles to LDS, so on a full
+// chip it costs more.
+
+// What the choice weighs: the query rows of each block or chunk, the visible (query, key)
+// pairs of one head, the most and the fewest keys that a row folds (a launch without a mask:
+// the same), the runs of rows over which the keys ascend (0 for explicit positions of which
+// nothing is known: every key may be visible), and whether the pairs are a host's exact count.
+struct LaunchLoad {
+  const int64_t* rows;
+  int n;
+  double pairs;
+  int64_t most, fewest;
+  int runs;
+  bool exact;
+};
+
+// us per workgroup (first loads, rows written), and per step of keys on an idle and on a
+// full chip (lower clock, shared L2).
+struct KeyPartCost {
+  double own, alone, full;
+};
+
+static int64_t launch_items(const LaunchLoad& L, int n_groups, int tq) {
+  int64_t items = 0;
+  for (int b = 0; b < L.n; ++b) items += ceil_div(L.rows[b], tq) * n_groups;
+  return items;
 }
-// 1, 2 or 4 parts for the modelled times of each; a split has to be 6% ahead.
+
+// Modelled time of a launch of workgroups of tq rows that fold `step` keys a step: one
+// workgroup a CU, so one round takes as long as its longest one; further ones as long as the
+// whole work spread over the CUs, those idle in the last round counted with the least that a
+// workgroup does.
+static double launch_time(const LaunchLoad& L, int n_groups, int tq, int step, const KeyPartCost& c) {
+  const double cus = device_cus(), items = static_cast<double>(launch_items(L, n_groups, tq)), rounds = items / cus;
+  const double most = static_cast<double>(ceil_div(L.most, step));
+  const double fewest = static_cast<double>(ceil_div(std::min(L.most, L.fewest + tq - 1), step));
+  const double chain = c.own + most * (c.alone + (c.full - c.alone) * std::min(1.0, rounds));
+  if (rounds <= 1.0) return chain;
+  // under a mask a workgroup folds half the keys its rows span, or half a step, past its mean row
+  const double steps = most == fewest ? items * most
+                                      : std::min(items * most, n_groups * L.pairs / (static_cast<double>(tq) * step) +
+                                                                   items * std::max(0.5, 0.5 * L.runs * tq / step));
+  return std::max(chain, (items * c.own + steps * c.full) / cus + (std::ceil(rounds) - rounds) * (c.own + fewest * c.full));
+}
+
+// How far ahead a split has to be: 8%.  Past one round of workgroups, 40% if the pairs are an
+// estimate (12-22% ahead there measured up to 15% slower), and none is taken if nothing is
+// known of them: in one round a launch that sees few keys loses at most 1 us, in two 6%.
+static double split_margin(const LaunchLoad& L, int64_t items) {
+  if (L.exact || items <= device_cus()) return 1.08;
+  return L.runs > 0 ? 1.4 : std::numeric_limits<double>::infinity();
+}
+
 static int fewest_parts(const double (&t)[3]) {
-  if (std::min(t[1], t[2]) * 1.06 >= t[0]) return 1;
+  if (std::min(t[1], t[2]) >= t[0]) return 1;
   return t[1] <= t[2] ? 2 : 4;
 }
 
-// Key parts (KW) of a launch.  A workgroup of 256 / KW rows splits every tile's keys over
-// KW waves: KW times the workgroups, each with a shorter chain of tiles, for launches that
-// leave CUs idle; but every workgroup still brings whole K / V tiles to LDS, so on a full
-// chip it costs more.  The modelled times take, per KW = 1, 2, 4, in us: `own` per
-// workgroup (first loads, rows written), `alone` and `full` per 128-key tile on an idle and
-// on a full chip (lower clock, shared L2), fitted on MI355X to 74
-// launches: blocks of 16-4096 queries against 256-16384 keys, causal rings of 512-8192
-// tokens and ZigZag ones, with 32/8, 16/2, 16/16 heads of 128 and 14/2 of 64 dims.  There
-// it costs at most 3% against KW = 1 and saves up to 59% (512 x 16384, 32/8 heads: 271 us
-// with KW = 1, 165 with 2, 143 with 4; a 900-token ring 24.6, 19.0, 24.7; 3000 tokens 76,
-// 86, 117).
-//   pairs, rows, n_max: visible (query, key) pairs of one query head, query rows (of
-//   `blocks` chunks), and the most 128-key tiles that one row folds
-static int key_parts(double pairs, double rows, int blocks, double n_max, int hq, int hkv, int d) {
-  static const double own[3] = {4.0, 3.0, 3.0};
-  static const double alone[2][3] = {{2.03, 1.20, 0.81}, {1.83, 1.04, 0.67}};
-  static const double full[2][3] = {{3.26, 1.77, 1.07}, {2.22, 1.20, 0.55}};
-  const int w = half_width_d(d) ? 1 : 0;
-  const double cus = device_cus();
+// Key parts of the 16-bit kernels, 256 / KW rows a workgroup.  The costs (per 128-key tile;
+// head dims above 64, then up to 64; 4 us are the launch's own) are fitted on MI355X to 1000
+// launches, each measured with every KW: blocks of 16-8192 queries against 16-16384 keys, causal and
+// full rings of 200-9000 tokens, 8-64 heads of 24-128 dims, up to 8 on a KV head.  Of these
+// and 320 ZigZag and Striped replays 11 are slower than with KW = 1 by more than 3%, by at most
+// 9%; on average the launches are 17% faster than with KW = 1, 0.5% slower than with the best.
+// 512 x 16384, 32/8 heads: 271 us with KW = 1, 165 with 2, 143 with 4; a 900-token causal ring
+// 24.6, 19.0, 24.7; 4096 causal tokens, 16/2 heads, one round exactly with KW = 1, 98 and 73
+// with 2; 4345 x 2780 full keys, 8/8 heads, 69 with 136 workgroups and 92 with 272.
+//   One tile of keys: a split pays where it still fits one round and KW = 1 would have
+// more than half a workgroup of rows (348 x 104, 16/16 heads: 18.2 us, 15.7 with KW = 2;
+// 68 x 48: 10.8, 11.6).
+static int key_parts(const LaunchLoad& L, int hq, int hkv, int d) {
+  static const KeyPartCost costs[2][3] = {{{7.90, 1.885, 2.87}, {7.80, 1.12, 1.67}, {8.40, 0.775, 1.05}},
+                                          {{4.45, 1.685, 2.03}, {4.50, 1.04, 1.165}, {4.65, 0.75, 0.56}}};
+  if (L.most <= kBK3) {
+    const Geometry two = geometry(hq, hkv, 2);
+    const int64_t longest = *std::max_element(L.rows, L.rows + L.n);
+    return longest > geometry(hq, hkv).tq / 2 && launch_items(L, two.n_groups, two.tq) <= device_cus() ? 2 : 1;
+  }
   double t[3];
   for (int i = 0; i < 3; ++i) {
     const Geometry geo = geometry(hq, hkv, 1 << i);
-    const double items = geo.n_groups * (rows / geo.tq + 0.5 * blocks);
-    const double tiles = geo.n_groups * (pairs / kBK3 + 0.5 * rows) / geo.tq;
-    t[i] = launch_time(own[i] + n_max * alone[w][i], (items * own[i] + tiles * full[w][i]) / cus);
+    t[i] = 4.0 + launch_time(L, geo.n_groups, geo.tq, kBK3, costs[half_width_d(d) ? 1 : 0][i]);
+    if (i > 0) t[i] *= split_margin(L, launch_items(L, geo.n_groups, geo.tq));
   }
   return fewest_parts(t);
 }
@@ -1675,6 +1728,7 @@ static void launch_pingpong(BlockGroup& grp, const Geometry& geo, hipStream_t st
   for (int i = 0; i < grp.n; ++i) grp.qt_begin[i + 1] = grp.qt_begin[i] + grp.a[i].n_qtiles;
   const dim3 grid(static_cast<unsigned>(grp.qt_begin[grp.n] * a0.n_groups));
   const bool pos = a0.q_lim != nullptr;
+  g_key_parts = geo.kw;
   if (half_width_d(a0.d)) launch_pingpong_w<DT, kD3 / 2>(grp, geo, pos, grid, stream);
   else launch_pingpong_w<DT, kD3>(grp, geo, pos, grid, stream);
 }
@@ -1694,23 +1748,34 @@ static double block_work(const BlockLaunch& L) {
   return w;
 }
 
-// 128-key tiles that the last row of a block sees (explicit positions: some row may see
-// every key).
-static double block_tiles(const BlockLaunch& L) {
-  int64_t keys = L.lk;
-  if (L.causal && L.q_lim == nullptr) keys = std::max<int64_t>(0, std::min(L.lk, L.q_off + L.lq - L.k_off));
-  return static_cast<double>(ceil_div(keys, kBK3));
+// Keys that a row of a block sees (explicit positions: some row may see every key).
+static int64_t row_keys(const BlockLaunch& L, int64_t row) {
+  if (!L.causal || L.q_lim != nullptr) return L.lk;
+  return std::max<int64_t>(0, std::min(L.lk, L.q_off + row + 1 - L.k_off));
 }
 
-// Decomposition of a launch over the blocks Ls[0 .. n) (same heads and head dim).
-static Geometry block_geometry(const BlockLaunch* const* Ls, int n) {
-  double pairs = 0.0, rows = 0.0, n_max = 0.0;
+// What key_parts weighs of a launch over the blocks Ls[0 .. n), their query rows into `rows`.
+static LaunchLoad block_load(const BlockLaunch* const* Ls, int n, int64_t* rows) {
+  LaunchLoad load{rows, n, 0.0, 0, INT64_MAX, INT_MAX, true};
   for (int i = 0; i < n; ++i) {
-    pairs += block_work(*Ls[i]);
-    rows += static_cast<double>(Ls[i]->lq);
-    n_max = std::max(n_max, block_tiles(*Ls[i]));
+    const BlockLaunch& L = *Ls[i];
+    const bool positions = L.causal && L.q_lim != nullptr;
+    const int runs = positions ? L.lim_runs : 1;
+    rows[i] = L.lq;
+    load.pairs += runs > 0 ? block_work(L) : static_cast<double>(L.lq) * static_cast<double>(L.lk);
+    load.most = std::max(load.most, row_keys(L, L.lq - 1));
+    load.fewest = std::min(load.fewest, positions && runs > 0 ? 1 : row_keys(L, 0));
+    load.runs = std::min(load.runs, runs);
+    load.exact = load.exact && (!positions || L.q_rows != nullptr);
   }
-  return geometry(Ls[0]->hq, Ls[0]->hkv, key_parts(pairs, rows, n, n_max, Ls[0]->hq, Ls[0]->hkv, Ls[0]->d));
+  return load;
+}
+
+// Decomposition of a launch over the blocks Ls[0 .. n) (same heads and head dim, at most
+// kMaxGroup).
+static Geometry block_geometry(const BlockLaunch* const* Ls, int n) {
+  int64_t rows[kMaxGroup];
+  return geometry(Ls[0]->hq, Ls[0]->hkv, key_parts(block_load(Ls, n, rows), Ls[0]->hq, Ls[0]->hkv, Ls[0]->d));
 }
 
 template <int DT>
@@ -1748,6 +1813,7 @@ template <int DT>
 static void launch_general(const BlockLaunch& L, hipStream_t stream) {
   const GenArgs a = make_gen_args(L);
   const dim3 grid(static_cast<unsigned>(ceil_div(L.lq, kGenRows)), static_cast<unsigned>(L.hq));
+  g_key_parts = 1;
   if (L.d <= 64) general_block_kernel<DT, 64><<<grid, kGenRows, 0, stream>>>(a);
   else if (L.d <= 128) general_block_kernel<DT, 128><<<grid, kGenRows, 0, stream>>>(a);
   else general_block_kernel<DT, 256><<<grid, kGenRows, 0, stream>>>(a);
@@ -1787,23 +1853,26 @@ static void launch_mfma_f32_k(const GenArgs& a, int64_t items, hipStream_t strea
   }
 }
 
-// Key parts of the fp32 kernel: 128 / KW rows a workgroup, as key_parts.  Per KW = 1, 2, 4
-// and 32, 64, 96, 128 padded dims, in us per 128 keys of a workgroup (96 dims between its
-// neighbours), fitted to causal sequences of 128-8192 tokens and blocks of 32-1024 queries
-// against 1024-4096 keys.  1024 tokens, 8 heads of 64 dims: 107 us with KW = 1, 64 with 2,
-// 43 with 4; 4096 tokens: 404, 285, 312; 32/8 heads of 128 dims, 4096 tokens: 1603, 1931,
-// 2717.
+// Key parts of the fp32 kernel: 128 / KW rows a workgroup, 32 KW keys a step, as key_parts.
+// Costs for 32, 64, 96, 128 padded dims, fitted to 855 launches as there (16-1500 queries,
+// 16-4096 keys; 8-64 heads of 24-128 dims): of these and 138 replays none is slower than with
+// KW = 1 by more than 3%.
+// 1024 tokens, 8 heads of 64 dims: 107 us with KW = 1, 64 with 2, 43 with 4; 4096 tokens:
+// 404, 285, 312; 32/8 heads of 128 dims, 4096 tokens: 1603, 1931, 2717; 439 x 138, 64 heads,
+// full: 49 in one round, 73, 136.
 static int f32_key_parts(const BlockLaunch& L) {
-  static const double alone[4][3] = {{7.4, 4.1, 2.3}, {12.3, 6.95, 4.25}, {18.0, 10.5, 6.9}, {23.5, 14.1, 9.5}};
-  static const double full[4][3] = {{6.0, 3.3, 1.75}, {11.0, 6.4, 4.5}, {17.6, 10.5, 7.4}, {24.3, 14.6, 10.3}};
-  constexpr double own = 5.0;
-  const int w = (L.d + 31) / 32 - 1;
-  const double cus = device_cus(), lq = static_cast<double>(L.lq), pairs = block_work(L), n_max = block_tiles(L);
+  static const KeyPartCost costs[4][3] = {{{6.2, 1.84, 1.80}, {6.3, 2.18, 1.74}, {6.1, 3.10, 1.64}},
+                                          {{7.6, 3.05, 3.15}, {7.9, 3.53, 3.49}, {8.7, 4.62, 4.20}},
+                                          {{8.9, 4.31, 4.48}, {9.5, 5.04, 5.26}, {11.3, 6.67, 6.52}},
+                                          {{11.6, 5.76, 6.06}, {12.5, 7.05, 7.18}, {14.4, 9.93, 9.53}}};
+  const BlockLaunch* const one = &L;
+  int64_t rows;
+  const LaunchLoad load = block_load(&one, 1, &rows);
   double t[3];
   for (int i = 0; i < 3; ++i) {
-    const double wgs = L.hq * std::ceil(lq / (kF32Rows >> i));
-    const double tiles = L.hq * (pairs / kBK3 + 0.25 * lq) / (kF32Rows >> i);
-    t[i] = launch_time(own + n_max * alone[w][i], (wgs * own + tiles * full[w][i]) / cus);
+    const int tq = kF32Rows >> i;
+    t[i] = launch_time(load, L.hq, tq, kF32BK << i, costs[(L.d + 31) / 32 - 1][i]);
+    if (i > 0) t[i] *= split_margin(load, launch_items(load, L.hq, tq));
   }
   return fewest_parts(t);
 }
@@ -1813,6 +1882,7 @@ static void launch_mfma_f32(const BlockLaunch& L, hipStream_t stream) {
   const int kw = f32_key_parts(L);
   const int64_t items = ceil_div(L.lq, kF32Rows / kw) * static_cast<int64_t>(L.hq);
   require(items <= INT32_MAX, "fp32 block: too many work items");
+  g_key_parts = kw;
   if (kw == 4) launch_mfma_f32_k<4>(a, items, stream);
   else if (kw == 2) launch_mfma_f32_k<2>(a, items, stream);
   else launch_mfma_f32_k<1>(a, items, stream);
@@ -1896,14 +1966,10 @@ bool ring_fused_applies(int dtype, int d) { return (dtype == kBF16 || dtype == k
 
 // Decomposition of a fused ring: its sources and rows as one launch (see key_parts).
 static Geometry ring_geometry(int d, int hq, int hkv, int n, const int64_t* len, int causal) {
-  double rows = 0.0, n_max = 0.0;
-  for (int i = 0; i < n; ++i) {
-    const double own = static_cast<double>(ceil_div(len[i], kBK3)), below = static_cast<double>(ceil_div(static_cast<int64_t>(rows), kBK3));
-    n_max = std::max(n_max, own + below);  // without a causal mask: the last domain's, within a tile of every domain's
-    rows += static_cast<double>(len[i]);
-  }
-  const double pairs = causal ? 0.5 * rows * (rows + 1.0) : rows * rows;
-  return geometry(hq, hkv, key_parts(pairs, rows, n, n_max, hq, hkv, d));
+  int64_t keys = 0;
+  for (int i = 0; i < n; ++i) keys += len[i];
+  const double rows = static_cast<double>(keys), pairs = causal ? 0.5 * rows * (rows + 1.0) : rows * rows;
+  return geometry(hq, hkv, key_parts({len, n, pairs, keys, causal ? 1 : keys, 1, true}, hq, hkv, d));
 }
 
 void launch_ring_fused(const RingLaunch& L, hipStream_t stream) {
@@ -1940,11 +2006,14 @@ void launch_ring_fused(const RingLaunch& L, hipStream_t stream) {
   for (int s = 0; s < L.n; ++s) p.qt_begin[s + 1] = p.qt_begin[s] + static_cast<int32_t>(ceil_div(p.len[L.n - 1 - s], tq));
   const int64_t blocks = static_cast<int64_t>(p.qt_begin[L.n]) * p.n_groups;
   require(blocks <= INT32_MAX, "fused ring: too many workgroups");
-  require(blocks == ring_fused_shape(L.d, L.hq, L.hkv, L.n, L.len, L.causal).workgroups, "fused ring: workgroup count");
   p.trace = L.trace;
   p.trace_stride = L.trace_stride;
-  if (L.trace != nullptr) require(L.trace_stride >= kTraceHeaderWords + 2 * L.n, "fused ring: trace stride");
+  if (L.trace != nullptr) {
+    require(L.trace_stride >= kTraceHeaderWords + 2 * L.n, "fused ring: trace stride");
+    require(blocks == ring_fused_shape(L.d, L.hq, L.hkv, L.n, L.len, L.causal).workgroups, "fused ring: workgroup count");
+  }
   const dim3 grid(static_cast<unsigned>(blocks));
+  g_key_parts = geo.kw;
   if (L.dtype == kBF16) {
     if (L.trace != nullptr) launch_ring_kernel<kBF16, true>(geo, grid, p, stream);
     else launch_ring_kernel<kBF16, false>(geo, grid, p, stream);

@@ -465,6 +465,7 @@ void run_replay_fused_positioned(const hcp_ring_replay_desc* d, const ReplayPlan
                                         hcp_ring_view{g.vc, hs, d->head_dim}, out, lse_out);
   L.q_lim = g.lim;
   L.q_rows = g.rows;
+  L.lim_runs = g.rows != nullptr ? 1 : p.n;
   timed(kTimedBlock, stream, [&] { launch_block_partial(L, stream); });
   g_last_path = block_path(L);
 }
@@ -718,7 +719,10 @@ void run_replay(const hcp_ring_replay_desc* d, hcp_ring_view q, hcp_ring_view k,
       float* po = reinterpret_cast<float*>(state);
       float* pl = reinterpret_cast<float*>(state + align256(rows * d->head_dim * sizeof(float)));
       BlockLaunch L = make_launch(&bd, qv, kv_k, kv_v, po, pl);
-      if (lims != nullptr) L.q_lim = lims + static_cast<int64_t>(src) * p.seq + p.off[t];
+      if (lims != nullptr) {
+        L.q_lim = lims + static_cast<int64_t>(src) * p.seq + p.off[t];
+        L.lim_runs = 1;
+      }
       if (idx + 1 == static_cast<int>(p.sources[t].size())) {
         L.fin_out = static_cast<char*>(out.data) + p.off[t] * out.seq_stride * es;
         L.fin_dtype = d->dtype;
@@ -783,6 +787,8 @@ extern "C" {
 const char* hcp_ring_last_error(void) { return g_last_error.c_str(); }
 
 int hcp_ring_last_path(void) { return g_last_path; }
+
+int hcp_ring_last_key_parts(void) { return last_key_parts(); }
 
 int hcp_ring_abi_version(void) { return HCP_RING_ABI_VERSION; }
 

@@ -35,6 +35,9 @@ struct BlockLaunch {
   // Positions mode (causal only, q_lim != nullptr): row i of the query chunk sees keys
   // [0, q_lim[i]) of the KV chunk instead of those with k_off + j <= q_off + i.
   const int32_t* q_lim = nullptr;
+  // Positions mode: the runs of rows over which q_lim ascends to about every key, half of all
+  // (row, key) pairs visible (0: not known).  It only chooses how a launch is split.
+  int lim_runs = 0;
   // Positions mode, 16-bit matrix-core kernels: query row i is row q_rows[i] of the q view
   // and of the final rows (null: row i).
   const int32_t* q_rows = nullptr;
@@ -84,6 +87,8 @@ struct RingShape {
   int64_t workgroups;
   int heads_div, rows_div;
 };
+// Key parts (1, 2 or 4 waves per tile) of this thread's last block or ring launch, 0 before one.
+int last_key_parts();
 RingShape ring_fused_shape(int d, int hq, int hkv, int n, const int64_t* len, int causal);
 // 32-bit words of one trace record of an n-domain fused ring.
 int ring_trace_words(int n);

@@ -99,6 +99,10 @@ enum hcp_ring_path {
 };
 int hcp_ring_last_path(void);
 
+/* Waves among which the last block or replay launch of the calling thread split each tile's
+ * keys: 1, 2 or 4 (1 too for the general kernel; 0 before the first launch). */
+int hcp_ring_last_key_parts(void);
+
 /*
  * Reads and clears the sticky device-side error flags of the current device
  * (bit 0: a paged block id outside [0, num_blocks) was met and that row skipped;

@@ -1427,8 +1427,8 @@ def test_d64_token_major_and_head_major_layouts_agree(gpu, schedule):
         assert launch["workgroups"] == sum(-(-c // 256) for c in chunks) * 14
 
 
-# Short launches split every tile's keys over 2 or 4 waves (KW): per head layout the
-# smallest shapes (KW = 4) and one that leaves fewer CUs idle (KW = 2); key counts around a
+# Short launches split every tile's keys over 2 or 4 waves (KW), those of one tile over 2 or
+# none: per head layout small shapes, some that leave fewer CUs idle, and key counts around a
 # part's 32 or 64 keys and a tile's 128, so that whole parts hold no visible key.
 SPLIT_KEY_CASES = [
     # Hq, Hkv, D, dtype, Lq list, Lk list
@@ -1598,7 +1598,7 @@ def test_decode_runs_over_shards(gpu, case):
 
 # The fp32 kernel's split forms (2 or 4 waves share a 32-row block and fold 32 of every 64
 # or 128 keys each): one and several steps, parts with no visible key, each padded width, and
-# a shape per number of parts.
+# shapes that leave many and few CUs idle.
 F32_SPLIT_CASES = [
     # Hq, Hkv, D, Lq list, Lk list
     (4, 2, 64, (1, 33, 100), (1, 31, 64, 129, 300)),
@@ -1895,3 +1895,94 @@ QKV_WIDE_CASES = [
 @pytest.mark.parametrize("case", QKV_WIDE_CASES, ids=[f"{c[0]}x{c[1]}_{c[2]}q{c[3]}kv_d{c[4]}" for c in QKV_WIDE_CASES])
 def test_qkv_rope_wide_layer_token_counts(gpu, case):
     test_qkv_rope_token_count_edges(gpu, case)
+
+
+# Every form of the block kernels that a launch can take -- key parts, query heads per
+# workgroup, 64 or 128 dims -- at a shape that takes it: ragged rows, and keys that end one, 33
+# or 44 keys into a tile, so that whole parts of it are empty.
+KEY_PART_CASES = [
+    # Hq, Hkv, D, dtype, Lq, Lk, key parts
+    (64, 8, 64, torch.bfloat16, 700, 300, 1),
+    (32, 4, 128, torch.float16, 1500, 161, 1),
+    (32, 8, 128, torch.bfloat16, 1500, 161, 1),
+    (64, 16, 64, torch.float16, 900, 300, 1),
+    (16, 8, 128, torch.bfloat16, 2100, 129, 1),
+    (16, 8, 64, torch.bfloat16, 2100, 129, 1),
+    (16, 16, 128, torch.float16, 2100, 129, 1),
+    (32, 32, 64, torch.bfloat16, 1500, 161, 1),
+    (8, 1, 128, torch.bfloat16, 2100, 300, 2),
+    (64, 8, 64, torch.float16, 300, 300, 2),
+    (16, 8, 128, torch.float16, 1500, 161, 2),
+    (16, 8, 64, torch.bfloat16, 1500, 161, 2),
+    (16, 16, 128, torch.bfloat16, 1500, 161, 2),
+    (16, 16, 64, torch.float16, 1500, 161, 2),
+    (8, 1, 128, torch.float16, 130, 257, 4),
+    (16, 2, 64, torch.bfloat16, 130, 257, 4),
+    (3, 3, 96, torch.bfloat16, 130, 257, 4),
+    (14, 2, 64, torch.float16, 130, 257, 4),
+    (32, 8, 128, torch.float32, 2000, 97, 1),
+    (64, 8, 32, torch.float32, 900, 97, 1),
+    (16, 16, 64, torch.float32, 600, 161, 2),
+    (16, 16, 32, torch.float32, 600, 161, 2),
+    (8, 8, 96, torch.float32, 1300, 129, 2),
+    (32, 8, 128, torch.float32, 320, 300, 2),
+    (4, 2, 64, torch.float32, 33, 300, 4),
+    (2, 2, 32, torch.float32, 40, 300, 4),
+    (4, 1, 96, torch.float32, 65, 161, 4),
+    (3, 1, 128, torch.float32, 96, 257, 4),
+]
+
+
+@pytest.mark.parametrize("case", KEY_PART_CASES,
+                         ids=[f"kw{c[6]}_{c[0]}q{c[1]}kv_d{c[2]}_{str(c[3])[6:]}" for c in KEY_PART_CASES])
+def test_key_part_forms_match_closed_form(gpu, case):
+    # Contiguous positions whose first row sees 40 keys fewer than the last tile's end, the
+    # same as explicit ones, and the first merged into its own state.
+    hq, hkv, d, dt, lq, lk, parts = case
+    (q, k, v), (q32, k32, v32) = draw(lq + 3 * lk + d, [(lq, hq, d), (lk, hkv, d), (lk, hkv, d)], dt)
+    qv, kv, vv = (x.permute(1, 0, 2) for x in (q, k, v))
+    q0 = lk - 40
+    ref_o, ref_l = C.attention_f64(q32, k32, v32, np.arange(q0, q0 + lq), np.arange(lk), 1 / math.sqrt(d))
+    ref_o, ref_l = ref_o.transpose(1, 0, 2), ref_l.T
+    path = "mfma_f32" if dt == torch.float32 else "mfma"
+    tol_o, tol_l = (1e-4, 1e-4) if dt == torch.float32 else (OUT_TOL, LSE_TOL)
+    cont = H.block_partial(qv, kv, vv, q0, 0)
+    assert (H.last_path(), H.last_key_parts()) == (path, parts)
+    pos = H.block_partial_positioned(qv, torch.arange(q0, q0 + lq, device="cuda"), kv, vv, torch.arange(lk, device="cuda"))
+    assert H.last_path() == path and H.last_key_parts() in (1, parts)
+    twice = cont[0].clone(), cont[1].clone()
+    H.block_partial(qv, kv, vv, q0, 0, o=twice[0], lse=twice[1], accumulate=True)
+    assert H.last_key_parts() == parts
+    torch.cuda.synchronize()
+    for (o, l), shift in ((cont, 0.0), (pos, 0.0), (twice, math.log(2.0))):
+        assert np.abs(o.cpu().numpy() - ref_o).max() <= tol_o
+        assert np.abs(l.cpu().numpy() - ref_l - shift).max() <= tol_l
+
+
+@pytest.mark.parametrize("strategy", ["striped", "zigzag"])
+@pytest.mark.parametrize("case", [
+    # chunks, Hq, Hkv, D, dtype, key parts: the query rows in position order in every form
+    ([300, 417], 128, 8, 128, torch.bfloat16, 1),
+    ([300, 417], 128, 16, 64, torch.float16, 1),
+    ([1700, 300], 64, 32, 128, torch.bfloat16, 1),
+    ([900, 817], 64, 64, 64, torch.bfloat16, 1),
+    ([300, 417], 32, 8, 128, torch.float16, 2),
+    ([300, 417], 16, 2, 64, torch.bfloat16, 4),
+], ids=["kw1_g8", "kw1_g8_d64", "kw1_g2", "kw1_g1_d64", "kw2", "kw4"])
+def test_strategy_replay_key_part_forms(gpu, case, strategy):
+    # Four of the heads, of different KV heads, against float64.
+    chunks, hq, hkv, d, dt, parts = case
+    s = sum(chunks)
+    (q, k, v), (q32, k32, v32) = draw(900 + hq + d, [(s, hq, d), (s, hkv, d), (s, hkv, d)], dt)
+    pos = np.array(sum(_strategy_rows(chunks, strategy)[0], []))
+    lse = torch.zeros(hq, s, dtype=torch.float32, device="cuda")
+    out = torch.zeros(hq, s, d, dtype=dt, device="cuda")
+    H.ring_attention_replay(*(x.permute(1, 0, 2) for x in (q, k, v)), chunks, strategy=strategy, out=out, lse_out=lse)
+    assert (H.last_path(), H.last_key_parts()) == ("mfma", parts)
+    torch.cuda.synchronize()
+    assert H.fetch_device_errors() == 0
+    for head in {0, hq // 3, hq // 2 + 1, hq - 1}:
+        kvh = slice(head * hkv // hq, head * hkv // hq + 1)
+        ref_o, ref_l = C.attention_f64(q32[:, head:head + 1], k32[:, kvh], v32[:, kvh], pos, pos, 1 / math.sqrt(d))
+        assert np.abs(out[head].float().cpu().numpy() - ref_o[:, 0]).max() <= OUT_TOL
+        assert np.abs(lse[head].cpu().numpy() - ref_l[:, 0]).max() <= LSE_TOL
