@@ -57,6 +57,16 @@ def test_decode_workspace_covers_every_shorter_context(hcp, batch, heads):
         assert s[0] > 0 and all(a <= b for a, b in zip(s, s[1:])), (batch, heads)
 
 
+@pytest.mark.parametrize("heads", [(4, 0), (0, 0), (-4, -2), (6, 4)])
+def test_static_decode_refuses_bad_heads(hcp, heads):
+    # An error, with or without a device, and never a division by the heads.
+    pool = hcp.PagedPool(256, 8, 16, heads[1], 64, 2)
+    desc = hcp.DecodeDesc(2, 1, heads[0], heads[1], 64, 0, 0, 100, 8, 8, 0.1)
+    rc = hcp.lib().hcp_paged_decode_partial_static(ctypes.byref(desc), ctypes.byref(pool), hcp.View(256, 64, 64), 256, None,
+                                                   256, 256, None)
+    assert rc != 0 and hcp.last_error()
+
+
 def test_null_descriptor_is_invalid(hcp):
     v = hcp.View(0, 0, 1)
     rc = hcp.lib().hcp_ring_block_partial(None, v, v, v, None, None, None)
