@@ -414,7 +414,10 @@ int most_parts(int batch, int hq, int d, int64_t groups) {
 //     sequences of 700 tokens, 24/4 heads, took 64.7 us as 390 workgroups of 8 waves, 45 as
 //     1560 of one.  Workgroups that read part of a token's row cost 2.5% more, and if their
 //     runs lie apart as well (runs that meet) up to a third: 32 sequences of 8000 tokens,
-//     32/8 heads, 190 us as 8 runs of one head a workgroup, 164 as 8 parts of whole rows;
+//     32/8 heads, 190 us as 8 runs of one head a workgroup, 164 as 8 parts of whole rows.
+//     Where the tokens are more than the Infinity Cache holds and only 8 waves are resident
+//     a CU (R = 8 of 128 dims), single runs of part rows cost 10% more: 32 sequences of 3000
+//     tokens, 64/8 heads, 84 us as 6 parts of two heads, 75 as 8 of whole rows;
 //   * `meet` where runs meet in LDS, the more the wider the accumulators: one sequence of 40
 //     tokens, 32/2 heads of 64 dims, 20.0 us with four runs that meet, 13.6 as three parts;
 //   * the parts written and read again, the merge's chain over them and its batches of
@@ -425,20 +428,20 @@ int most_parts(int batch, int hq, int d, int64_t groups) {
 // tokens, some 70 plans each: the model's choice among them is 1.6% above the fastest on
 // average.  Against as many runs as fill the chip once, the heads halved while more than 16
 // parts resulted, these calls take 8% less on average; 32/8, 16/2 and 14/2 heads, 1-64
-// sequences: none more than 6% longer; the worst, 16 sequences of 6000 tokens of 64/8 heads,
-// 89 us against 77.
+// sequences: none more than 6% longer.
 DecodePlan plan_decode(int batch, int hq, int hkv, int d, int n, const DecodeSpan* spans) {
   static const double group[3][2] = {{0.181, 0.157}, {0.229, 0.146}, {0.281, 0.322}};
   static const double chain[3][2] = {{1.09, 0.84}, {1.37, 0.78}, {1.97, 1.36}};
   static const double meet[3] = {1.1, 1.95, 6.9};
   static const int waves_per_cu[3][2] = {{12, 16}, {8, 12}, {8, 8}};  // resident, by registers
-  constexpr double kPartRows = 0.025, kApart = 0.047;
+  constexpr double kPartRows = 0.025, kApart = 0.047, kPartRowsHbm = 1.1, kCacheBytes = 240e6;
   constexpr double kPartValue = 4.4e-6, kPart = 0.029, kPartBatch = 0.8, kStart = 0.05;
   const int64_t groups = span_groups(n, spans);
   const int r = decode_width(hq / hkv), w = r <= 4 ? 0 : r <= 8 ? 1 : 2, h = d == 64 ? 1 : 0;
   const int cus = device_cus(), most = most_parts(batch, hq, d, groups);
   const int whole = static_cast<int>(ceil_div(hkv, ceil_div(hkv, kDecWaves)));
   const double part = kPartValue * batch * hq * d + kPart;
+  const bool uncached = w == 1 && h == 0 && 64.0 * groups * batch * hkv * d > kCacheBytes;  // 16 tokens of K and V a group
   DecodePlan best{1, whole, 1};
   double best_t = 0.0;
   for (int heads = whole;; heads = (heads + 1) / 2) {
@@ -446,7 +449,8 @@ DecodePlan plan_decode(int batch, int hq, int hkv, int d, int n, const DecodeSpa
     for (int subs = 1; heads * subs <= kDecWaves; subs *= 2) {
       const int waves = heads * subs, resident = std::max(1, waves_per_cu[w][h] / waves);
       const double apart = subs > 1 ? kApart * (static_cast<double>(whole) / heads - 1.0) : 0.0;
-      const double unit = group[w][h] * d / 128 * waves * (1.0 + (heads < whole ? kPartRows : 0.0) + apart);
+      const double unit = group[w][h] * d / 128 * waves * (1.0 + (heads < whole ? kPartRows : 0.0) + apart) *
+                          (uncached && heads < whole && subs == 1 ? kPartRowsHbm : 1.0);
       const int64_t shares = std::min<int64_t>(ceil_div(groups, subs), most);  // most parts
       auto consider = [&](int64_t want) {
         const int64_t len = ceil_div(groups, subs * std::min(std::max<int64_t>(want, 1), shares));  // groups of a run
