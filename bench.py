@@ -553,7 +553,7 @@ def bench_decode_ring(H, torch, steps: int, warmup: int):
         shards.append((tab, torch.full((b,), lens[dom], dtype=torch.int32, device="cuda"), lens[dom]))
     out = torch.empty(b, hq, d, dtype=torch.bfloat16, device="cuda")
     lse = torch.empty(b, hq, dtype=torch.float32, device="cuda")
-    # the replay's workspace (split partials and the N domain partials), allocated once
+    # the replay's workspace (the partials of its parts), allocated once
     ws = torch.empty(max(H.decode_ring_workspace_size(q, pool, shards), 1), dtype=torch.uint8, device="cuda")
 
     def step():
@@ -565,11 +565,11 @@ def bench_decode_ring(H, torch, steps: int, warmup: int):
     log(f"decode ring timed x{steps}")
     ms = time_cuda(torch, step, steps)
     kv_bytes = 2 * b * sum(lens) * hkv * d * 2
-    alg = kv_bytes + q.numel() * 2 + 2 * n * b * hq * (d + 1) * 4 + b * sum(nblk) * 4 + out.numel() * 2 + lse.numel() * 4
+    alg = kv_bytes + q.numel() * 2 + b * sum(nblk) * 4 + out.numel() * 2 + lse.numel() * 4
     gbs = alg / (ms * 1e-3) / 1e9
     res = dict(workload=f"f1 decode Q-ring: B={b}, ctx {c['ctx']} growth-sharded over {n} domains "
                         f"(prefill {chunks}, {dec} decode tokens by owner p mod {n}), {hq}q/{hkv}kv, D={d}, bf16, "
-                        f"bs={bs}; one hcp_decode_ring_replay (paged decode per shard + journey-order merge)",
+                        f"bs={bs}; one hcp_decode_ring_replay (one paged decode over the shards + the merge of its parts)",
                value=round(gbs, 1), unit="GB/s", ms_per_step=round(ms, 4), frac_hbm=round(gbs / PEAK_HBM_GBS, 4),
                bytes=alg, finite=bool(torch.isfinite(out.float()).all().item()))
     del pool

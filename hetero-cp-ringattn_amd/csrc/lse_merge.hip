@@ -247,9 +247,10 @@ void launch_lse_merge(int n, const float* const* o_parts, const float* const* ls
   const int64_t threads = ceil_div(static_cast<int64_t>(heads) * q_len, R) * lpr;
   const dim3 grid(static_cast<unsigned>(ceil_div(threads, 256)));
   const int64_t rows = static_cast<int64_t>(heads) * q_len;
-  // Up to four partials the kernel below has all loads of a row in flight too, and from
-  // 2048 rows on it has the workgroups (a decode step of 64 sequences x 32 heads: 165 us
-  // either way; of 16: 55 us with it, 52 with one row per workgroup).
+  // One row per workgroup: up to four partials the kernel below has all loads of a row in
+  // flight too, and with many rows it fills the chip as well and reads wider.  In us, below /
+  // here, 128 dims: 4 partials of 64 rows 3.70 / 3.47; 8 of 64 4.50 / 3.48, of 1024 4.81 /
+  // 4.05, of 1536 4.93 / 4.82, of 2048 4.85 / 5.28; 19 of 64 7.85 / 3.83, of 2048 8.70 / 7.40.
   if (n > 4 && rows <= 1024) {
     const dim3 g(static_cast<unsigned>(rows));
     switch (out_dtype) {

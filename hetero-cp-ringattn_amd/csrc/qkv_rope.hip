@@ -11,18 +11,18 @@
 //     hidden-contiguous), so a lane owns one token and 16 features of each 32-feature
 //     block.  A workgroup computes 256 features x 128, 256 or 384 tokens, 384 features
 //     x 256 tokens or 128 x 128 (chosen per launch) with 8 waves of 64 features x half
-//     the tokens, 192 x a quarter or 64 x a quarter: a wave's features come in pairs of 32-feature blocks at d and
-//     d + D/2 of one head, so each RoPE partner pair sits in the same lane and register
-//     slot of the wave's two blocks -- the rotation needs no data exchange.
+//     the tokens, 192 x a quarter or 64 x a quarter: a wave's features come in pairs of
+//     32-feature blocks at d and d + D/2 of one head, so each RoPE partner pair sits in
+//     the same lane and register slot of the wave's two blocks -- the rotation needs no
+//     data exchange.
 //   * Weight and token tiles of 32 hidden values reach LDS through buffer_load ... lds
 //     (four buffers, three stages in flight, eight and seven for 128 x 128 tiles; one
-//     barrier per stage); chunk p of tile row
-//     r holds global chunk p ^ ((r >> 2) & 3), which keeps the fragment reads free of
-//     bank conflicts.  The loop is software-pipelined: a stage's DMA instructions are
-//     spread through the MFMAs of the stage three before it, the second K half's
-//     fragments are read while the first half's MFMAs run, and the next stage's barrier
-//     sits inside this stage's second half, so its first fragments arrive while the
-//     matrix core still has this stage's MFMAs queued (measured on the Llama-3-8B layer:
+//     barrier per stage); chunk p of tile row r holds global chunk p ^ ((r >> 2) & 3),
+//     which keeps the fragment reads free of bank conflicts.  The loop is software-pipelined:
+//     a stage's DMA instructions are spread through the MFMAs of the stage three before it,
+//     the second K half's fragments are read while the first half's MFMAs run, and the next
+//     stage's barrier sits inside this stage's second half, so its first fragments arrive
+//     while the matrix core still has this stage's MFMAs queued (measured on the Llama-3-8B layer:
 //     +7.6% over one barrier and one DMA burst at each stage start).
 //   * Epilogue, in fp32: + bias, rotate (x1 cos - x2 sin, x1 sin + x2 cos) with cos/sin
 //     from the table row of the token's position, round once to the storage dtype and
