@@ -1622,7 +1622,7 @@ static int fewest_parts(const double (&t)[3]) {
 }
 
 // Key parts of the 16-bit kernels, 256 / KW rows a workgroup.  The costs (per 128-key tile;
-// head dims above 64, then up to 64; 4 us are the launch's own) are fitted on MI355X to 1000
+// head dims above 64; up to 64, masked and not; 4 us are the launch's own) are fitted on MI355X to 1000
 // launches, each measured with every KW: blocks of 16-8192 queries against 16-16384 keys, causal and
 // full rings of 200-9000 tokens, 8-64 heads of 24-128 dims, up to 8 on a KV head.  Of these
 // and 320 ZigZag and Striped replays 11 are slower than with KW = 1 by more than 3%, by at most
@@ -1634,17 +1634,19 @@ static int fewest_parts(const double (&t)[3]) {
 // more than half a workgroup of rows (348 x 104, 16/16 heads: 18.2 us, 15.7 with KW = 2;
 // 68 x 48: 10.8, 11.6).
 static int key_parts(const LaunchLoad& L, int hq, int hkv, int d) {
-  static const KeyPartCost costs[2][3] = {{{7.90, 1.885, 2.87}, {7.80, 1.12, 1.67}, {8.40, 0.775, 1.05}},
+  static const KeyPartCost costs[3][3] = {{{7.90, 1.885, 2.87}, {7.80, 1.12, 1.67}, {8.40, 0.775, 1.05}},
+                                          {{4.45, 1.685, 2.03}, {4.50, 1.04, 1.165}, {4.65, 0.75, 0.505}},
                                           {{4.45, 1.685, 2.03}, {4.50, 1.04, 1.165}, {4.65, 0.75, 0.56}}};
   if (L.most <= kBK3) {
     const Geometry two = geometry(hq, hkv, 2);
     const int64_t longest = *std::max_element(L.rows, L.rows + L.n);
     return longest > geometry(hq, hkv).tq / 2 && launch_items(L, two.n_groups, two.tq) <= device_cus() ? 2 : 1;
   }
+  const int w = !half_width_d(d) ? 0 : L.most > L.fewest ? 1 : 2;
   double t[3];
   for (int i = 0; i < 3; ++i) {
     const Geometry geo = geometry(hq, hkv, 1 << i);
-    t[i] = 4.0 + launch_time(L, geo.n_groups, geo.tq, kBK3, costs[half_width_d(d) ? 1 : 0][i]);
+    t[i] = 4.0 + launch_time(L, geo.n_groups, geo.tq, kBK3, costs[w][i]);
     if (i > 0) t[i] *= split_margin(L, launch_items(L, geo.n_groups, geo.tq));
   }
   return fewest_parts(t);
