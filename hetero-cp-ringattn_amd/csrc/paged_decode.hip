@@ -399,9 +399,16 @@ int64_t span_groups(int n, const DecodeSpan* spans) {
 // Most parts of a plan: what one merge takes, no more than the groups, and within the static
 // scratch of the entry point that uses it (at least one).  Never fewer for more groups.
 int most_parts(int batch, int hq, int d, int64_t groups) {
-  int parts = static_cast<int>(std::min<int64_t>(groups, kMaxParts));
+  const int64_t fit = HCP_DECODE_STATIC_SCRATCH_BYTES / (sizeof(float) * (d + 1) * std::max<int64_t>(1, int64_t(batch) * hq));
+  int parts = static_cast<int>(std::min<int64_t>({groups, kMaxParts, std::max<int64_t>(1, fit)}));
   while (parts > 1 && parts_bytes(parts, batch, hq, d) > HCP_DECODE_STATIC_SCRATCH_BYTES) --parts;
   return parts;
+}
+
+// ceil(a / b) of values that nearly always fit 32 bits, whose division takes a third of the time.
+static int64_t quot(int64_t a, int64_t b) {
+  if (((a + b) >> 32) == 0) return (static_cast<uint32_t>(a) + static_cast<uint32_t>(b) - 1) / static_cast<uint32_t>(b);
+  return ceil_div(a, b);
 }
 
 // The plan with the least modelled time, in us, over 1, 2, 4 or 8 runs a workgroup, all kv
@@ -452,25 +459,36 @@ DecodePlan plan_decode(int batch, int hq, int hkv, int d, int n, const DecodeSpa
       const double unit = group[w][h] * d / 128 * waves * (1.0 + (heads < whole ? kPartRows : 0.0) + apart) *
                           (uncached && heads < whole && subs == 1 ? kPartRowsHbm : 1.0);
       const int64_t shares = std::min<int64_t>(ceil_div(groups, subs), most);  // most parts
+      // Candidates that cannot win are left out: no plan of these heads and subs is better
+      // than its groups spread evenly, none than the chain of its runs (host time of a plan
+      // 0.1-0.7 us; 1.0-2.3 with every candidate worked out, in 64-bit divisions).
+      const double fixed = subs > 1 ? meet[w] : 0.0;
+      if (best_t > 0.0 && unit * rows * groups / (static_cast<double>(subs) * cus) + fixed + part >= best_t) continue;
+      uint64_t seen = 0;
       auto consider = [&](int64_t want) {
-        const int64_t len = ceil_div(groups, subs * std::min(std::max<int64_t>(want, 1), shares));  // groups of a run
-        const int64_t parts = ceil_div(groups, subs * len), per_cu = ceil_div(rows * parts, cus);
+        want = std::min(std::max<int64_t>(want, 1), shares);
+        if (seen >> (want - 1) & 1) return;
+        seen |= uint64_t(1) << (want - 1);
+        const int64_t len = quot(groups, subs * want);  // groups of a run
+        if (best_t > 0.0 && chain[w][h] * len + fixed >= best_t) return;
+        const int64_t parts = quot(groups, subs * len), per_cu = quot(rows * parts, cus);
         const double run = static_cast<double>(len);
-        const double t = std::max(unit * per_cu * run, chain[w][h] * run * ceil_div(per_cu, resident)) +
-                         (subs > 1 ? meet[w] : 0.0) + part * parts + kPartBatch * ((parts - 1) / (h ? 64 : 32)) +
+        const double t = std::max(unit * per_cu * run, chain[w][h] * run * quot(per_cu, resident)) +
+                         fixed + part * parts + kPartBatch * ((parts - 1) / (h ? 64 : 32)) +
                          kStart * per_cu;
         if (best_t == 0.0 || t < best_t) {
           best = DecodePlan{static_cast<int>(parts), heads, subs};
           best_t = t;
         }
       };
-      for (int64_t len : {1, 2, 3, 4, 6, 8}) consider(ceil_div(groups, subs * len));
+      for (int64_t len : {1, 2, 3, 4, 6, 8}) consider(quot(groups, subs * len));
       if (rows >= cus)
         for (int64_t parts : {1, 2, 3, 4, 6, 8, 12}) consider(parts);
       else
-        for (int64_t k : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16}) {
-          consider(k * cus / rows);
-          if (k * cus / rows >= shares) break;
+        for (int k : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16}) {
+          const int parts = k * cus / static_cast<int>(rows);
+          consider(parts);
+          if (parts >= shares) break;
         }
     }
     if (heads == 1) break;
